@@ -179,43 +179,83 @@ __device__ __forceinline__ void pass(cx<R>* buf, const cx<R>* twl, int t) {
   __syncthreads();
 }
 
-// The last pass of a transform with its outputs handed to post(x, value)
-// (x the natural-order index) instead of written to LDS.
-template <typename R, int P, int T, int NS, int RAD, bool INV, int LOG2N, int TSCALE, typename Post>
-__device__ __forceinline__ void last_pass(const cx<R>* buf, const cx<R>* twl, int t, Post post) {
-  constexpr int NB = P / (RAD * T);
-  static_assert(NB >= 1, "too few elements per thread");
-  static_assert(NS * RAD == P, "not the last pass");
-  cx<R> v[NB][RAD];
-#pragma unroll
-  for (int b = 0; b < NB; ++b) {
-    const int j = t + b * T;
-#pragma unroll
-    for (int r = 0; r < RAD; ++r) v[b][r] = buf[pad(j + r * (P / RAD))];
-  }
-  __syncthreads();
-#pragma unroll
-  for (int b = 0; b < NB; ++b) {
-    const int j = t + b * T;  // j < NS: the butterfly's outputs land at j + r*NS
-    if (NS > 1) apply_twiddles<RAD, INV, LOG2N>(v[b], twl, j * (P / (NS * RAD)) * TSCALE);
-    dft_small<RAD, INV>(v[b]);
-#pragma unroll
-    for (int r = 0; r < RAD; ++r) post(j + r * NS, v[b][r]);
-  }
+// Register-resident transform: v[k] holds element t + k T (k < E = P / T) on entry
+// and on exit, for every radix sequence, because both the first pass's inputs
+// j + r P / RAD and the last pass's outputs j + r NS (NS = P / RAD) of the
+// butterflies j = t + b T are congruent to t mod T.  So the stage values enter the
+// first butterfly straight from registers and the results leave the last one in
+// registers: a transform of p passes exchanges p - 1 times through LDS, where the
+// LDS-to-LDS form exchanges p times and is filled and drained once more.
+// PP: two buffers (buf and, padded_size(2^LOG2N) further, the other) used in turn, so an
+// exchange takes one barrier instead of two; BUF is the one that the next exchange writes.
+// post(x): applied to each output.
+//
+// Which product of a sum of two the compiler fuses hangs on the order in which it sees the
+// operands, and on which loads it finds equal.  leaf() makes the first pass's inputs opaque
+// values in the order in which an LDS-to-LDS pass loads them, and FENCE ends each of the last
+// pass's butterflies as its stores would, so a transform rounds alike in every kernel that
+// inlines it.
+template <typename R>
+__device__ __forceinline__ void leaf(cx<R>& v) {
+  asm volatile("" : "+v"(v.re));
+  asm volatile("" : "+v"(v.im));
 }
 
-template <typename R, int P, int T, int NS, bool INV, int LOG2N, int TSCALE, int MAXR, typename Post>
-__device__ __forceinline__ void chain_post(cx<R>* buf, const cx<R>* twl, int t, Post post) {
+template <typename R, int P, int T, int NS, bool INV, int LOG2N, int TSCALE, int MAXR, bool PP, int BUF, bool FENCE, typename Post>
+__device__ __forceinline__ void chain_reg(cx<R> (&v)[P / T], cx<R>* buf, const cx<R>* twl, int t, Post post) {
   constexpr int E = P / T;
   constexpr int R0 = pick_radix<E, MAXR>::v;
   constexpr int REM = P / NS;
   constexpr int RAD = (R0 <= REM) ? R0 : REM;
-  if constexpr (NS * RAD == P) {
-    last_pass<R, P, T, NS, RAD, INV, LOG2N, TSCALE>(buf, twl, t, post);
-  } else {
-    pass<R, P, T, NS, RAD, INV, LOG2N, TSCALE>(buf, twl, t);
-    chain_post<R, P, T, NS * RAD, INV, LOG2N, TSCALE, MAXR>(buf, twl, t, post);
+  constexpr int NB = E / RAD;
+  constexpr bool LAST = NS * RAD == P;
+  constexpr int PREV = PP ? 1 - BUF : 0;  // the buffer of the exchange before this pass
+  constexpr int BS = padded_size(1 << LOG2N);
+  cx<R> w[NB][RAD];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    const int j = t + b * T;
+#pragma unroll
+    for (int r = 0; r < RAD; ++r) {
+      if constexpr (NS == 1) {
+        w[b][r] = v[b + r * NB];
+        leaf(w[b][r]);
+      } else {
+        w[b][r] = buf[PREV * BS + pad(j + r * (P / RAD))];
+      }
+    }
   }
+  if constexpr (NS > 1 && !PP) __syncthreads();
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    const int j = t + b * T;
+    const int k = j & (NS - 1);
+    if constexpr (NS > 1) apply_twiddles<RAD, INV, LOG2N>(w[b], twl, k * (P / (NS * RAD)) * TSCALE);
+    dft_small<RAD, INV>(w[b]);
+    const int base = (j - k) * RAD + k;
+#pragma unroll
+    for (int r = 0; r < RAD; ++r) {
+      if constexpr (LAST) v[b + r * NB] = post(w[b][r]);
+      else buf[(PP ? BUF : 0) * BS + pad(base + r * NS)] = w[b][r];
+    }
+    if constexpr (LAST && FENCE && NB > 1) asm volatile("" ::: "memory");
+  }
+  if constexpr (!LAST) {
+    __syncthreads();
+    chain_reg<R, P, T, NS * RAD, INV, LOG2N, TSCALE, MAXR, PP, PP ? 1 - BUF : 0, FENCE>(v, buf, twl, t, post);
+  }
+}
+
+// number of LDS exchanges of a register-resident P-point transform
+template <int P, int T, int MAXR>
+constexpr int exchanges() {
+  int n = 0, ns = 1;
+  const int r0 = pick_radix<P / T, MAXR>::v;
+  while (ns < P) {
+    ns *= r0 <= P / ns ? r0 : P / ns;
+    ++n;
+  }
+  return n - 1;
 }
 
 template <typename R, int P, int T, int NS, bool INV, int LOG2N, int TSCALE, int MAXR>
@@ -230,24 +270,14 @@ __device__ __forceinline__ void chain(cx<R>* buf, const cx<R>* twl, int t) {
   }
 }
 
-// Full P-point transform in LDS (padded layout).  twl: LDS tables of the
-// 2^LOG2N-point base table (P divides 2^LOG2N).  Callers synchronise before.
-template <typename R, int P, int T, bool INV, int LOG2N, int MAXR = 32>
-__device__ __forceinline__ void fft(cx<R>* buf, const cx<R>* twl) {
+// Full P-point register-resident transform (chain_reg).  The buffers are free when it
+// is called.  Without PP they are free again when it returns; with PP the buffer of the
+// last exchange, (BUF + exchanges - 1) % 2, may still be read by other threads.
+template <typename R, int P, int T, bool INV, int LOG2N, int MAXR, bool PP, int BUF, bool FENCE, typename Post>
+__device__ __forceinline__ void fft_reg(cx<R> (&v)[P / T], cx<R>* buf, const cx<R>* twl, Post post) {
   static_assert((P & (P - 1)) == 0, "power of two");
   static_assert(P / T >= 2, "need at least two elements per thread");
-  chain<R, P, T, 1, INV, LOG2N, (1 << LOG2N) / P, MAXR>(buf, twl, threadIdx.x);
-}
-
-// Full P-point transform whose last pass hands each output (natural-order
-// index x, value) to post instead of storing it: post may write LDS (only the
-// index it is given) or global memory.  Ends after the last pass's reads are
-// synchronised; callers synchronise before reading what post wrote to LDS.
-template <typename R, int P, int T, bool INV, int LOG2N, int MAXR, typename Post>
-__device__ __forceinline__ void fft_post(cx<R>* buf, const cx<R>* twl, Post post) {
-  static_assert((P & (P - 1)) == 0, "power of two");
-  static_assert(P / T >= 2, "need at least two elements per thread");
-  chain_post<R, P, T, 1, INV, LOG2N, (1 << LOG2N) / P, MAXR>(buf, twl, threadIdx.x, post);
+  chain_reg<R, P, T, 1, INV, LOG2N, (1 << LOG2N) / P, MAXR, PP, BUF, FENCE>(v, buf, twl, threadIdx.x, post);
 }
 
 // G independent P-point transforms by one workgroup of G*TG threads: threads

@@ -1,6 +1,6 @@
 // Host side of the stepping engine: plans, launches and the C ABI of
-// include/rkstiff_amd.h.  Kernel instantiations live in rks_k_*.hip (one
-// translation unit per precision x nonlinearity, compiled in parallel).
+// include/rkstiff_amd.h.  Kernel instantiations live in rks_k.hip (compiled once
+// per precision x nonlinearity x method, in parallel).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -101,23 +101,24 @@ __global__ void rks_f64_to_f32(const double* a, float* b, int n) {
 }
 
 
-// explicit instantiations are in rks_k_<prec>_<nl>.hip
-RKS_KERNEL_SIZES(RKS_DECLARE, double, double, NLK_ADVECT)
-RKS_KERNEL_SIZES(RKS_DECLARE, double, double, NLK_CUBIC)
-RKS_KERNEL_SIZES(RKS_DECLARE, float, float, NLK_ADVECT)
-RKS_KERNEL_SIZES(RKS_DECLARE, float, float, NLK_CUBIC)
-RKS_KERNEL_SIZES(RKS_DECLARE, double, float, NLK_ADVECT)
-RKS_KERNEL_SIZES(RKS_DECLARE, double, float, NLK_CUBIC)
-RKS_KERNEL_HANKEL_SIZES(RKS_DECLARE, double, double)
-RKS_KERNEL_HANKEL_SIZES(RKS_DECLARE, double, float)
-RKS_KERNEL_HANKEL_SIZES(RKS_DECLARE, float, float)
-
 // ===========================================================================
 // host side: plans and the C ABI
 // ===========================================================================
 #include "rkstiff_amd.h"
 
 int rks_build_tableau(int method, rks_tableau* out);
+
+// the stepping kernels of each precision (f64, f32, mix) x nonlinearity (advect, cubic,
+// hankel) x method (any: the tableau read from memory); rks_k.hip, RKS_TABLE
+#define RKS_TABLES(X)                                                                        \
+  X(f64_advect_any) X(f64_advect_etd35) X(f64_advect_if34) X(f64_cubic_any) X(f64_cubic_etd35) \
+  X(f64_cubic_if34) X(f64_hankel_any) X(f64_hankel_etd35) X(f32_advect_any)                   \
+  X(f32_advect_etd35) X(f32_advect_if34) X(f32_cubic_any) X(f32_cubic_etd35) X(f32_cubic_if34) \
+  X(f32_hankel_any) X(f32_hankel_etd35) X(mix_advect_any) X(mix_advect_etd35)                 \
+  X(mix_advect_if34) X(mix_cubic_any) X(mix_cubic_etd35) X(mix_cubic_if34) X(mix_hankel_any)  \
+  X(mix_hankel_etd35)
+#define RKS_DECLARE_TABLE(name) bool rks_k_##name(int log2n, bool learn, int tile, rks_kernel_entry* e);
+RKS_TABLES(RKS_DECLARE_TABLE)
 rks_mlp_dev rks_mlp_device(const rks_mlp* n, int policy, double margin, double keep_lo, double keep_hi, int period);
 int rks_mlp_device_of(const rks_mlp* n);
 
@@ -143,101 +144,42 @@ namespace {
     if (e_ != hipSuccess) return fail(RKS_ERR_HIP, std::string(#x) + ": " + hipGetErrorString(e_)); \
   } while (0)
 
-typedef void (*kernel_fn)(rks_launch);
+typedef rks_kernel_entry KernelEntry;
 
-struct KernelEntry {
-  const void* fn;
-  int threads;
-  int lds;
-};
-
-template <typename R, typename RN, int LOG2N, int NLK, bool LE, int TI = 0>
-KernelEntry entry_of() {
-  KernelEntry e;
-  e.fn = (const void*)&rks_kernel<R, RN, LOG2N, NLK, LE, TI>;
-  e.threads = rks_threads(LOG2N, NLK) << TI;
-  e.lds = rks_lds_bytes<R, LOG2N, NLK>();
-  return e;
-}
-
-template <typename R, typename RN, int NLK>
-bool lookup_nlk(int log2n, bool learn, int tile, KernelEntry* e) {
-  if (tile == 1) {
-    if (learn) {
-      switch (log2n) {
-        case 9: *e = entry_of<R, RN, 9, NLK, true, 1>(); return true;
-        case 10: *e = entry_of<R, RN, 10, NLK, true, 1>(); return true;
-        case 11: *e = entry_of<R, RN, 11, NLK, true, 1>(); return true;
-        case 12: *e = entry_of<R, RN, 12, NLK, true, 1>(); return true;
-        default: return false;
-      }
-    }
-    switch (log2n) {
-      case 9: *e = entry_of<R, RN, 9, NLK, false, 1>(); return true;
-      case 10: *e = entry_of<R, RN, 10, NLK, false, 1>(); return true;
-      case 11: *e = entry_of<R, RN, 11, NLK, false, 1>(); return true;
-      case 12: *e = entry_of<R, RN, 12, NLK, false, 1>(); return true;
-      default: return false;
-    }
-  }
-  if (tile != 0) return false;
-  if (learn) {
-    switch (log2n) {
-      case 7: *e = entry_of<R, RN, 7, NLK, true>(); return true;
-      case 8: *e = entry_of<R, RN, 8, NLK, true>(); return true;
-      case 9: *e = entry_of<R, RN, 9, NLK, true>(); return true;
-      case 10: *e = entry_of<R, RN, 10, NLK, true>(); return true;
-      case 11: *e = entry_of<R, RN, 11, NLK, true>(); return true;
-      case 12: *e = entry_of<R, RN, 12, NLK, true>(); return true;
-      case 13: *e = entry_of<R, RN, 13, NLK, true>(); return true;
-      default: return false;
-    }
-  }
-  switch (log2n) {
-    case 4: *e = entry_of<R, RN, 4, NLK, false>(); return true;
-    case 5: *e = entry_of<R, RN, 5, NLK, false>(); return true;
-    case 6: *e = entry_of<R, RN, 6, NLK, false>(); return true;
-    case 7: *e = entry_of<R, RN, 7, NLK, false>(); return true;
-    case 8: *e = entry_of<R, RN, 8, NLK, false>(); return true;
-    case 9: *e = entry_of<R, RN, 9, NLK, false>(); return true;
-    case 10: *e = entry_of<R, RN, 10, NLK, false>(); return true;
-    case 11: *e = entry_of<R, RN, 11, NLK, false>(); return true;
-    case 12: *e = entry_of<R, RN, 12, NLK, false>(); return true;
-    case 13: *e = entry_of<R, RN, 13, NLK, false>(); return true;
-    default: return false;
-  }
+// Which stepping kernel runs a plan: the one compiled for its method where that exists, else
+// the one that reads the tableau.  ETD35 and IF34 are the methods of every workload; their
+// kernels are compiled for the coefficient storage that goes with the nonlinearity (real
+// lin_op with the advective term, complex with the cubic ones), so a complex lin_op with the
+// advective term (KdV) or a real one with a cubic term takes the general kernel.
+int method_variant(int method, int nlk, int coef_real) {
+  if ((nlk == RKS_NL_ADVECT_RFFT) != (coef_real != 0)) return RKS_METH_ANY;
+  if (method == RKS_M_ETD35) return method;
+  if (method == RKS_M_IF34 && nlk != RKS_NL_HANKEL_CUBIC) return method;
+  return RKS_METH_ANY;
 }
 
 // learn: the proposer variant (a proposer or training records are attached);
 // tile: 0 the default tile, 1 twice the threads per trajectory (n = 2^9 .. 2^12)
-// the Hankel kind: size classes 2^4 .. 2^10, one tile, no proposer variant
-template <typename R, typename RN>
-bool lookup_hankel(int log2n, bool learn, int tile, KernelEntry* e) {
-  if (learn || tile != 0) return false;
-  switch (log2n) {
-    case 4: *e = entry_of<R, RN, 4, NLK_HANKEL, false>(); return true;
-    case 5: *e = entry_of<R, RN, 5, NLK_HANKEL, false>(); return true;
-    case 6: *e = entry_of<R, RN, 6, NLK_HANKEL, false>(); return true;
-    case 7: *e = entry_of<R, RN, 7, NLK_HANKEL, false>(); return true;
-    case 8: *e = entry_of<R, RN, 8, NLK_HANKEL, false>(); return true;
-    case 9: *e = entry_of<R, RN, 9, NLK_HANKEL, false>(); return true;
-    case 10: *e = entry_of<R, RN, 10, NLK_HANKEL, false>(); return true;
-    default: return false;
-  }
-}
-
-bool lookup(int prec, int nlk, int log2n, bool learn, KernelEntry* e, int tile = 0) {
-  if (nlk == NLK_HANKEL) {
-    if (prec == RKS_F64) return lookup_hankel<double, double>(log2n, learn, tile, e);
-    if (prec == RKS_MIXED) return lookup_hankel<double, float>(log2n, learn, tile, e);
-    return lookup_hankel<float, float>(log2n, learn, tile, e);
-  }
-  if (prec == RKS_F64) return nlk == NLK_ADVECT ? lookup_nlk<double, double, NLK_ADVECT>(log2n, learn, tile, e)
-                                                : lookup_nlk<double, double, NLK_CUBIC>(log2n, learn, tile, e);
-  if (prec == RKS_MIXED) return nlk == NLK_ADVECT ? lookup_nlk<double, float, NLK_ADVECT>(log2n, learn, tile, e)
-                                                  : lookup_nlk<double, float, NLK_CUBIC>(log2n, learn, tile, e);
-  return nlk == NLK_ADVECT ? lookup_nlk<float, float, NLK_ADVECT>(log2n, learn, tile, e)
-                           : lookup_nlk<float, float, NLK_CUBIC>(log2n, learn, tile, e);
+bool lookup(int prec, int nlk, int variant, int log2n, bool learn, KernelEntry* e, int tile = 0) {
+#define RKS_PICK(p)                                                                                        \
+  do {                                                                                                     \
+    if (nlk == RKS_NL_ADVECT_RFFT)                                                                         \
+      return variant == RKS_M_ETD35  ? rks_k_##p##_advect_etd35(log2n, learn, tile, e)                     \
+             : variant == RKS_M_IF34 ? rks_k_##p##_advect_if34(log2n, learn, tile, e)                      \
+                                     : rks_k_##p##_advect_any(log2n, learn, tile, e);                      \
+    if (nlk == RKS_NL_CUBIC_FFT)                                                                           \
+      return variant == RKS_M_ETD35  ? rks_k_##p##_cubic_etd35(log2n, learn, tile, e)                      \
+             : variant == RKS_M_IF34 ? rks_k_##p##_cubic_if34(log2n, learn, tile, e)                       \
+                                     : rks_k_##p##_cubic_any(log2n, learn, tile, e);                       \
+    if (nlk == RKS_NL_HANKEL_CUBIC)                                                                        \
+      return variant == RKS_M_ETD35 ? rks_k_##p##_hankel_etd35(log2n, learn, tile, e)                      \
+                                    : rks_k_##p##_hankel_any(log2n, learn, tile, e);                       \
+    return false;                                                                                          \
+  } while (0)
+  if (prec == RKS_F64) RKS_PICK(f64);
+  if (prec == RKS_MIXED) RKS_PICK(mix);
+  RKS_PICK(f32);
+#undef RKS_PICK
 }
 
 int ilog2(int n) {
@@ -259,6 +201,7 @@ struct rks_plan {
   int method = 0, nlk = 0, prec = 0, ninst = 0, device = 0, cu = 256;
   int esize = 16;  // state element bytes (complex)
   int coef_real = 0;  // coefficients stored real (RKS_CST_*_REAL)
+  int variant = RKS_METH_ANY;  // method_variant
   int nsize = 16;  // NL / coefficient storage element bytes (complex)
   size_t coef_bytes_per_mode = 0;
   rks_tableau tab;
@@ -382,21 +325,8 @@ int rks_plan_create(int method, int nl_kind, int precision, const rks_config* cf
     bool real = nl_kind != RKS_NL_NONE;
     for (int i = 0; i < ninst && real; ++i) real = !desc[i].L_is_complex;
     p->coef_real = real ? 1 : 0;
-    const int rs_b = (precision == RKS_MIXED ? 16 : p->esize) / (real ? 2 : 1);
-    const int rn_b = (precision == RKS_MIXED ? 8 : p->esize) / (real ? 2 : 1);
-    int n_rs = 0;
-    for (int c = 0; c < p->tab.ncoef; ++c) n_rs += p->tab.coef_rs[c] ? 1 : 0;
-    int rank_rs = 0, rank_rn = 0;
-    for (int c = 0; c < p->tab.ncoef; ++c) {
-      int rs = p->tab.coef_rs[c] ? 1 : 0;
-      if (precision != RKS_MIXED) rs = 1;  // one storage precision
-      if (precision != RKS_MIXED) p->tab.coef_off[c] = c * rs_b;
-      else if (rs) p->tab.coef_off[c] = rs_b * rank_rs++;
-      else p->tab.coef_off[c] = rs_b * n_rs + rn_b * rank_rn++;
-      p->tab.coef_rs[c] = real ? (rs ? RKS_CST_RS_REAL : RKS_CST_RN_REAL) : (rs ? RKS_CST_RS : RKS_CST_RN);
-    }
-    p->coef_bytes_per_mode = precision == RKS_MIXED ? (size_t)(rs_b * n_rs + rn_b * (p->tab.ncoef - n_rs))
-                                                    : (size_t)p->tab.ncoef * rs_b;
+    p->coef_bytes_per_mode = (size_t)rks_tab::layout(p->tab, p->esize, p->nsize, real);
+    p->variant = method_variant(method, nl_kind, p->coef_real);
   }
   fill_ctrl(&p->ctl, cfg);
   if (cfg->contour_points < 2) {
@@ -582,15 +512,15 @@ int rks_plan_create(int method, int nl_kind, int precision, const rks_config* cf
       p->bucket_count.push_back((int)byl[l].size());
       for (int i : byl[l]) p->order.push_back(i);
       KernelEntry e;
-      if (!lookup(precision, nl_kind, l, false, &e)) {
+      if (!lookup(precision, nl_kind, p->variant, l, false, &e)) {
         rks_plan_destroy(p);
         return fail(RKS_ERR_INVALID, "no kernel for this size");
       }
       HIPCHK(hipFuncSetAttribute(e.fn, hipFuncAttributeMaxDynamicSharedMemorySize, e.lds));
       KernelEntry el;
-      if (lookup(precision, nl_kind, l, true, &el))
+      if (lookup(precision, nl_kind, p->variant, l, true, &el))
         HIPCHK(hipFuncSetAttribute(el.fn, hipFuncAttributeMaxDynamicSharedMemorySize, el.lds));
-      if (lookup(precision, nl_kind, l, false, &el, 1))
+      if (lookup(precision, nl_kind, p->variant, l, false, &el, 1))
         HIPCHK(hipFuncSetAttribute(el.fn, hipFuncAttributeMaxDynamicSharedMemorySize, el.lds));
       if (hankel) continue;  // no transform tables
       const int N = 1 << l;
@@ -755,7 +685,7 @@ static int launch_all(rks_plan* p, int mode, double h_mode, hipStream_t stream) 
     KernelEntry e;
     const bool learn = p->mlp.on || p->d_rec != nullptr;
     const int ti = b < p->tile.size() ? p->tile[b] : 0;
-    if (!lookup(p->prec, p->nlk, p->bucket_log2[b], learn, &e, ti))
+    if (!lookup(p->prec, p->nlk, p->variant, p->bucket_log2[b], learn, &e, ti))
       return fail(RKS_ERR_INVALID, "no kernel for this grid size, variant and tile");
     L.order = p->d_order + p->bucket_start[b];
     L.count = p->bucket_count[b];
@@ -1075,12 +1005,12 @@ int rks_plan_buckets(rks_plan* p, int* nbucket, int* log2n, int* count, int* max
     if (count) count[b] = p->bucket_count[b];
     if (ntile) {
       KernelEntry e1;
-      ntile[b] = lookup(p->prec, p->nlk, p->bucket_log2[b], false, &e1, 1) ? 2 : 1;
+      ntile[b] = lookup(p->prec, p->nlk, p->variant, p->bucket_log2[b], false, &e1, 1) ? 2 : 1;
     }
     if (max_wg_per_cu) {
       KernelEntry e;
       int per_cu = 0;
-      if (!lookup(p->prec, p->nlk, p->bucket_log2[b], p->mlp.on || p->d_rec != nullptr, &e) ||
+      if (!lookup(p->prec, p->nlk, p->variant, p->bucket_log2[b], p->mlp.on || p->d_rec != nullptr, &e) ||
           hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, e.fn, e.threads, e.lds) != hipSuccess || per_cu < 1)
         per_cu = 1;
       max_wg_per_cu[b] = per_cu;
@@ -1102,7 +1032,7 @@ int rks_plan_set_launch(rks_plan* p, int concurrent, const int* wg_per_cu, const
     }
     if (tile) {
       KernelEntry e1;
-      if (tile[b] != 0 && !(tile[b] == 1 && lookup(p->prec, p->nlk, p->bucket_log2[b], false, &e1, 1)))
+      if (tile[b] != 0 && !(tile[b] == 1 && lookup(p->prec, p->nlk, p->variant, p->bucket_log2[b], false, &e1, 1)))
         return fail(RKS_ERR_INVALID, "tile 1 exists for n = 512 .. 4096 only");
       ti[b] = tile[b];
     }

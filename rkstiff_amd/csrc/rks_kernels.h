@@ -25,6 +25,7 @@
 
 #include "rks_fft.h"
 #include "rks_math.h"
+#include "rks_method.h"
 #include "rks_mlp.h"
 #include "rks_types.h"
 
@@ -61,14 +62,6 @@ __host__ __device__ constexpr int rks_threads(int log2n, int nlk) {
 
 // largest in-register radix of the LDS FFT passes
 #define RKS_MAXR 16
-
-// LDS bytes of the persistent kernel: padded FFT buffer + twiddle tables (Hankel:
-// the stage values and the |f|^2 f vector)
-template <typename R, int LOG2N, int NLK>
-__host__ __device__ constexpr int rks_lds_bytes() {
-  return (rksfft::padded_size(1 << LOG2N) + (NLK == NLK_HANKEL ? (1 << LOG2N) : rksfft::TwSplit<LOG2N>::SIZE)) *
-         (int)sizeof(cx<R>);
-}
 
 __device__ __forceinline__ double nanmax(double a, double b) {
   if (a != a) return a;
@@ -359,10 +352,97 @@ __device__ __attribute__((noinline)) void coef_update(const rks_tableau& tb_in, 
   __syncthreads();
 }
 
+// All fractions of one method's tableau for one mode: recipe constants as literals.
+// v: the basis values of fraction F, by get(F, v)
+template <typename TT, int F, typename RS, typename RN, typename Get>
+__device__ __forceinline__ void method_fracs(Get get, double h, int m, size_t M, char* __restrict__ cbase) {
+  if constexpr (F < TT::tab.nfrac) {
+    z64 v[4];
+    v[1] = v[2] = v[3] = mkc(0.0, 0.0);
+    get(TT::tab.frac[F].fnum, TT::tab.frac[F].fden, TT::tab.frac[F].mask, v);
+    coef_recipes<TT, F, RS, RN>(v, h, m, M, cbase, std::make_integer_sequence<int, TT::tab.ncoef>{});
+    method_fracs<TT, F + 1, RS, RN>(get, h, m, M, cbase);
+  }
+}
+
+template <typename TT, int F, typename RS, typename RN, int GS, typename CT>
+__device__ __forceinline__ void method_small(CT& ct, z64 z, int lane, double h, int m, size_t M,
+                                             char* __restrict__ cbase) {
+  if constexpr (F < TT::tab.nfrac) {
+#pragma clang fp contract(off)
+    constexpr int fnum = TT::tab.frac[F].fnum, fden = TT::tab.frac[F].fden, fmask = TT::tab.frac[F].mask;
+    z64 v[4];
+    v[1] = v[2] = v[3] = mkc(0.0, 0.0);
+    if constexpr ((fmask & 14) != 0) {
+      z64 acc[4];
+      acc[1] = acc[2] = acc[3] = mkc(0.0, 0.0);
+      for (int j = lane; j < ct.contour_points; j += GS) {
+        const z64 nd = contour_node(ct.contour_points, ct.contour_radius, j);
+        frac_contour_add(fnum, fden, fmask, mkc(z.re + nd.re, z.im + nd.im), acc);
+      }
+#pragma unroll
+      for (int o = GS / 2; o >= 1; o >>= 1) {
+#pragma unroll
+        for (int r = 1; r <= 3; ++r) {
+          acc[r].re += __shfl_xor(acc[r].re, o, 64);
+          acc[r].im += __shfl_xor(acc[r].im, o, 64);
+        }
+      }
+#pragma unroll
+      for (int r = 1; r <= 3; ++r) v[r] = np_rdiv(np_rmul(h, acc[r]), (double)ct.contour_points);
+    }
+    if (lane == 0) {
+      v[0] = np_exp(frac_arg(z, fnum, fden, 1));
+      coef_recipes<TT, F, RS, RN>(v, h, m, M, cbase, std::make_integer_sequence<int, TT::tab.ncoef>{});
+    }
+    method_small<TT, F + 1, RS, RN, GS>(ct, z, lane, h, m, M, cbase);
+  }
+}
+
+// coef_update of one method.  The generator was bound by the tableau it walked: per mode,
+// every fraction searched the whole coefficient list and divided by run-time constants.
+template <typename TT, typename RS, typename RN, int T, int MPT>
+__device__ __attribute__((noinline)) void coef_update_method(const rks_ctrl& ct_in, const double* __restrict__ L,
+                                                             int M, int Mg, double h, char* __restrict__ cbase,
+                                                             int* list, int* count) {
+#pragma clang fp contract(off)
+  rks_cctl& ct = *rks_uniform_const<rks_cctl>(&ct_in);
+  constexpr int LC = TT::tab.coef_rs[0] == RKS_CST_RS || TT::tab.coef_rs[0] == RKS_CST_RN;
+  constexpr int cplx = LC || TT::tab.uses_contour;
+  const int t = threadIdx.x;
+  if (TT::tab.uses_contour) {
+    if (t == 0) *count = 0;
+    __syncthreads();
+  }
+#pragma unroll 1
+  for (int i = 0; i < MPT; ++i) {
+    const int m = t + i * T;
+    if (m >= Mg) break;
+    const z64 z = mode_z(L, LC, m, h);
+    if (TT::tab.uses_contour && hypot(z.re, z.im) < ct.modecutoff) {
+      list[atomicAdd(count, 1)] = m;
+      continue;
+    }
+    method_fracs<TT, 0, RS, RN>(
+        [&](int fnum, int fden, int fmask, z64(&v)[4]) { frac_direct(fnum, fden, fmask, z, h, cplx, v); }, h, m,
+        (size_t)M, cbase);
+  }
+  if constexpr (TT::tab.uses_contour != 0) {
+    __syncthreads();
+    const int nsmall = *count;
+    constexpr int GS = T < 32 ? T : 32;
+    const int g = t / GS, lane = t % GS;
+    for (int idx = g; idx < nsmall; idx += T / GS) {
+      const int m = list[idx];
+      method_small<TT, 0, RS, RN, GS>(ct, mode_z(L, LC, m, h), lane, h, m, (size_t)M, cbase);
+    }
+  }
+  __syncthreads();
+}
+
 // ---------------------------------------------------------------------------
 // Stage combinations and the error estimate, chunked and term-major: CH modes
-// of one thread at once (a ChunkIdx: m0 + i*T, or the persistent kernel's
-// own_chunk map), so every term issues CH independent loads.  Arithmetic is in the state precision RS; NL arrays and the non-
+// of one thread at once (a ChunkIdx: m0 + i*T), so every term issues CH independent loads.  Arithmetic is in the state precision RS; NL arrays and the non-
 // propagator coefficients may be stored in RN (converted on load).
 //   term (rks_term grouping):  inner = NL[src] + scale2 * NL[src2]
 //     hmode 0: scale * (C * inner)   1: ((h * C) * inner) * scale   2: ((scale*h)/den) * inner
@@ -371,11 +451,11 @@ __device__ __attribute__((noinline)) void coef_update(const rks_tableau& tb_in, 
 // branching, so a chunk's loads are straight-line code and issue back to
 // back; callers discard the lanes with ok[i] false.
 //
-// Mirror pairs (sym): slots 2j and 2j+1 hold a mode and its mirror (1-D: q
-// and n - q; 2-D: rows q and n - q of one column; q = 0 pairs with n/2), and
+// Mirror pairs (sym): slots 2j and 2j+1 hold a mode and its mirror (2-D: rows
+// q and n - q of one column; q = 0 pairs with n/2), and
 // the linear operator is mirror-symmetric, so both have the same
-// coefficients.  Coefficients are stored for the modes below `lim` only (1-D:
-// 0..n/2; 2-D: rows 0..n/2); an odd slot at or past lim reads its even
+// coefficients.  Coefficients are stored for the modes below `lim` only
+// (rows 0..n/2); an odd slot at or past lim reads its even
 // slot's coefficient, one below lim (the n/2 partner of q = 0) its own.
 // anyq = 0: only slot 1 can hold such a partner.
 // ---------------------------------------------------------------------------
@@ -386,8 +466,9 @@ struct ChunkIdx {
   int sym;   // slots are mirror pairs sharing coefficients
   int lim;   // first mode without stored coefficients (sym only)
   int anyq;  // any odd slot may lie below lim (else only slot 1)
+  int fold;  // 1-D: mode m > fold / 2 reads the coefficient of fold - m (0: every mode its own)
   __device__ __forceinline__ ChunkIdx() {}
-  __device__ __forceinline__ ChunkIdx(int m0, int T, int mlim) : sym(0), lim(0), anyq(0) {
+  __device__ __forceinline__ ChunkIdx(int m0, int T, int mlim) : sym(0), lim(0), anyq(0), fold(0) {
 #pragma unroll
     for (int i = 0; i < CH; ++i) {
       const int x = m0 + i * T;
@@ -397,42 +478,70 @@ struct ChunkIdx {
   }
 };
 
-// Mode ownership in the persistent kernel: thread t holds MPT modes in
-// chunks of CH.  Complex-state kernels (M = N) hold mirror pairs, mode
-// q = t + j*T (j < N/(2T)) in slot 2j and its mirror N - q (N/2 for q = 0) in
-// slot 2j + 1; the rfft-layout kernels hold m = t + k*T.  Every M-sized array
-// (state, candidates, NL slots, coefficients) is read and written through
-// this map by the stage passes, so each element a stage pass produces is
-// consumed by the same thread.
-// PAIRS = false (the Hankel layout): m = t + k*T below the runtime limit mlim.
-template <int N, int M, int T, int CH, bool PAIRS = (M == N)>
-__device__ __forceinline__ ChunkIdx<CH> own_chunk(int c, int sym, int mlim = M) {
+// Mode ownership in the persistent kernel: thread t holds the modes m = t + k T, the
+// elements that its first and last transform butterflies hold (rks_fft.h chain_reg), so
+// stage values, NL values and the state pass between the stage sums and the transforms
+// in registers.  rfft layout: slots k < N / (2T), and slot N / (2T) is the n/2 mode of
+// thread 0.  Every M-sized array is read and written through this map, so each element a
+// stage pass produces is consumed by the same thread.
+template <int N, int M, int T, int NLK>
+struct Own {
+  static constexpr int MPT = (M + T - 1) / T;
+  static constexpr bool RFFT = M == N / 2 + 1;
+  int lim;   // modes below it (the Hankel kind's radial points; every mode otherwise)
+  int fold;  // mirror-symmetric lin_op: N (coefficients of modes 0..N/2 only), else 0
+  int t;     // the thread
+  __device__ __forceinline__ int raw(int k) const { return t + k * T; }
+  // The same map behind an opaque copy of the thread index: addresses derived from it are
+  // formed where they are used.  Otherwise the compiler hoists every slot's offset out of
+  // the stage loop and holds them (up to 48 registers) through the transforms.
+  __device__ __forceinline__ Own fresh() const {
+    Own o = *this;
+    asm volatile("" : "+v"(o.t));
+    return o;
+  }
+  __device__ __forceinline__ bool ok(int k) const {
+    if (M % T == 0 && NLK != NLK_HANKEL) return true;
+    if (RFFT && M == (MPT - 1) * T + 1 && k < MPT - 1) return true;
+    return raw(k) < lim;
+  }
+  // always in bounds: a slot without a mode reads one of the thread's (or mode 0)
+  __device__ __forceinline__ int m(int k) const { return ok(k) ? raw(k) : 0; }
+  __device__ __forceinline__ int c(int k) const {
+    const int x = m(k);
+    return (fold && x > N / 2) ? N - x : x;
+  }
+};
+
+template <int N, int M, int T, int NLK, int CH>
+__device__ __forceinline__ ChunkIdx<CH> own_chunk(int c, const Own<N, M, T, NLK>& ow) {
   ChunkIdx<CH> ix;
-  const int t = threadIdx.x;
-  if constexpr (PAIRS) {
-    static_assert(CH % 2 == 0 && N % (2 * T) == 0, "whole mirror pairs per chunk");
-    ix.sym = sym;
-    ix.lim = N / 2 + 1;
-    ix.anyq = 0;
+  ix.sym = 0;
+  ix.lim = 0;
+  ix.anyq = 0;
+  ix.fold = ow.fold;
 #pragma unroll
-    for (int j = 0; j < CH / 2; ++j) {
-      const int q = t + (c * (CH / 2) + j) * T;
-      ix.m[2 * j] = q;
-      ix.m[2 * j + 1] = q == 0 ? N / 2 : N - q;
-      ix.ok[2 * j] = ix.ok[2 * j + 1] = true;
-    }
-  } else {
-    ix.sym = 0;
-    ix.lim = 0;
-    ix.anyq = 0;
-#pragma unroll
-    for (int i = 0; i < CH; ++i) {
-      const int x = t + (c * CH + i) * T;
-      ix.ok[i] = x < mlim;
-      ix.m[i] = ix.ok[i] ? x : 0;
-    }
+  for (int i = 0; i < CH; ++i) {
+    const int x = (int)threadIdx.x + (c * CH + i) * T;
+    ix.ok[i] = x < ow.lim;
+    ix.m[i] = ix.ok[i] ? x : 0;
   }
   return ix;
+}
+
+// Slot k's mode in the order of the error norm's sums: fft layout, thread t adds the mirror
+// pairs q = t + jT (slot 2j) and N - q (slot 2j + 1; N/2 for q = 0), else its own modes.  One
+// order for all kernels of a size: s in its last bits reaches h, in MIXED a changed h rounds
+// the FP32 coefficients anew (~1e-9 of the state), and unresolved runs amplify any change.
+template <int N, int M, int T, int NLK>
+__device__ __forceinline__ int norm_mode(int k) {
+  const int t = threadIdx.x;
+  if constexpr (M == N && NLK != NLK_HANKEL) {
+    const int q = t + (k >> 1) * T;
+    return (k & 1) == 0 ? q : (q == 0 ? N / 2 : N - q);
+  } else {
+    return t + k * T;
+  }
 }
 
 // coefficient array c of the chunk's modes; M is the array stride (modes)
@@ -447,7 +556,7 @@ __device__ __forceinline__ void load_coef(const rks_tableau& tb, const char* cba
   // address and the caches serve the repeat.
   int ci[CH];
 #pragma unroll
-  for (int i = 0; i < CH; ++i) ci[i] = ix.m[i];
+  for (int i = 0; i < CH; ++i) ci[i] = (ix.fold && ix.m[i] > ix.fold / 2) ? ix.fold - ix.m[i] : ix.m[i];
   if constexpr (CH % 2 == 0 && sizeof(RS) > 4) {
 #pragma unroll
     for (int j = 0; j < CH / 2; ++j)
@@ -686,14 +795,16 @@ __device__ __forceinline__ void final_chunk(const rks_tableau& tb, const cx<RS>*
 }
 
 // ---------------------------------------------------------------------------
-// nonlinear term in LDS.  fill_nl writes the spectrum produced by getk
-// into the padded LDS buffer (inlined into the stage loop); nl_core runs the
-// transforms and writes NL to dst in the transform's own thread order and
-// ends on a barrier, after which any thread of the workgroup reads NL.
-// nl_core is not inlined: its register allocation is independent of the
-// controller and coefficient code around it.
+// nonlinear term.  The spectrum is in registers, slot k of thread t holding mode
+// t + kT (Own), and the NL values come back in the same slots: the transforms take
+// their inputs from and leave their results in registers (fft_reg), and the
+// pointwise products are formed between them without a trip through LDS.  A cubic
+// n = 8192 evaluation (radix 16, 16, 16, 2) makes 6 exchanges; filling the buffer,
+// two LDS-to-LDS transforms and the product between them made 8 and a third more
+// barriers.  Called by all threads; the LDS buffers are free at the call and at the
+// return.
 // ---------------------------------------------------------------------------
-// modes per chunk of the stage combination
+// modes per chunk of the stage combination of the generic kernels
 #ifndef RKS_CHUNK
 #define RKS_CHUNK 8
 #endif
@@ -703,44 +814,26 @@ struct Chunk {
   static constexpr int NCH = (MPT + CH - 1) / CH;
 };
 
-// getk(ix, acc): the CH spectrum values of the chunk's modes ix.m (own_chunk)
-// mlim: modes below it (the Hankel kind's radial points; the grid's modes otherwise)
-template <typename R, int LOG2N, int T, int NLK, typename GetK>
-__device__ __forceinline__ void fill_nl(GetK getk, cx<R>* buf, const R* __restrict__ kx, int sym, int mlim) {
-  using C = cx<R>;
-  constexpr int N = 1 << LOG2N;
-  constexpr int M = (NLK == NLK_ADVECT) ? N / 2 + 1 : N;
-  constexpr int MPT = (M + T - 1) / T;
-  constexpr int CH = Chunk<MPT>::CH;
-  constexpr int H = N / 2;
-#pragma unroll 1
-  for (int c = 0; c < Chunk<MPT>::NCH; ++c) {
-    const ChunkIdx<CH> ix = own_chunk<N, M, T, CH, (M == N && NLK != NLK_HANKEL)>(c, sym, mlim);
-    C acc[CH];
-    getk(ix, acc);
-#pragma unroll
-    for (int i = 0; i < CH; ++i) {
-      if (!ix.ok[i]) continue;
-      const int m = ix.m[i];
-      if constexpr (NLK == NLK_HANKEL) {
-        buf[m] = acc[i];
-      } else if constexpr (NLK == NLK_CUBIC) {
-        buf[rksfft::pad(m)] = acc[i];
-      } else {
-        const C U = acc[i];
-        const R k = kx[m];
-        const C V = mkc(-k * U.im, k * U.re);
-        // spectrum of u + i u_x: Y[m] = U + iV, Y[N-m] = conj(U) + i conj(V); DC and
-        // Nyquist keep only the real parts, as irfft does
-        if (m == 0 || m == H) {
-          buf[rksfft::pad(m)] = mkc(U.re, V.re);
-        } else {
-          buf[rksfft::pad(m)] = mkc(U.re - V.im, U.im + V.re);
-          buf[rksfft::pad(N - m)] = mkc(U.re + V.im, V.re - U.im);
-        }
-      }
-    }
-  }
+// Two exchange buffers where they fit beside the register-bound number of waves: a
+// workgroup takes at most 512 threads x 16 elements x 8 bytes (padded, 70 KB) per
+// buffer then, and a one-wave workgroup has no barriers to save.
+template <typename R, int LOG2N, int T, int NLK>
+__host__ __device__ constexpr bool rks_two_buffers() {
+  return NLK != NLK_HANKEL && T > 64 && ((1 << LOG2N) / T) * (int)sizeof(cx<R>) <= 128;
+}
+
+// LDS elements of the exchange buffers
+template <typename R, int LOG2N, int T, int NLK>
+__host__ __device__ constexpr int rks_buf_elems() {
+  return rksfft::padded_size(1 << LOG2N) * (rks_two_buffers<R, LOG2N, T, NLK>() ? 2 : 1);
+}
+
+// LDS bytes of the persistent kernel: exchange buffers + twiddle tables (Hankel:
+// the stage values and the |f|^2 f vector)
+template <typename R, int LOG2N, int T, int NLK>
+__host__ __device__ constexpr int rks_lds_bytes() {
+  return (rks_buf_elems<R, LOG2N, T, NLK>() + (NLK == NLK_HANKEL ? (1 << LOG2N) : rksfft::TwSplit<LOG2N>::SIZE)) *
+         (int)sizeof(cx<R>);
 }
 
 // Hankel kind: yk = Y (nr x nr, row-major, engine precision), hs = S.  Each thread
@@ -748,35 +841,39 @@ __device__ __forceinline__ void fill_nl(GetK getk, cx<R>* buf, const R* __restri
 // (buf) and |f|^2 f (the second LDS vector) are read by every lane at the same
 // index, so LDS serves them as broadcasts.  Arithmetic as the batched transform
 // (rks_hankel.hip): f = (1/S) sum, |f|^2 f, then i gamma (S sum).
-template <typename R, typename RN, int LOG2N, int T, int NLK>
-__device__ __attribute__((noinline)) void nl_core(cx<R>* buf, const cx<R>* twl, R coef, cx<RN>* __restrict__ dst,
-                                                  const R* __restrict__ yk, int nr, double hs) {
+template <typename R, int LOG2N, int T, int MPT>
+__device__ __forceinline__ void nl_hankel(cx<R> (&v)[MPT], cx<R>* buf, R coef, const R* __restrict__ yk, int nr,
+                                          double hs) {
   using C = cx<R>;
-  using rksfft::pad;
   constexpr int N = 1 << LOG2N;
   const int t = threadIdx.x;
-  const R inv = (R)1 / (R)N;
+  C* w = buf + rksfft::padded_size(N);
+  const R ci = (R)(1.0 / hs), cs = (R)hs;
+#pragma unroll
+  for (int i = 0; i < MPT; ++i)
+    if (t + i * T < nr) buf[t + i * T] = v[i];
   __syncthreads();
-  if constexpr (NLK == NLK_HANKEL) {
-    C* w = buf + rksfft::padded_size(N);
-    const R ci = (R)(1.0 / hs), cs = (R)hs;
-    for (int r = t; r < nr; r += T) {
-      const R* __restrict__ y = yk + (size_t)r * nr;
-      R ar = (R)0, ai = (R)0;
-      for (int k = 0; k < nr; ++k) {
-        const R yv = y[k];
-        const C x = buf[k];
-        ar = fma(yv, x.re, ar);
-        ai = fma(yv, x.im, ai);
-      }
-      R vr = ci * ar, vi = ci * ai;
-      const R m2 = vr * vr + vi * vi;
-      vr *= m2;
-      vi *= m2;
-      w[r] = mkc(vr, vi);
+#pragma unroll 1
+  for (int r = t; r < nr; r += T) {
+    const R* __restrict__ y = yk + (size_t)r * nr;
+    R ar = (R)0, ai = (R)0;
+    for (int k = 0; k < nr; ++k) {
+      const R yv = y[k];
+      const C x = buf[k];
+      ar = fma(yv, x.re, ar);
+      ai = fma(yv, x.im, ai);
     }
-    __syncthreads();
-    for (int r = t; r < nr; r += T) {
+    R vr = ci * ar, vi = ci * ai;
+    const R m2 = vr * vr + vi * vi;
+    vr *= m2;
+    vi *= m2;
+    w[r] = mkc(vr, vi);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < MPT; ++i) {
+    const int r = t + i * T;
+    if (r < nr) {
       const R* __restrict__ y = yk + (size_t)r * nr;
       R ar = (R)0, ai = (R)0;
       for (int k = 0; k < nr; ++k) {
@@ -786,58 +883,115 @@ __device__ __attribute__((noinline)) void nl_core(cx<R>* buf, const cx<R>* twl, 
         ai = fma(yv, x.im, ai);
       }
       const R vr = cs * ar, vi = cs * ai;
-      dst[r] = mkc((RN)(-coef * vi), (RN)(coef * vr));
-    }
-  } else if constexpr (NLK == NLK_CUBIC) {
-    // |v|^2 v applied as the inverse transform's last pass produces v, and the
-    // forward transform's last pass writes i coef w straight to dst
-    rksfft::fft_post<R, N, T, true, LOG2N, RKS_MAXR>(buf, twl, [&](int x, C w) {
-      const C v = inv * w;
-      const R a = v.re * v.re + v.im * v.im;
-      buf[pad(x)] = a * v;
-    });
-    __syncthreads();
-    rksfft::fft_post<R, N, T, false, LOG2N, RKS_MAXR>(
-        buf, twl, [&](int x, C w) { dst[x] = mkc((RN)(-coef * w.im), (RN)(coef * w.re)); });
-  } else {
-    constexpr int M = N / 2 + 1;
-    constexpr int MPT = (M + T - 1) / T;
-    constexpr int H = N / 2;
-    rksfft::fft<R, N, T, true, LOG2N, RKS_MAXR>(buf, twl);
-    C zz[H / T];
-#pragma unroll
-    for (int i = 0; i < H / T; ++i) {
-      const int j = t + i * T;
-      const C a = buf[pad(2 * j)], b = buf[pad(2 * j + 1)];
-      zz[i] = mkc((a.re * inv) * (a.im * inv), (b.re * inv) * (b.im * inv));
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < H / T; ++i) buf[pad(t + i * T)] = zz[i];
-    __syncthreads();
-    rksfft::fft<R, H, T, false, LOG2N, RKS_MAXR>(buf, twl);
-#pragma unroll
-    for (int i = 0; i < MPT; ++i) {
-      const int m = t + i * T;
-      if (m < M) {
-        const C Zk = buf[pad(m & (H - 1))];
-        const C Zc = conjc(buf[pad((H - m) & (H - 1))]);
-        const C E = (R)0.5 * (Zk + Zc);
-        const C D = Zk - Zc;
-        const C O = mkc((R)0.5 * D.im, (R)-0.5 * D.re);
-        const C W = E + rksfft::twiddle<R, LOG2N>(twl, m) * O;
-        dst[m] = cvt<RN>(coef * W);
-      }
+      v[i] = mkc(-coef * vi, coef * vr);
     }
   }
   __syncthreads();
 }
 
-template <typename R, typename RN, int LOG2N, int T, int NLK, typename GetK>
-__device__ __forceinline__ void eval_nl(GetK getk, cx<R>* buf, const cx<R>* twl, const R* __restrict__ kx, R coef,
-                                        cx<RN>* __restrict__ dst, int sym, int mlim, double hs) {
-  fill_nl<R, LOG2N, T, NLK>(getk, buf, kx, sym, mlim);
-  nl_core<R, RN, LOG2N, T, NLK>(buf, twl, coef, dst, kx, mlim, hs);
+// Slots whose imaginary parts of U + iV take the product unrounded.  On a spectrum that
+// reaches the grid's end k U outweighs U a thousandfold and a run that is not resolved
+// amplifies the last bit, so the choice, once made, is kept.
+template <int T>
+__device__ __forceinline__ constexpr bool fused_imag(int k) {
+  return k >= 1 && k <= (T == 512 ? 6 : T == 256 ? 4 : 0);
+}
+
+template <typename R, int LOG2N, int T, int NLK, int MPT>
+__device__ __forceinline__ void nl_regs(cx<R> (&v)[MPT], cx<R>* buf, const cx<R>* twl, R coef,
+                                        const R* __restrict__ kx, int nr, double hs) {
+  using C = cx<R>;
+  using rksfft::pad;
+  constexpr int N = 1 << LOG2N;
+  constexpr bool PP = rks_two_buffers<R, LOG2N, T, NLK>();
+  constexpr int PS = rksfft::padded_size(N);
+  const int t = threadIdx.x;
+  const R inv = (R)1 / (R)N;
+  if constexpr (NLK == NLK_HANKEL) {
+    nl_hankel<R, LOG2N, T, MPT>(v, buf, coef, kx, nr, hs);
+  } else if constexpr (NLK == NLK_CUBIC) {
+    constexpr int X = rksfft::exchanges<N, T, RKS_MAXR>();
+    rksfft::fft_reg<R, N, T, true, LOG2N, RKS_MAXR, PP, 0, true>(v, buf, twl, [&](C w) {
+      const C v1 = inv * w;
+      const R a = v1.re * v1.re + v1.im * v1.im;
+      return a * v1;
+    });
+    rksfft::fft_reg<R, N, T, false, LOG2N, RKS_MAXR, PP, X & 1, false>(v, buf, twl,
+                                                               [&](C w) { return mkc(-coef * w.im, coef * w.re); });
+    if constexpr (PP) __syncthreads();
+  } else {
+    // inverse transform of the spectrum of u + i u_x: Y[m] = U + iV, Y[N-m] = conj(U) +
+    // i conj(V); DC and Nyquist keep only the real parts, as irfft does.  The lower half
+    // is the thread's own, the upper half comes from its mirror through LDS.
+    constexpr int H = N / 2, E = N / T, EH = E / 2;
+    static_assert(MPT == EH + 1 && EH >= 2, "rfft layout");
+    constexpr int XI = rksfft::exchanges<N, T, RKS_MAXR>(), XF = rksfft::exchanges<H, T, RKS_MAXR>();
+    C y[E];
+#pragma unroll
+    for (int k = 0; k < MPT; ++k) {
+      if (k == EH && t != 0) continue;
+      const int m = t + k * T;
+      const C U = v[k];
+      const R q = gload_real(kx, m);
+      const R vr = scaled_re(-q, U.im);  // V = i q U
+      C lo = mkc(fma(-q, U.re, U.re), add_re(U.im, vr));
+      C up = mkc(fma(q, U.re, U.re), add_re(vr, -U.im));
+      if (fused_imag<T>(k)) {
+        lo.im = fma(-q, U.im, U.im);
+        up.im = fma(-q, U.im, -U.im);
+      }
+      const C edge = mkc(U.re, vr);
+      if (k == EH) {
+        buf[0] = edge;
+      } else if (k == 0) {
+        // m = 0 keeps the real parts and has no mirror
+        y[0] = t == 0 ? edge : lo;
+        if (t != 0) buf[pad(H - m)] = up;
+      } else {
+        y[k] = lo;
+        buf[pad(H - m)] = up;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < EH; ++k) y[EH + k] = buf[pad(t + k * T)];
+    if constexpr (!PP) __syncthreads();
+    rksfft::fft_reg<R, N, T, true, LOG2N, RKS_MAXR, PP, 1, true>(y, buf, twl, [](C w) { return w; });
+    // u u_x, a real sequence: complex element j of its half-length transform is the pair 2j, 2j+1
+    constexpr int B2 = PP ? (1 + XI) & 1 : 0;
+    C* const bp = buf + B2 * PS;
+#pragma unroll
+    for (int k = 0; k < E; ++k) {
+      const int x = t + k * T;
+      ((R*)(bp + pad(x >> 1)))[x & 1] = (y[k].re * inv) * (y[k].im * inv);
+    }
+    __syncthreads();
+    C z[EH];
+#pragma unroll
+    for (int k = 0; k < EH; ++k) z[k] = bp[pad(t + k * T)];
+    if constexpr (!PP) __syncthreads();
+    constexpr int B3 = PP ? (B2 + 1) & 1 : 0;
+    rksfft::fft_reg<R, H, T, false, LOG2N, RKS_MAXR, PP, B3, true>(z, buf, twl, [](C w) { return w; });
+    constexpr int B4 = PP ? (B3 + XF) & 1 : 0;
+    C* const bm = buf + B4 * PS;
+#pragma unroll
+    for (int k = 0; k < EH; ++k) bm[pad(t + k * T)] = z[k];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < MPT; ++k) {
+      if (k == EH && t != 0) continue;
+      const int m = t + k * T;
+      C Zk = k < EH ? z[k < EH ? k : 0] : z[0];
+      rksfft::leaf(Zk);
+      const C Zc = conjc(bm[pad((H - m) & (H - 1))]);
+      const C Ev = (R)0.5 * (Zk + Zc);
+      const C D = Zk - Zc;
+      const C O = mkc((R)0.5 * D.im, (R)-0.5 * D.re);
+      const C W = Ev + rksfft::twiddle<R, LOG2N>(twl, m) * O;
+      v[k] = coef * W;
+    }
+    __syncthreads();
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -960,81 +1114,115 @@ __device__ __forceinline__ double learned_after_accept(const rks_launch& P, cons
 }
 
 // ---------------------------------------------------------------------------
-// one instance: evolve / step / nl / coefficients
+// one instance: evolve / step / nl
 // ---------------------------------------------------------------------------
+// Modes per chunk of the literal stage sums: what a chunk loads is in flight in registers
+// together (up to 12 values per mode), beside the stage value and the last NL value.
+template <typename R>
+__host__ __device__ constexpr int rks_sum_chunk() {
+  return sizeof(R) == 4 ? 8 : 4;
+}
+
+// Argument of stage s for a method known at compile time.
+template <typename TT, int S, typename RS, typename RN, int MPT, typename OW, typename SlotF>
+__device__ __forceinline__ void stage_switch(int s, cx<RS> (&acc)[MPT], const cx<RN> (&nv)[MPT], const cx<RS>* u,
+                                             const OW& ow, SlotF slotp, const char* cbase, size_t Mc, double h) {
+  if constexpr (S < TT::tab.nstage && TT::tab.st[S < TT::tab.nstage ? S : 0].has_nl) {
+    // the evaluation just before stage S > 0 is that of stage S - 1
+    constexpr int NEW = S > 0 ? TT::tab.st[S > 0 ? S - 1 : 0].nl_slot : -1;
+    if (s == S) stage_sum<TT, S, NEW, 0, rks_sum_chunk<RS>()>(acc, nv, u, ow, slotp, cbase, Mc, h);
+    else stage_switch<TT, S + 1>(s, acc, nv, u, ow, slotp, cbase, Mc, h);
+  }
+}
+
 // Returns nonzero (proposer variant only) when the evolve stopped after an
 // accepted step for the proposer: the state is in the instance record, and the
 // caller runs learned_between_steps and calls again with reenter set.
-template <typename R, typename RN, int LOG2N, int T, int NLK, bool LEARN>
+template <typename R, typename RN, int LOG2N, int T, int NLK, bool LEARN, int METH>
 __device__ int run_instance(const rks_launch& P, int idx, cx<R>* buf, const cx<R>* twl, double* red,
                             int* lds_count, bool reenter) {
   using C = cx<R>;
   using CN = cx<RN>;
   constexpr int N = 1 << LOG2N;
   constexpr int M = (NLK == NLK_ADVECT) ? N / 2 + 1 : N;
-  constexpr int MPT = (M + T - 1) / T;
+  using OW = Own<N, M, T, NLK>;
+  constexpr int MPT = OW::MPT;
   constexpr int CH = Chunk<MPT>::CH;
+  constexpr bool METHOD = METH != RKS_METH_ANY;
+  using TT = MethodTab<METHOD ? METH : 0, (int)sizeof(C), (int)sizeof(CN), NLK == NLK_ADVECT>;
+  constexpr bool FUSED = TT::tab.st[TT::tab.nstage - 1].has_nl == 0;  // (METHOD) no NL in the last stage
+  constexpr int LAST_SLOT = TT::tab.st[FUSED ? TT::tab.nstage - 2 : TT::tab.nstage - 1].nl_slot;
   const rks_tableau* __restrict__ tbp = P.tab;
   const rks_ctrl* __restrict__ ctp = P.ctl;
   const rks_tableau& tb = *tbp;
   const rks_ctrl& ct = *ctp;
-  rks_inst* in = P.inst + idx;
+  rks_inst* in = uni(P.inst + idx);
   const rks_io io = P.io[idx];
   const int t = threadIdx.x;
-  const R* kx = (const R*)in->kx;
-  const R nlc = (R)in->nl_coef;
-  const double* Ld = in->L;
-  const int Lc = in->L_complex;
+  const R* kx = uni((const R*)in->kx);
+  const R nlc = (R)uni(in->nl_coef);
+  const double* Ld = uni(in->L);
+  const int Lc = uni(in->L_complex);
   // workspace: nslot NL arrays (RN) | 2 candidate states (R) | coefficients
   // (each region 256-byte aligned; layout computed by the host, rks_ws_layout)
-  char* ws = (char*)in->ws;
-  const int nslot = tb.nslot;
-  CN* slot_base = (CN*)ws;
+  char* ws = uni((char*)in->ws);
+  const int nslot = METHOD ? TT::tab.nslot : tb.nslot;
+  CN* const slot_base = (CN*)ws;
   C* const cand0 = (C*)(ws + rks_align256((size_t)nslot * M * sizeof(CN)));
   C* const cand1 = cand0 + rks_align256((size_t)M * sizeof(C)) / sizeof(C);
   char* cbase = (char*)(cand1 + rks_align256((size_t)M * sizeof(C)) / sizeof(C));
   // mirror-symmetric L (complex state): coefficients of modes 0..N/2 in
   // arrays of stride Mc (a multiple of 64 modes, at most M)
-  const int sym = (M == N) && in->coef_sym;
+  const int sym = (M == N) && uni(in->coef_sym);
   constexpr int MSYM = ((N / 2 + 1 + 63) / 64) * 64 < M ? ((N / 2 + 1 + 63) / 64) * 64 : M;
   const int Mc = sym ? MSYM : M;
   // modes in use: the Hankel kind's nr radial points (arrays keep the stride M of
   // its size class), every mode otherwise
-  const int Mr = NLK == NLK_HANKEL ? in->m : M;
+  const int Mr = NLK == NLK_HANKEL ? uni(in->m) : M;
   const int Mg = sym ? N / 2 + 1 : Mr;
-  const double hs = in->nl_scale;
-  // the modes this thread owns, chunk c
-  auto own = [&](int c) { return own_chunk<N, M, T, CH, (M == N && NLK != NLK_HANKEL)>(c, sym, Mr); };
+  const double hs = uni(in->nl_scale);
+  OW ow;
+  ow.lim = Mr;
+  ow.fold = sym ? N : 0;
+  ow.t = t;
+  const C* const uin = uni((const C*)io.u_in);
+  // the thread's modes of an array, and back
+  auto load_modes = [&](C(&v)[MPT], const C* src) {
+    const OW of = ow.fresh();
+#pragma unroll
+    for (int k = 0; k < MPT; ++k) v[k] = gload(src, of.m(k));
+  };
+  auto copy_modes = [&](C* dst, const C* src) {
+    C v[MPT];
+    load_modes(v, src);
+#pragma unroll
+    for (int k = 0; k < MPT; ++k)
+      if (ow.ok(k)) gstore(dst, ow.m(k), v[k]);
+  };
 
   if (P.mode == RKS_MODE_NL) {
-    const C* u = (const C*)io.u_in;
-    auto getu = [&](const ChunkIdx<CH>& ix, C(&acc)[CH]) {
+    C v[MPT];
+    load_modes(v, uin);
+    nl_regs<R, LOG2N, T, NLK>(v, buf, twl, nlc, kx, Mr, hs);
+    C* out = uni((C*)io.u_out);
 #pragma unroll
-      for (int i = 0; i < CH; ++i) acc[i] = ix.ok[i] ? u[ix.m[i]] : mkc((R)0, (R)0);
-    };
-    eval_nl<R, R, LOG2N, T, NLK>(getu, buf, twl, kx, nlc, (C*)io.u_out, 0, Mr, hs);
-    return 0;
-  }
-  if (P.mode == RKS_MODE_COEFFS) {
-    for (int i = 0; i < MPT; ++i) {
-      const int m = t + i * T;
-      if (m < Mr) coef_mode<R, RN>(tb, ct, Ld, Lc, m, M, P.h_mode, cbase);
-    }
+    for (int k = 0; k < MPT; ++k)
+      if (ow.ok(k)) gstore(out, ow.m(k), v[k]);
     return 0;
   }
 
   // ---- load persistent state (uniform across the workgroup) ----
-  double tc = in->tc, tf = in->tf, h = in->h, h_coeff = in->h_coeff, h_next = in->h_next;
-  double h_used = in->h_used;
-  int started = in->started, accept = in->accept, steps = in->steps, attempts = in->attempts;
-  int rejects = in->rejects, status = in->status, ubuf = in->ubuf;
-  int log_count = in->log_count, snap_count = in->snap_count;
-  int nl_calls = in->nl_calls, coef_updates = in->coef_updates;
+  double tc = uni(in->tc), tf = uni(in->tf), h = uni(in->h), h_coeff = uni(in->h_coeff), h_next = uni(in->h_next);
+  double h_used = uni(in->h_used);
+  int started = uni(in->started), accept = uni(in->accept), steps = uni(in->steps), attempts = uni(in->attempts);
+  int rejects = uni(in->rejects), status = uni(in->status), ubuf = uni(in->ubuf);
+  int log_count = uni(in->log_count), snap_count = uni(in->snap_count);
+  int nl_calls = uni(in->nl_calls), coef_updates = uni(in->coef_updates);
   // slot map packed 4 bits per slot (no dynamically indexed register array)
   unsigned smap = 0;
 #pragma unroll
-  for (int s = 0; s < RKS_MAX_SLOTS; ++s) smap |= (unsigned)(in->slot_map[s] & 15) << (4 * s);
-  const int store_freq = in->store_freq, snap_cap = in->snap_cap, log_cap = in->log_cap;
+  for (int s = 0; s < RKS_MAX_SLOTS; ++s) smap |= (unsigned)(uni(in->slot_map[s]) & 15) << (4 * s);
+  const int store_freq = uni(in->store_freq), snap_cap = uni(in->snap_cap), log_cap = uni(in->log_cap);
 
   if (io.reset && !reenter) {
     started = 0;
@@ -1042,22 +1230,22 @@ __device__ int run_instance(const rks_launch& P, int idx, cx<R>* buf, const cx<R
     h_coeff = __builtin_nan("");
     smap = 0x76543210u;
   }
+  const bool adaptive = METHOD ? TT::tab.adaptive != 0 : tb.adaptive != 0;
   const bool evolve = (P.mode == RKS_MODE_EVOLVE);
-  const C* uin = (const C*)io.u_in;
   if (reenter) {
     // back from the proposer: h_next holds its proposal (solveras.py:638-641)
     status = RKS_ST_RUNNING;
-    h = (tc + h_next > tf) ? tf - tc : h_next;
+    h = uni((tc + h_next > tf) ? tf - tc : h_next);
   } else if (evolve && !io.resume) {
-    tc = io.t0;
-    tf = io.tf;
-    h = io.h_in;
+    tc = uni(io.t0);
+    tf = uni(io.tf);
+    h = uni(io.h_in);
     steps = attempts = rejects = 0;
     log_count = snap_count = 0;
     nl_calls = coef_updates = 0;
     ubuf = -1;
     status = RKS_ST_RUNNING;
-    if (tb.adaptive && tc + h > tf) h = tf - tc;  // solveras.py:620-621
+    if (adaptive && tc + h > tf) h = uni(tf - tc);  // solveras.py:620-621
     if (LEARN && in->rec != nullptr) {
       // record counters live in the instance record: the stepping loop does not carry them
       __syncthreads();
@@ -1069,24 +1257,23 @@ __device__ int run_instance(const rks_launch& P, int idx, cx<R>* buf, const cx<R
       __syncthreads();
     }
     if (store_freq > 0) {
-      for (int i = 0; i < MPT; ++i) {
-        const int m = t + i * T;
-        if (m < Mr) ((C*)in->snap)[m] = uin[m];
-      }
+      copy_modes(uni((C*)in->snap), uin);
       if (t == 0) in->snap_t[0] = tc;
       snap_count = 1;
     }
   } else if (evolve) {
     status = RKS_ST_RUNNING;
   } else {
-    h = io.h_in;
+    h = uni(io.h_in);
     status = RKS_ST_RUNNING;
     attempts = rejects = 0;
   }
 
   auto slot = [&](int s) -> CN* { return slot_base + (size_t)((smap >> (4 * s)) & 15u) * M; };
   auto cur_u = [&]() -> const C* { return ubuf < 0 ? uin : (const C*)(ubuf == 0 ? cand0 : cand1); };
-  const bool fused = rks_fused_final(tb);
+  const bool fused = METHOD ? FUSED : rks_fused_final(tb);
+  const bool recompute = (METHOD ? TT::tab.nl1_policy : tb.nl1_policy) == RKS_NL1_RECOMPUTE;
+  const int nstage = METHOD ? TT::tab.nstage : tb.nstage;
 
   bool done = false;
   int pending = 0;      // proposer variant: stopped after an accept for the proposer
@@ -1102,141 +1289,222 @@ __device__ int run_instance(const rks_launch& P, int idx, cx<R>* buf, const cx<R
         break;
       }
     }
-    const C* u = evolve ? cur_u() : uin;
-    C* cand = evolve ? (ubuf == 0 ? cand1 : cand0) : (C*)io.u_out;
+    const C* u = uni(evolve ? cur_u() : uin);
+    C* cand = uni(evolve ? (ubuf == 0 ? cand1 : cand0) : (C*)io.u_out);
     int numloops = 0;
     double h_suggest = h;
     double s_acc;  // s of the accepted attempt (set where the attempt loop accepts)
     // ---------------- attempt loop (solveras.py:384-410) ----------------
     for (;;) {
       if (h != h_coeff) {
-        coef_update<R, RN, T, MPT>(tb, ct, Ld, Lc, Mc, Mg, h, cbase, (int*)buf, lds_count);
+        if constexpr (METHOD)
+          coef_update_method<TT, R, RN, T, MPT>(ct, Ld, Mc, Mg, h, cbase, (int*)buf, lds_count);
+        else
+          coef_update<R, RN, T, MPT>(tb, ct, Ld, Lc, Mc, Mg, h, cbase, (int*)buf, lds_count);
         h_coeff = h;
         ++coef_updates;
       }
-      auto getu = [&](const ChunkIdx<CH>& ix, C(&acc)[CH]) {
-#pragma unroll
-        for (int i = 0; i < CH; ++i) acc[i] = ix.ok[i] ? u[ix.m[i]] : mkc((R)0, (R)0);
-      };
+      bool first_nl = false;  // NL1 = nl(u) before the first stage
       if (!started) {
-        eval_nl<R, RN, LOG2N, T, NLK>(getu, buf, twl, kx, nlc, slot(0), sym, Mr, hs);
-        ++nl_calls;
+        first_nl = true;
         started = 1;
-      } else if (accept || !tb.adaptive) {
-        if (tb.nl1_policy == RKS_NL1_RECOMPUTE) {
-          eval_nl<R, RN, LOG2N, T, NLK>(getu, buf, twl, kx, nlc, slot(0), sym, Mr, hs);
-          ++nl_calls;
+      } else if (accept || !adaptive) {
+        if (recompute) {
+          first_nl = true;
         } else {
-          const unsigned f4 = 4u * (unsigned)tb.fsal_slot;
+          const unsigned f4 = 4u * (unsigned)(METHOD ? TT::tab.fsal_slot : tb.fsal_slot);
           const unsigned a = smap & 15u, b = (smap >> f4) & 15u;
           smap = (smap & ~(15u | (15u << f4))) | b | (a << f4);
         }
       }
-      // max |u_new| is taken where the candidate is formed; with the fused final
-      // stage the per-mode |u_new| and |err|^2 (FP32 buffer: |err|) wait in the (idle) LDS buffer
-      double mx = 0.0;
-      for (int s = 0; s < tb.nstage; ++s) {
-        const rks_stage& S = tb.st[s];
-        const bool last = (s == tb.nstage - 1);
-        if (last && fused) {
-          __syncthreads();  // the previous stage's write-back still reads buf
-#pragma unroll 1
-          for (int c = 0; c < Chunk<MPT>::NCH; ++c) {
-            const ChunkIdx<CH> ix = own(c);
-            C acc[CH], ev[CH];
-            final_chunk<R, RN, CH>(tb, u, slot, cbase, (size_t)Mc, ix, h, acc, ev);
+      double mx = 0.0;    // max |u_new| (fused last stage) or |u_new|^2
+      double su = 0.0, se = 0.0;
+      CN nv[MPT];         // NL values of the last evaluation
 #pragma unroll
-            for (int i = 0; i < CH; ++i) {
-              const int m = ix.m[i];
-              if (ix.ok[i]) {
-                cand[m] = acc[i];
-                const double a = hypot((double)acc[i].re, (double)acc[i].im);
-                const double er = (double)ev[i].re, ei = (double)ev[i].im;
-                mx = nanmax(mx, a);
-                // FP64 keeps |err|^2; an FP32 buffer keeps |err| (|err|^2 would flush to zero
-                // below ~1e-19 and turn a real error into an unconditional accept)
-                if constexpr (sizeof(R) == sizeof(double)) buf[m] = mkc((R)a, (R)(er * er + ei * ei));
-                else buf[m] = mkc((R)a, (R)hypot(er, ei));
+      for (int k = 0; k < MPT; ++k) nv[k] = mkc((RN)0, (RN)0);
+#pragma unroll 1
+      for (int s = first_nl ? -1 : 0; s < nstage; ++s) {
+        const bool last = s == nstage - 1;
+        C v[MPT];
+        int ns = 0;  // NL slot this pass writes
+        if (s < 0) {
+          load_modes(v, u);
+        } else if constexpr (METHOD) {
+          if (FUSED && last) break;
+          stage_switch<TT, 0>(s, v, nv, u, ow, slot, cbase, (size_t)Mc, h);
+          if (!FUSED && last) {
+#pragma unroll
+            for (int k = 0; k < MPT; ++k) {
+              if (ow.ok(k)) {
+                gstore(cand, ow.m(k), v[k]);
+                if (TT::tab.adaptive)
+                  mx = nanmax(mx, (double)v[k].re * (double)v[k].re + (double)v[k].im * (double)v[k].im);
               }
             }
           }
-          continue;
-        }
-        auto getk = [&](const ChunkIdx<CH>& ix, C(&acc)[CH]) {
-          stage_chunk<R, RN, CH>(tb, S, u, slot, cbase, (size_t)Mc, ix, h, acc);
-          if (last) {
-#pragma unroll
-            for (int i = 0; i < CH; ++i)
-              if (ix.ok[i]) {
-                cand[ix.m[i]] = acc[i];
-                if (tb.adaptive) mx = nanmax(mx, hypot((double)acc[i].re, (double)acc[i].im));
-              }
-          }
-        };
-        if (S.has_nl) {
-          eval_nl<R, RN, LOG2N, T, NLK>(getk, buf, twl, kx, nlc, slot(S.nl_slot), sym, Mr, hs);
-          ++nl_calls;
+          static_assert(TT::tab.st[0].nl_slot == 1 && LAST_SLOT == TT::tab.nslot - 1, "stage s writes slot s + 1");
+          ns = s + 1;
         } else {
+          const rks_stage& S = tb.st[s];
+          if (last && fused) {
+            // per-mode |u_new| and |err|^2 (FP32 buffer: |err|) wait in the idle LDS buffer
+#pragma unroll 1
+            for (int c = 0; c < Chunk<MPT>::NCH; ++c) {
+              const ChunkIdx<CH> ix = own_chunk<N, M, T, NLK, CH>(c, ow);
+              C acc[CH], ev[CH];
+              final_chunk<R, RN, CH>(tb, u, slot, cbase, (size_t)Mc, ix, h, acc, ev);
+#pragma unroll
+              for (int i = 0; i < CH; ++i) {
+                const int m = ix.m[i];
+                if (ix.ok[i]) {
+                  cand[m] = acc[i];
+                  const double a = hypot((double)acc[i].re, (double)acc[i].im);
+                  const double er = (double)ev[i].re, ei = (double)ev[i].im;
+                  mx = nanmax(mx, a);
+                  // FP64 keeps |err|^2; an FP32 buffer keeps |err| (|err|^2 would flush to zero
+                  // below ~1e-19 and turn a real error into an unconditional accept)
+                  if constexpr (sizeof(R) == sizeof(double)) buf[m] = mkc((R)a, (R)(er * er + ei * ei));
+                  else buf[m] = mkc((R)a, (R)hypot(er, ei));
+                }
+              }
+            }
+            break;
+          }
+          // the stage argument through the thread's own places of the LDS buffer: the
+          // run-time term loop stays rolled over the chunks
 #pragma unroll 1
           for (int c = 0; c < Chunk<MPT>::NCH; ++c) {
+            const ChunkIdx<CH> ix = own_chunk<N, M, T, NLK, CH>(c, ow);
             C acc[CH];
-            getk(own(c), acc);
+            stage_chunk<R, RN, CH>(tb, S, u, slot, cbase, (size_t)Mc, ix, h, acc);
+#pragma unroll
+            for (int i = 0; i < CH; ++i) {
+              if (!ix.ok[i]) continue;
+              if (last) {
+                cand[ix.m[i]] = acc[i];
+                if (adaptive)
+                  mx = nanmax(mx, (double)acc[i].re * (double)acc[i].re + (double)acc[i].im * (double)acc[i].im);
+              }
+              buf[ix.m[i]] = acc[i];
+            }
           }
+          if (!S.has_nl) continue;
+#pragma unroll
+          for (int k = 0; k < MPT; ++k) v[k] = buf[ow.m(k)];
+          __syncthreads();
+          ns = S.nl_slot;
+        }
+        nl_regs<R, LOG2N, T, NLK>(v, buf, twl, nlc, kx, Mr, hs);
+        ++nl_calls;
+        CN* const dst = slot(ns);
+        const OW of = ow.fresh();
+#pragma unroll
+        for (int k = 0; k < MPT; ++k) {
+          nv[k] = cvt<RN>(v[k]);
+          if (of.ok(k)) gstore(dst, of.m(k), nv[k]);
         }
       }
-      if (!tb.adaptive) {
+      if (!adaptive) {
         h_suggest = h;
         accept = 1;
         break;
       }
       // ---------------- embedded error norm (solveras.py:449-455) ----------------
-      // max |u_new| (taken above); masked sums of |u_new|^2 and |err|^2 (FP64)
-      mx = wg_max<T>(mx, red);
-      double su = 0.0, se = 0.0;
-      // each thread reads back the modes it wrote (own_chunk)
-      if (fused) {
+      // masked sums of |u_new|^2 and |err|^2 (FP64) over |u_new| / max |u_new| > cutoff.  Where
+      // the last stage has no NL, |u_new| is kept (mx: its maximum), else its square; the mask
+      // compares those instead of dividing.  A square that overflows or vanishes does so in the
+      // sums as well, and the attempt is rejected either way.
+      const double cut = ct.adapt_cutoff;
+      if constexpr (METHOD) {
+#pragma clang fp contract(off)
+        double a[MPT], e[MPT];
+        final_sum<TT, LAST_SLOT, 0, rks_sum_chunk<R>(), !FUSED>(a, e, cand, nv, u, ow, slot, cbase, (size_t)Mc, h);
+        if constexpr (FUSED) {
+#pragma unroll
+          for (int k = 0; k < MPT; ++k) mx = nanmax(mx, a[k]);
+        }
+        if constexpr (M == N && NLK != NLK_HANKEL) {
+          // into norm_mode's order through the idle buffer, where the proposer finds |u_new|
+          double* const db = (double*)buf;
+          constexpr bool PAIRS = FUSED || sizeof(R) == sizeof(double);  // both values fit an element
+#pragma unroll
+          for (int k = 0; k < MPT; ++k) {
+            if constexpr (PAIRS) buf[ow.m(k)] = mkc((R)a[k], (R)e[k]);
+            else db[ow.m(k)] = a[k];
+          }
+          __syncthreads();
+#pragma unroll
+          for (int k = 0; k < MPT; ++k) {
+            const int m = norm_mode<N, M, T, NLK>(k);
+            if constexpr (PAIRS) {
+              a[k] = (double)buf[m].re;
+              e[k] = (double)buf[m].im;
+            } else {
+              a[k] = db[m];
+            }
+          }
+          __syncthreads();
+          if constexpr (!PAIRS) {
+#pragma unroll
+            for (int k = 0; k < MPT; ++k) db[ow.m(k)] = e[k];
+            __syncthreads();
+#pragma unroll
+            for (int k = 0; k < MPT; ++k) e[k] = db[norm_mode<N, M, T, NLK>(k)];
+            __syncthreads();
+          }
+        } else if constexpr (LEARN && FUSED) {
+#pragma unroll
+          for (int k = 0; k < MPT; ++k)
+            if (ow.ok(k)) buf[ow.m(k)].re = (R)a[k];
+        }
+        mx = wg_max<T>(mx, red);
+        const double lim = FUSED ? cut * mx : (cut < 0.0 ? -1.0 : cut * cut * mx);
+#pragma unroll
+        for (int k = 0; k < MPT; ++k) {
+          const bool on = a[k] > lim && a[k] <= __DBL_MAX__;
+          const double x = on ? a[k] : 0.0, y = on ? e[k] : 0.0;
+          su = FUSED ? fma(x, x, su) : su + x;
+          se = (FUSED && sizeof(R) < sizeof(double)) ? fma(y, y, se) : se + y;
+        }
+      } else {
+#pragma clang fp contract(off)
+        mx = wg_max<T>(mx, red);
+        const double lim = fused ? cut * mx : (cut < 0.0 ? -1.0 : cut * cut * mx);
+        __syncthreads();  // every thread's last NL values, candidate and buffer values
 #pragma unroll 1
         for (int c = 0; c < Chunk<MPT>::NCH; ++c) {
-          const ChunkIdx<CH> ix = own(c);
+          ChunkIdx<CH> ix = own_chunk<N, M, T, NLK, CH>(c, ow);
+#pragma unroll
+          for (int i = 0; i < CH; ++i)
+            if (M == N && NLK != NLK_HANKEL) ix.m[i] = norm_mode<N, M, T, NLK>(c * CH + i);
+          C ev[CH];
+          if (!fused) error_chunk<R, RN, CH>(tb, slot, cbase, (size_t)Mc, ix, h, ev);
 #pragma unroll
           for (int i = 0; i < CH; ++i) {
             if (!ix.ok[i]) continue;
-            const C v = buf[ix.m[i]];
-            const double a = (double)v.re;
-            if (a / mx > ct.adapt_cutoff) {
-              su += a * a;
-              if constexpr (sizeof(R) == sizeof(double)) {
-                se += (double)v.im;
-              } else {
-                const double e = (double)v.im;
-                se += e * e;
+            if (fused) {
+              const C q = buf[ix.m[i]];
+              const double a = (double)q.re, e = (double)q.im;
+              if (a > lim && a <= __DBL_MAX__) {
+                su = fma(a, a, su);
+                se = sizeof(R) < sizeof(double) ? fma(e, e, se) : se + e;
+              }
+            } else {
+              const C kv = cand[ix.m[i]];
+              const double kr = (double)kv.re, ki = (double)kv.im, er = (double)ev[i].re, ei = (double)ev[i].im;
+              const double a = fma(kr, kr, ki * ki);
+              if (a > lim && a <= __DBL_MAX__) {
+                su += a;
+                se += fma(er, er, ei * ei);
               }
             }
           }
         }
-      } else {
-#pragma unroll 1
-      for (int c = 0; c < Chunk<MPT>::NCH; ++c) {
-        const ChunkIdx<CH> ix = own(c);
-        C ev[CH];
-        error_chunk<R, RN, CH>(tb, slot, cbase, (size_t)Mc, ix, h, ev);
-#pragma unroll
-        for (int i = 0; i < CH; ++i) {
-          const int m = ix.m[i];
-          if (ix.ok[i]) {
-            const C kv = cand[m];
-            const double kr = (double)kv.re, ki = (double)kv.im;
-            if (hypot(kr, ki) / mx > ct.adapt_cutoff) {
-              const double er = (double)ev[i].re, ei = (double)ev[i].im;
-              su += kr * kr + ki * ki;
-              se += er * er + ei * ei;
-            }
-          }
-        }
-      }
+        if (fused) __syncthreads();  // the buffer's values are read
       }
       wg_sum2<T>(su, se, red);
-      const double sv = rks_error_ratio(su, se, ct.epsilon, ct.safety_f, tb.q, sizeof(RN) < sizeof(double));
+      const int q = METHOD ? TT::tab.q : tb.q;
+      const double sv = uni(rks_error_ratio(su, se, ct.epsilon, ct.safety_f, q, sizeof(RN) < sizeof(double)));
       ++attempts;
       if (t == 0 && log_count < log_cap) {
         in->log[2 * log_count] = h;
@@ -1260,11 +1528,11 @@ __device__ int run_instance(const rks_launch& P, int idx, cx<R>* buf, const cx<R
         accept = 0;
         ++rejects;
         if (isinf(sv) || isnan(sv)) {
-          h = ct.min_s * h;
+          h = uni(ct.min_s * h);
         } else {
           double sc = sv > ct.min_s ? sv : ct.min_s;
           sc = sc < ct.decr_f ? sc : ct.decr_f;
-          h = sc * h;
+          h = uni(sc * h);
         }
         ++numloops;
         if (numloops > ct.max_loops) {
@@ -1283,7 +1551,7 @@ __device__ int run_instance(const rks_launch& P, int idx, cx<R>* buf, const cx<R
       accept = 1;
       s_acc = sv;
       const double sc = sv < ct.max_s ? sv : ct.max_s;
-      h_suggest = (sc > ct.incr_f) ? sc * h : h;
+      h_suggest = uni((sc > ct.incr_f) ? sc * h : h);
       break;
     }
     if (done) break;
@@ -1297,7 +1565,7 @@ __device__ int run_instance(const rks_launch& P, int idx, cx<R>* buf, const cx<R
     }
     ubuf = (ubuf == 0) ? 1 : 0;
     const double tprev = tc;
-    tc += h;
+    tc = uni(tc + h);
     ++steps;
     if (!(tc > tprev)) {
       // h below the resolution of tc: the reference would loop forever here;
@@ -1306,14 +1574,7 @@ __device__ int run_instance(const rks_launch& P, int idx, cx<R>* buf, const cx<R
       break;
     }
     if (store_freq > 0 && (steps % store_freq) == 0) {
-      C* dst = (C*)in->snap + (size_t)snap_count * Mr;
-      const C* src = cur_u();
-      for (int c = 0; c < Chunk<MPT>::NCH; ++c) {
-        const ChunkIdx<CH> ix = own(c);
-#pragma unroll
-        for (int i = 0; i < CH; ++i)
-          if (ix.ok[i]) dst[ix.m[i]] = src[ix.m[i]];
-      }
+      copy_modes(uni((C*)in->snap) + (size_t)snap_count * Mr, cur_u());
       if (t == 0) in->snap_t[snap_count] = tc;
       ++snap_count;
     }
@@ -1325,24 +1586,15 @@ __device__ int run_instance(const rks_launch& P, int idx, cx<R>* buf, const cx<R
       // outside this loop (the caller, learned_between_steps): a call here would keep
       // every loop-carried value live across it and spill inside the stage passes.
       const bool run_net = P.mlp.on && (steps % (P.mlp.period * (512 / T))) == 0;
-      if (tb.adaptive && tc < tf && (run_net || in->rec != nullptr)) {
+      if (adaptive && tc < tf && (run_net || in->rec != nullptr)) {
         pending = run_net ? 3 : 1;
         s_hand = s_acc;
         break;
       }
     }
-    if (tb.adaptive) h = (tc + h_suggest > tf) ? tf - tc : h_suggest;  // solveras.py:638-641
+    if (adaptive) h = uni((tc + h_suggest > tf) ? tf - tc : h_suggest);  // solveras.py:638-641
   }
-  if (evolve && status != RKS_ST_PAUSED && !pending) {
-    const C* src = cur_u();
-    C* dst = (C*)io.u_out;
-    for (int c = 0; c < Chunk<MPT>::NCH; ++c) {
-      const ChunkIdx<CH> ix = own(c);
-#pragma unroll
-      for (int i = 0; i < CH; ++i)
-        if (ix.ok[i]) dst[ix.m[i]] = src[ix.m[i]];
-    }
-  }
+  if (evolve && status != RKS_ST_PAUSED && !pending) copy_modes(uni((C*)io.u_out), cur_u());
   __syncthreads();
   if (t == 0) {
     in->tc = tc;
@@ -1414,7 +1666,9 @@ __host__ __device__ constexpr int rks_min_waves(int /*log2n*/, int /*state_bytes
 // keeps its register allocation.
 // TILE 1: twice the threads per trajectory (half the modes per thread in the
 // stage passes and FFTs), where every transform keeps >= 2 elements per thread.
-template <typename R, typename RN, int LOG2N, int NLK, bool LEARN, int TILE>
+// METH: one method's stage sums and coefficients as literals (rks_method.h), or
+// RKS_METH_ANY.
+template <typename R, typename RN, int LOG2N, int NLK, bool LEARN, int TILE, int METH>
 __global__ __launch_bounds__(rks_threads(LOG2N, NLK) << TILE, rks_min_waves(LOG2N, (int)sizeof(R))) void rks_kernel(
     rks_launch P) {
   constexpr int T = rks_threads(LOG2N, NLK) << TILE;
@@ -1431,47 +1685,33 @@ __global__ __launch_bounds__(rks_threads(LOG2N, NLK) << TILE, rks_min_waves(LOG2
   __shared__ float s_bins[LEARN ? 2 * RKS_MLP_NBIN : 1];
   __shared__ float s_scr[(LEARN && !kScrInBuf) ? RKS_MLP_LDS_FLOATS : 1];
   cx<R>* buf = (cx<R>*)rks_smem;
-  cx<R>* twl = buf + rksfft::padded_size(1 << LOG2N);
+  cx<R>* twl = buf + rks_buf_elems<R, LOG2N, T, NLK>();
   float* scr = kScrInBuf ? (float*)rks_smem : s_scr;
   if constexpr (NLK != NLK_HANKEL) rksfft::load_twiddles<R, LOG2N, T>(twl, (const cx<R>*)P.tw);
   for (;;) {
     if (threadIdx.x == 0) s_item = atomicAdd(P.queue, 1);
     __syncthreads();
-    const int item = s_item;
+    const int item = uni(s_item);
     __syncthreads();
     if (item >= P.count) break;
-    const int idx = P.order[item];
+    const int idx = uni(P.order[item]);
     if constexpr (LEARN && T >= 64) {
       bool reenter = false;
-      while (run_instance<R, RN, LOG2N, T, NLK, LEARN>(P, idx, buf, twl, red, &s_count, reenter)) {
+      while (run_instance<R, RN, LOG2N, T, NLK, LEARN, METH>(P, idx, buf, twl, red, &s_count, reenter)) {
         learned_between_steps<R, RN, LOG2N, T, NLK>(P, idx, buf, s_bins, scr);
         reenter = true;
       }
     } else {
-      run_instance<R, RN, LOG2N, T, NLK, LEARN>(P, idx, buf, twl, red, &s_count, false);
+      run_instance<R, RN, LOG2N, T, NLK, LEARN, METH>(P, idx, buf, twl, red, &s_count, false);
     }
     __syncthreads();
   }
 }
 
-
-// Explicit instantiations of one precision x nonlinearity (rks_k_*.hip): every
-// size, and the proposer variant for the sizes whose workgroups can be whole
-// waves (n >= 128; the host refuses smaller rfft grids).
-// The second tile (TILE 1) exists for n = 2^9 .. 2^12, with and without the proposer.
-#define RKS_KERNEL_SIZES(X, R, RN, NLK)                                                                      \
-  X(R, RN, 4, NLK, false, 0) X(R, RN, 5, NLK, false, 0) X(R, RN, 6, NLK, false, 0)                          \
-  X(R, RN, 7, NLK, false, 0) X(R, RN, 8, NLK, false, 0) X(R, RN, 9, NLK, false, 0)                          \
-  X(R, RN, 10, NLK, false, 0) X(R, RN, 11, NLK, false, 0) X(R, RN, 12, NLK, false, 0)                       \
-  X(R, RN, 13, NLK, false, 0) X(R, RN, 7, NLK, true, 0) X(R, RN, 8, NLK, true, 0) X(R, RN, 9, NLK, true, 0) \
-  X(R, RN, 10, NLK, true, 0) X(R, RN, 11, NLK, true, 0) X(R, RN, 12, NLK, true, 0)                          \
-  X(R, RN, 13, NLK, true, 0) X(R, RN, 9, NLK, false, 1) X(R, RN, 10, NLK, false, 1)                         \
-  X(R, RN, 11, NLK, false, 1) X(R, RN, 12, NLK, false, 1) X(R, RN, 9, NLK, true, 1)                         \
-  X(R, RN, 10, NLK, true, 1) X(R, RN, 11, NLK, true, 1) X(R, RN, 12, NLK, true, 1)
-// The Hankel kind: size classes 2^4 .. 2^10 (nr <= 1024 radial points), one tile.
-#define RKS_KERNEL_HANKEL_SIZES(X, R, RN)                                                                \
-  X(R, RN, 4, NLK_HANKEL, false, 0) X(R, RN, 5, NLK_HANKEL, false, 0) X(R, RN, 6, NLK_HANKEL, false, 0)  \
-  X(R, RN, 7, NLK_HANKEL, false, 0) X(R, RN, 8, NLK_HANKEL, false, 0) X(R, RN, 9, NLK_HANKEL, false, 0)  \
-  X(R, RN, 10, NLK_HANKEL, false, 0)
-#define RKS_INSTANTIATE(R, RN, L, K, LE, TI) template __global__ void rks_kernel<R, RN, L, K, LE, TI>(rks_launch);
-#define RKS_DECLARE(R, RN, L, K, LE, TI) extern template __global__ void rks_kernel<R, RN, L, K, LE, TI>(rks_launch);
+// What a launch needs of a kernel; the host's table of them is filled by the units that
+// instantiate the kernels (rks_k.hip, one per precision x nonlinearity x method).
+struct rks_kernel_entry {
+  const void* fn;
+  int threads;
+  int lds;
+};

@@ -16,6 +16,15 @@
 #define RKS_MAX_SLOTS 8
 #define RKS_COEF_ONE (-1)
 
+// method ids (rks_tableau.method)
+#define RKS_M_ETD35 0
+#define RKS_M_ETD34 1
+#define RKS_M_ETD4 2
+#define RKS_M_ETD5 3
+#define RKS_M_IF34 4
+#define RKS_M_IF45DP 5
+#define RKS_M_IF4 6
+
 // basis value kinds (rks_coef.kind)
 #define RKS_BASIS_EXP 0  // exp(f z)
 #define RKS_BASIS_PSI1 1 // h * psi1(f z)   (psi_r = r! phi_r)
