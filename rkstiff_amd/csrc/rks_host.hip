@@ -100,6 +100,14 @@ __global__ void rks_f64_to_f32(const double* a, float* b, int n) {
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) b[i] = (float)a[i];
 }
 
+// the Hankel matrix for the stepping kernels: transposed, engine precision
+template <typename R>
+__global__ void rks_transpose(const double* a, R* b, int n) {
+  const int total = n * n;
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < total; i += gridDim.x * blockDim.x)
+    b[i] = (R)a[(i % n) * n + i / n];
+}
+
 
 // ===========================================================================
 // host side: plans and the C ABI
@@ -449,7 +457,19 @@ int rks_plan_create(int method, int nl_kind, int precision, const rks_config* cf
     if (desc[i].kx) HIPCHK(hipMemcpy(d_kx64 + kxoff[i], desc[i].kx, sizeof(double) * nk, hipMemcpyDefault));
     else HIPCHK(hipMemset(d_kx64 + kxoff[i], 0, sizeof(double) * nk));
   }
-  if (precision != RKS_F32) {
+  if (hankel) {
+    for (int i = 0; i < ninst; ++i) {
+      if (!kx_copy[i]) continue;
+      const int m = p->modes[i];
+      if (precision != RKS_F32)
+        hipLaunchKernelGGL(rks_transpose<double>, dim3(256), dim3(256), 0, 0, d_kx64 + kxoff[i],
+                           (double*)p->d_kx + kxoff[i], m);
+      else
+        hipLaunchKernelGGL(rks_transpose<float>, dim3(256), dim3(256), 0, 0, d_kx64 + kxoff[i],
+                           (float*)p->d_kx + kxoff[i], m);
+      HIPCHK(hipGetLastError());
+    }
+  } else if (precision != RKS_F32) {
     HIPCHK(hipMemcpy(p->d_kx, d_kx64, kx_total * sizeof(double), hipMemcpyDeviceToDevice));
   } else if (kx_total) {
     hipLaunchKernelGGL(rks_f64_to_f32, dim3(256), dim3(256), 0, 0, d_kx64, (float*)p->d_kx, (int)kx_total);

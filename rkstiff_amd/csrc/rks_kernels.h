@@ -54,7 +54,7 @@ struct rks_launch {
 // at least two elements per thread in every transform)
 __host__ __device__ constexpr int rks_threads(int log2n, int nlk) {
   const int N = 1 << log2n;
-  if (nlk == NLK_HANKEL) return N / 4 < 64 ? 64 : (N / 4 > 256 ? 256 : N / 4);
+  if (nlk == NLK_HANKEL) return N < 64 ? 64 : (N > 512 ? 512 : N);
   const int lo = (nlk == NLK_ADVECT) ? (N / 4 < 64 ? N / 4 : 64) : (N / 2 < 64 ? N / 2 : 64);
   const int t = N / 16 > lo ? N / 16 : lo;
   return t > 512 ? 512 : t;
@@ -529,20 +529,27 @@ __device__ __forceinline__ ChunkIdx<CH> own_chunk(int c, const Own<N, M, T, NLK>
   return ix;
 }
 
-// Slot k's mode in the order of the error norm's sums: fft layout, thread t adds the mirror
+// The order of the error norm's sums, mode(k) of slot k: fft layout, thread t adds the mirror
 // pairs q = t + jT (slot 2j) and N - q (slot 2j + 1; N/2 for q = 0), else its own modes.  One
 // order for all kernels of a size: s in its last bits reaches h, in MIXED a changed h rounds
 // the FP32 coefficients anew (~1e-9 of the state), and unresolved runs amplify any change.
+// The Hankel kind's sums run over the lanes of NT threads (t + k NT), whatever T is.
 template <int N, int M, int T, int NLK>
-__device__ __forceinline__ int norm_mode(int k) {
-  const int t = threadIdx.x;
-  if constexpr (M == N && NLK != NLK_HANKEL) {
-    const int q = t + (k >> 1) * T;
-    return (k & 1) == 0 ? q : (q == 0 ? N / 2 : N - q);
-  } else {
-    return t + k * T;
+struct NormOrder {
+  static constexpr int NT = NLK == NLK_HANKEL ? (N / 4 < 64 ? 64 : (N / 4 > 256 ? 256 : N / 4)) : T;
+  static constexpr int SLOTS = (M + NT - 1) / NT;
+  static constexpr bool OWN = !(M == N && (NLK != NLK_HANKEL || NT != T));  // the thread's own modes in order
+  static __device__ __forceinline__ int mode(int k) {
+    const int t = threadIdx.x;
+    if constexpr (M == N && NLK != NLK_HANKEL) {
+      const int q = t + (k >> 1) * T;
+      return (k & 1) == 0 ? q : (q == 0 ? N / 2 : N - q);
+    } else {
+      return t + k * NT;
+    }
   }
-}
+  static __device__ __forceinline__ bool ok(int k, int lim) { return (int)threadIdx.x < NT && mode(k) < lim; }
+};
 
 // coefficient array c of the chunk's modes; M is the array stride (modes)
 template <typename RS, typename RN, int CH>
@@ -836,57 +843,73 @@ __host__ __device__ constexpr int rks_lds_bytes() {
          (int)sizeof(cx<R>);
 }
 
-// Hankel kind: yk = Y (nr x nr, row-major, engine precision), hs = S.  Each thread
-// forms whole rows, summing over the columns in order with FMAs; the stage values
-// (buf) and |f|^2 f (the second LDS vector) are read by every lane at the same
-// index, so LDS serves them as broadcasts.  Arithmetic as the batched transform
-// (rks_hankel.hip): f = (1/S) sum, |f|^2 f, then i gamma (S sum).
+// Hankel kind: yt = Y transposed (nr x nr, engine precision), hs = S.  A thread forms whole
+// rows of both products, summing over the columns in order with FMAs.  Column k of Y is a row
+// of yt, so a wave reads it as one run of memory (row by row of Y, every lane would touch a
+// line of its own), and the vector comes from LDS as broadcasts: the products are bound by
+// the 8 nr^2 bytes of yt per product that each trajectory streams from L2 (80 KB at nr = 100,
+// beyond the L1), with a thread per row so that all of a row's latency is spent once.  1024
+// beams, nr = 100, ETD35 FP64: RKS_HANKEL_FIGURES.
+// Arithmetic as the batched transform (rks_hankel.hip): f = (1/S) sum, |f|^2 f, then
+// i gamma (S sum).
 template <typename R, int LOG2N, int T, int MPT>
-__device__ __forceinline__ void nl_hankel(cx<R> (&v)[MPT], cx<R>* buf, R coef, const R* __restrict__ yk, int nr,
+__device__ __forceinline__ void hankel_rows(cx<R> (&v)[MPT], const cx<R>* x, const R* __restrict__ yt, int nr) {
+#pragma unroll
+  for (int i = 0; i < MPT; ++i) {
+    const int r = (int)threadIdx.x + i * T;
+    const R* col = yt;
+    const int rr = r < nr ? r : 0;
+    R ar = (R)0, ai = (R)0;
+    int k = 0;
+    constexpr int U = 10;
+    for (; k + U <= nr; k += U, col += U * nr) {
+      R y[U];
+#pragma unroll
+      for (int j = 0; j < U; ++j) y[j] = gload_real(col, rr + j * nr);
+#pragma unroll
+      for (int j = 0; j < U; ++j) {
+        const cx<R> q = x[k + j];
+        ar = fma(y[j], q.re, ar);
+        ai = fma(y[j], q.im, ai);
+      }
+    }
+    for (; k < nr; ++k, col += nr) {
+      const R y = gload_real(col, rr);
+      const cx<R> q = x[k];
+      ar = fma(y, q.re, ar);
+      ai = fma(y, q.im, ai);
+    }
+    v[i] = mkc(ar, ai);
+  }
+}
+
+template <typename R, int LOG2N, int T, int MPT>
+__device__ __forceinline__ void nl_hankel(cx<R> (&v)[MPT], cx<R>* buf, R coef, const R* __restrict__ yt, int nr,
                                           double hs) {
+#pragma clang fp contract(off)
   using C = cx<R>;
-  constexpr int N = 1 << LOG2N;
   const int t = threadIdx.x;
-  C* w = buf + rksfft::padded_size(N);
+  C* w = buf + rksfft::padded_size(1 << LOG2N);
   const R ci = (R)(1.0 / hs), cs = (R)hs;
 #pragma unroll
   for (int i = 0; i < MPT; ++i)
     if (t + i * T < nr) buf[t + i * T] = v[i];
   __syncthreads();
-#pragma unroll 1
-  for (int r = t; r < nr; r += T) {
-    const R* __restrict__ y = yk + (size_t)r * nr;
-    R ar = (R)0, ai = (R)0;
-    for (int k = 0; k < nr; ++k) {
-      const R yv = y[k];
-      const C x = buf[k];
-      ar = fma(yv, x.re, ar);
-      ai = fma(yv, x.im, ai);
-    }
-    R vr = ci * ar, vi = ci * ai;
-    const R m2 = vr * vr + vi * vi;
-    vr *= m2;
-    vi *= m2;
-    w[r] = mkc(vr, vi);
-  }
-  __syncthreads();
+  hankel_rows<R, LOG2N, T, MPT>(v, buf, yt, nr);
 #pragma unroll
   for (int i = 0; i < MPT; ++i) {
-    const int r = t + i * T;
-    if (r < nr) {
-      const R* __restrict__ y = yk + (size_t)r * nr;
-      R ar = (R)0, ai = (R)0;
-      for (int k = 0; k < nr; ++k) {
-        const R yv = y[k];
-        const C x = w[k];
-        ar = fma(yv, x.re, ar);
-        ai = fma(yv, x.im, ai);
-      }
-      const R vr = cs * ar, vi = cs * ai;
-      v[i] = mkc(-coef * vi, coef * vr);
-    }
+    const R vr = ci * v[i].re, vi = ci * v[i].im;
+    const R m2 = fma(vi, vi, vr * vr);
+    if (t + i * T < nr) w[t + i * T] = mkc(vr * m2, vi * m2);
   }
   __syncthreads();
+  hankel_rows<R, LOG2N, T, MPT>(v, w, yt, nr);
+#pragma unroll
+  for (int i = 0; i < MPT; ++i) {
+    const R vr = cs * v[i].re, vi = cs * v[i].im;
+    v[i] = mkc(-coef * vi, coef * vr);
+  }
+  // w is next written after the barrier that follows the next fill of buf
 }
 
 // Slots whose imaginary parts of U + iV take the product unrounded.  On a spectrum that
@@ -1417,52 +1440,62 @@ __device__ int run_instance(const rks_launch& P, int idx, cx<R>* buf, const cx<R
       const double cut = ct.adapt_cutoff;
       if constexpr (METHOD) {
 #pragma clang fp contract(off)
-        double a[MPT], e[MPT];
+        using NO = NormOrder<N, M, T, NLK>;
+        constexpr int NS = NO::OWN ? MPT : NO::SLOTS;
+        double a[MPT], e[MPT], an[NS], en[NS];
         final_sum<TT, LAST_SLOT, 0, rks_sum_chunk<R>(), !FUSED>(a, e, cand, nv, u, ow, slot, cbase, (size_t)Mc, h);
         if constexpr (FUSED) {
 #pragma unroll
           for (int k = 0; k < MPT; ++k) mx = nanmax(mx, a[k]);
         }
-        if constexpr (M == N && NLK != NLK_HANKEL) {
-          // into norm_mode's order through the idle buffer, where the proposer finds |u_new|
+        if constexpr (!NO::OWN) {
+          // into NormOrder through the idle buffer, where the proposer finds |u_new|
           double* const db = (double*)buf;
           constexpr bool PAIRS = FUSED || sizeof(R) == sizeof(double);  // both values fit an element
 #pragma unroll
           for (int k = 0; k < MPT; ++k) {
-            if constexpr (PAIRS) buf[ow.m(k)] = mkc((R)a[k], (R)e[k]);
-            else db[ow.m(k)] = a[k];
+            if (!ow.ok(k)) continue;
+            if constexpr (PAIRS) buf[ow.raw(k)] = mkc((R)a[k], (R)e[k]);
+            else db[ow.raw(k)] = a[k];
           }
           __syncthreads();
 #pragma unroll
-          for (int k = 0; k < MPT; ++k) {
-            const int m = norm_mode<N, M, T, NLK>(k);
+          for (int k = 0; k < NS; ++k) {
+            const bool ok = NO::ok(k, ow.lim);
+            const int m = ok ? NO::mode(k) : 0;
             if constexpr (PAIRS) {
-              a[k] = (double)buf[m].re;
-              e[k] = (double)buf[m].im;
+              an[k] = ok ? (double)buf[m].re : 0.0;
+              en[k] = ok ? (double)buf[m].im : 0.0;
             } else {
-              a[k] = db[m];
+              an[k] = ok ? db[m] : 0.0;
             }
           }
           __syncthreads();
           if constexpr (!PAIRS) {
 #pragma unroll
-            for (int k = 0; k < MPT; ++k) db[ow.m(k)] = e[k];
+            for (int k = 0; k < MPT; ++k)
+              if (ow.ok(k)) db[ow.raw(k)] = e[k];
             __syncthreads();
 #pragma unroll
-            for (int k = 0; k < MPT; ++k) e[k] = db[norm_mode<N, M, T, NLK>(k)];
+            for (int k = 0; k < NS; ++k) en[k] = NO::ok(k, ow.lim) ? db[NO::mode(k)] : 0.0;
             __syncthreads();
           }
-        } else if constexpr (LEARN && FUSED) {
+        } else {
 #pragma unroll
-          for (int k = 0; k < MPT; ++k)
-            if (ow.ok(k)) buf[ow.m(k)].re = (R)a[k];
+          for (int k = 0; k < NS; ++k) {
+            an[k] = a[k];
+            en[k] = e[k];
+            if constexpr (LEARN && FUSED) {
+              if (ow.ok(k)) buf[ow.m(k)].re = (R)a[k];
+            }
+          }
         }
         mx = wg_max<T>(mx, red);
         const double lim = FUSED ? cut * mx : (cut < 0.0 ? -1.0 : cut * cut * mx);
 #pragma unroll
-        for (int k = 0; k < MPT; ++k) {
-          const bool on = a[k] > lim && a[k] <= __DBL_MAX__;
-          const double x = on ? a[k] : 0.0, y = on ? e[k] : 0.0;
+        for (int k = 0; k < NS; ++k) {
+          const bool on = an[k] > lim && an[k] <= __DBL_MAX__;
+          const double x = on ? an[k] : 0.0, y = on ? en[k] : 0.0;
           su = FUSED ? fma(x, x, su) : su + x;
           se = (FUSED && sizeof(R) < sizeof(double)) ? fma(y, y, se) : se + y;
         }
@@ -1471,12 +1504,16 @@ __device__ int run_instance(const rks_launch& P, int idx, cx<R>* buf, const cx<R
         mx = wg_max<T>(mx, red);
         const double lim = fused ? cut * mx : (cut < 0.0 ? -1.0 : cut * cut * mx);
         __syncthreads();  // every thread's last NL values, candidate and buffer values
+        using NO = NormOrder<N, M, T, NLK>;
+        constexpr int NCH = (NO::SLOTS + CH - 1) / CH;
 #pragma unroll 1
-        for (int c = 0; c < Chunk<MPT>::NCH; ++c) {
+        for (int c = 0; c < NCH; ++c) {
           ChunkIdx<CH> ix = own_chunk<N, M, T, NLK, CH>(c, ow);
 #pragma unroll
-          for (int i = 0; i < CH; ++i)
-            if (M == N && NLK != NLK_HANKEL) ix.m[i] = norm_mode<N, M, T, NLK>(c * CH + i);
+          for (int i = 0; i < CH; ++i) {
+            ix.ok[i] = NO::ok(c * CH + i, ow.lim);
+            ix.m[i] = ix.ok[i] ? NO::mode(c * CH + i) : 0;
+          }
           C ev[CH];
           if (!fused) error_chunk<R, RN, CH>(tb, slot, cbase, (size_t)Mc, ix, h, ev);
 #pragma unroll

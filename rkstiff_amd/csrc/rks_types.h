@@ -150,7 +150,7 @@ typedef struct rks_inst {
   int L_complex;       // L stored as complex128 (1) or float64 (0)
   int log_cap;         // attempt-log capacity (entries of 2 doubles)
   const double* L;     // FP64 lin_op
-  const void* kx;      // wavenumbers (advect nl) or the Hankel matrix (Hankel nl), engine precision
+  const void* kx;      // wavenumbers (advect nl) or the transposed Hankel matrix (Hankel nl), engine precision
   double nl_coef;
   double nl_scale;     // S of the Hankel transform (Hankel nl)
   void* ws;            // workspace (engine precision complex)
