@@ -141,7 +141,29 @@ __device__ __forceinline__ void rks2_states(const rks2_launch& P, const rks_inst
 // load of each NL value; |u_new| and |err|^2 (FP32: |err|) per mode go to T,
 // idle at that point, for k2_norm_fused.  A separate instantiation, so the
 // other stages keep their register allocation (no spills at 4 waves per SIMD).
-template <typename R, typename RN, int LOG2, bool FUSE>
+// METH: the stage sums of one method as literals (rks_method.h), else the tableau.
+// A pass is bound by HBM once its loads are all in flight; the interpreted fused pass was not
+// (64 x 512^2 ETD35 FP32: 370 us for 0.8 GB).  The whole batch went 75.2 -> 61.2 ms with the
+// literal passes and coefficients, 8 x 128^2 FP64 10.3 -> 6.6 ms (there the coefficients were
+// 71 of 240 us an attempt: one thread summed a small mode's contour means).
+
+// The chunk's modes for the literal stage sums: mirror row pairs (slot 2j row q, slot
+// 2j + 1 row n - q), coefficients of the mirror row where L is mirror-symmetric.
+template <int N, int XS, int CH>
+struct OwnRows {
+  int row[CH];
+  int col, sym;
+  bool valid;
+  __device__ __forceinline__ bool ok(int) const { return valid; }
+  __device__ __forceinline__ int m(int k) const { return valid ? row[k] * XS + col : 0; }
+  __device__ __forceinline__ int c(int k) const {
+    const int r = (sym && row[k] > N / 2) ? N - row[k] : row[k];
+    return valid ? r * XS + col : 0;
+  }
+  __device__ __forceinline__ OwnRows fresh() const { return *this; }
+};
+
+template <typename R, typename RN, int LOG2, bool FUSE, int METH>
 __global__ __launch_bounds__((Geo2<R, LOG2>::CT), 4) void k2_col(rks2_launch P, int fwd_slot, int fwd_need_nl1,
                                                             int arg, int prelude) {
   using G = Geo2<R, LOG2>;
@@ -161,14 +183,16 @@ __global__ __launch_bounds__((Geo2<R, LOG2>::CT), 4) void k2_col(rks2_launch P, 
   const rks_tableau& tb = *P.tab;
   rks_inst* in = P.inst + inst;
   const rks_io& io = P.io[inst];
-  char* ws = (char*)in->ws;
-  const double h = in->h;
-  const unsigned smap = rks2_smap(in);
+  char* ws = uni((char*)in->ws);
+  const double h = uni(in->h);
+  const unsigned smap = (unsigned)uni((int)rks2_smap(in));
   CN* const slot_base = (CN*)ws;
   auto slot = [&](int s) -> CN* { return slot_base + (size_t)((smap >> (4 * s)) & 15u) * MI; };
   const C* u;
   C* cand;
   rks2_states<R>(P, in, io, &u, &cand);
+  u = uni(u);
+  cand = uni(cand);
   const int ustride = P.mode == RKS_MODE_NL ? NXH : XS;  // the caller's u in the nonlinear-term mode
   C* Tb = (C*)(ws + P.off_T);
   const char* cbase = ws + P.off_coef;
@@ -212,6 +236,8 @@ __global__ __launch_bounds__((Geo2<R, LOG2>::CT), 4) void k2_col(rks2_launch P, 
   const int sym = in->coef_sym;
   const size_t Mc = sym ? G::MSYM : MI;
   const bool fused = FUSE && last;
+  constexpr bool METHOD = METH != RKS_METH_ANY;
+  using TT = MethodTab<METHOD ? METH : 0, (int)sizeof(C), (int)sizeof(CN), true>;
   double mx = 0.0;
   // stage combination over mirror row pairs: slot 2j row q = r0 + (ch CH/2 + j) RS,
   // slot 2j + 1 row n - q (n/2 for q = 0), so a mirror-symmetric L shares coefficients
@@ -233,7 +259,36 @@ __global__ __launch_bounds__((Geo2<R, LOG2>::CT), 4) void k2_col(rks2_launch P, 
       ix.ok[2 * j] = ix.ok[2 * j + 1] = valid;
     }
     C acc[CH];
-    if (arg < 0) {
+    if constexpr (METHOD) {
+      OwnRows<N, XS, CH> ow;
+#pragma unroll
+      for (int i = 0; i < CH; ++i) ow.row[i] = row[i];
+      ow.col = col;
+      ow.sym = sym;
+      ow.valid = valid;
+      CN none[CH];  // no NL values kept in registers between kernels
+#pragma unroll
+      for (int i = 0; i < CH; ++i) none[i] = mkc((RN)0, (RN)0);
+      if (fused) {
+        if constexpr (FUSE) {
+          double a[CH], e[CH];
+          final_sum<TT, -1, 0, CH, false>(a, e, cand, none, u, ow, slot, cbase, Mc, h);
+#pragma unroll
+          for (int i = 0; i < CH; ++i) {
+            if (!valid) continue;
+            gstore(Tb, row[i] * G::TXS + col, mkc((R)a[i], (R)e[i]));
+            mx = nanmax(mx, a[i]);
+          }
+        }
+        continue;
+      }
+      if (arg < 0) {
+#pragma unroll
+        for (int i = 0; i < CH; ++i) acc[i] = valid ? gload(u, row[i] * ustride + col) : zero;
+      } else {
+        stage_switch<TT, 0, false>(arg, acc, none, u, ow, slot, cbase, Mc, h);
+      }
+    } else if (arg < 0) {
 #pragma unroll
       for (int i = 0; i < CH; ++i) acc[i] = valid ? u[row[i] * ustride + col] : zero;
     } else if (fused) {
@@ -345,21 +400,61 @@ __global__ __launch_bounds__((Geo2<R, LOG2>::RT)) void k2_row(rks2_launch P, int
 // ---------------------------------------------------------------------------
 // coefficients (FP64 arithmetic) of trajectories whose h changed
 // ---------------------------------------------------------------------------
-template <typename R, typename RN, int LOG2>
+template <typename R, typename RN, int LOG2, int METH>
 __global__ __launch_bounds__(256) void k2_coef(rks2_launch P) {
   using G = Geo2<R, LOG2>;
   const int inst = blockIdx.y;
   const rks2_state st = P.st[inst];
   if (!st.active || !st.need_coef) return;
   const rks_inst* in = P.inst + inst;
-  char* cbase = (char*)in->ws + P.off_coef;
+  char* cbase = uni((char*)in->ws) + P.off_coef;
   // mirror-symmetric L: rows 0..n/2 only (stride MSYM); lin_op in the caller's
   // layout, coefficients in the internal one
   const int Mg = in->coef_sym ? G::MGEN_SYM : G::M;
   const int Mc = in->coef_sym ? G::MSYM : G::MI;
-  for (int m = blockIdx.x * 256 + threadIdx.x; m < Mg; m += gridDim.x * 256) {
-    const int r = m / G::NXH, c = m - r * G::NXH;
-    coef_mode_at<R, RN>(*P.tab, *P.ctl, in->L, in->L_complex, m, r * G::XS + c, Mc, in->h, cbase);
+  if constexpr (METH == RKS_METH_ANY) {
+    for (int m = blockIdx.x * 256 + threadIdx.x; m < Mg; m += gridDim.x * 256) {
+      const int r = m / G::NXH, c = m - r * G::NXH;
+      coef_mode_at<R, RN>(*P.tab, *P.ctl, in->L, in->L_complex, m, r * G::XS + c, Mc, in->h, cbase);
+    }
+  } else {
+    // literal recipes; a workgroup's few small modes (|z| < modecutoff), whose contour
+    // means are 32 psi evaluations each, wait in a list and are spread over its lanes
+    using TT = MethodTab<METH, (int)sizeof(cx<R>), (int)sizeof(cx<RN>), true>;
+    __shared__ int list[256];
+    __shared__ int count;
+    rks_cctl& ct = *rks_uniform_const<rks_cctl>(P.ctl);
+    const double* L = uni(in->L);
+    const double h = uni(in->h);
+    for (int m0 = blockIdx.x * 256; m0 < Mg; m0 += gridDim.x * 256) {
+      const int m = m0 + (int)threadIdx.x;
+      if constexpr (TT::tab.uses_contour != 0) {
+        if (threadIdx.x == 0) count = 0;
+        __syncthreads();
+      }
+      if (m < Mg) {
+        const int r = m / G::NXH, c = m - r * G::NXH;
+        const z64 z = mode_z(L, 0, m, h);
+        if (TT::tab.uses_contour && hypot(z.re, z.im) < ct.modecutoff)
+          list[atomicAdd(&count, 1)] = m;
+        else
+          method_fracs<TT, 0, R, RN>(
+              [&](int fnum, int fden, int fmask, z64(&v)[4]) {
+                frac_direct(fnum, fden, fmask, z, h, TT::tab.uses_contour, v);
+              },
+              h, r * G::XS + c, (size_t)Mc, cbase);
+      }
+      if constexpr (TT::tab.uses_contour != 0) {
+        __syncthreads();
+        const int nsmall = count;
+        for (int idx = threadIdx.x / 32; idx < nsmall; idx += 256 / 32) {
+          const int ms = list[idx], r = ms / G::NXH, c = ms - r * G::NXH;
+          method_small<TT, 0, R, RN, 32, true>(ct, mode_z(L, 0, ms, h), threadIdx.x % 32, h, r * G::XS + c, (size_t)Mc,
+                                               cbase);
+        }
+        __syncthreads();
+      }
+    }
   }
 }
 

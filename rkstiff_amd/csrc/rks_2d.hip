@@ -7,7 +7,7 @@
 #include "rks_2d_host.h"
 
 struct rks2_ctx {
-  int prec = 0, log2n = 0, ninst = 0, M = 0;
+  int prec = 0, variant = 0, log2n = 0, ninst = 0, M = 0;
   rks2_launch L;
   rks2_state* d_st = nullptr;
   double* d_pmax = nullptr;
@@ -20,14 +20,15 @@ struct rks2_ctx {
   bool use_graph = true;
 };
 
-template <typename R, typename RN, int LOG2>
+// METH: RKS_METH_ANY, or the method whose stage sums and coefficients are compiled in
+template <typename R, typename RN, int LOG2, int METH>
 struct Eng2 {
   using G = Geo2<R, LOG2>;
   static hipError_t setup() {
-    hipError_t e = hipFuncSetAttribute((const void*)k2_col<R, RN, LOG2, false>,
+    hipError_t e = hipFuncSetAttribute((const void*)k2_col<R, RN, LOG2, false, METH>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, G::COL_LDS);
     if (e == hipSuccess)
-      e = hipFuncSetAttribute((const void*)k2_col<R, RN, LOG2, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
+      e = hipFuncSetAttribute((const void*)k2_col<R, RN, LOG2, true, METH>, hipFuncAttributeMaxDynamicSharedMemorySize,
                               G::COL_LDS);
     if (e != hipSuccess) return e;
     return hipFuncSetAttribute((const void*)k2_row<R, LOG2>, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -37,10 +38,10 @@ struct Eng2 {
   static int nnb() { return G::NNB; }
   static void col(const rks2_launch& L, hipStream_t s, int fwd, int cond, int arg, int prelude, bool fuse = false) {
     if (fuse)
-      hipLaunchKernelGGL((k2_col<R, RN, LOG2, true>), dim3(G::NCG, L.ninst), dim3(G::CT), G::COL_LDS, s, L, fwd,
+      hipLaunchKernelGGL((k2_col<R, RN, LOG2, true, METH>), dim3(G::NCG, L.ninst), dim3(G::CT), G::COL_LDS, s, L, fwd,
                          cond, arg, prelude);
     else
-      hipLaunchKernelGGL((k2_col<R, RN, LOG2, false>), dim3(G::NCG, L.ninst), dim3(G::CT), G::COL_LDS, s, L, fwd,
+      hipLaunchKernelGGL((k2_col<R, RN, LOG2, false, METH>), dim3(G::NCG, L.ninst), dim3(G::CT), G::COL_LDS, s, L, fwd,
                          cond, arg, prelude);
   }
   static void row(const rks2_launch& L, hipStream_t s, int prelude) {
@@ -59,7 +60,9 @@ struct Eng2 {
   // one attempt of every running trajectory
   static void attempt(const rks2_launch& L, const rks_tableau& tb, hipStream_t s) {
     hipLaunchKernelGGL(k2_begin, dim3(1), dim3(256), 0, s, L);
-    hipLaunchKernelGGL((k2_coef<R, RN, LOG2>), dim3((G::M + 256 * 8 - 1) / (256 * 8), L.ninst), dim3(256), 0, s, L);
+    // a mode per thread until there are 8 workgroups for every CU, then several
+    const int one = (G::M + 255) / 256, cap = 2048 / L.ninst > one / 8 ? 2048 / L.ninst : one / 8 + 1;
+    hipLaunchKernelGGL((k2_coef<R, RN, LOG2, METH>), dim3(one < cap ? one : cap, L.ninst), dim3(256), 0, s, L);
     // NL1 = nl(u) where needed (start; after an accept for RECOMPUTE methods)
     col(L, s, -1, 0, -1, 1);
     row(L, s, 1);
@@ -91,42 +94,50 @@ struct Eng2 {
   }
 };
 
-template <typename R, typename RN, typename F>
+template <typename R, typename RN, int METH, typename F>
 static bool with_size(int log2n, F&& f) {
   switch (log2n) {
-    case 5: f(Eng2<R, RN, 5>{}); return true;
-    case 6: f(Eng2<R, RN, 6>{}); return true;
-    case 7: f(Eng2<R, RN, 7>{}); return true;
-    case 8: f(Eng2<R, RN, 8>{}); return true;
-    case 9: f(Eng2<R, RN, 9>{}); return true;
+    case 5: f(Eng2<R, RN, 5, METH>{}); return true;
+    case 6: f(Eng2<R, RN, 6, METH>{}); return true;
+    case 7: f(Eng2<R, RN, 7, METH>{}); return true;
+    case 8: f(Eng2<R, RN, 8, METH>{}); return true;
+    case 9: f(Eng2<R, RN, 9, METH>{}); return true;
     default: return false;
   }
 }
 
+template <typename R, typename RN, typename F>
+static bool with_method(int variant, int log2n, F&& f) {
+  if (variant == RKS_M_ETD35) return with_size<R, RN, RKS_M_ETD35>(log2n, f);
+  if (variant == RKS_M_IF34) return with_size<R, RN, RKS_M_IF34>(log2n, f);
+  return with_size<R, RN, RKS_METH_ANY>(log2n, f);
+}
+
 template <typename F>
-static bool with_engine(int prec, int log2n, F&& f) {
-  if (prec == RKS_F64) return with_size<double, double>(log2n, f);
-  if (prec == RKS_F32) return with_size<float, float>(log2n, f);
-  if (prec == RKS_MIXED) return with_size<double, float>(log2n, f);
+static bool with_engine(int prec, int variant, int log2n, F&& f) {
+  if (prec == RKS_F64) return with_method<double, double>(variant, log2n, f);
+  if (prec == RKS_F32) return with_method<float, float>(variant, log2n, f);
+  if (prec == RKS_MIXED) return with_method<double, float>(variant, log2n, f);
   return false;
 }
 
 int rks2_supported(int prec, int log2n) {
-  return with_engine(prec, log2n, [](auto) {}) ? 1 : 0;
+  return (prec == RKS_F64 || prec == RKS_F32 || prec == RKS_MIXED) && log2n >= 5 && log2n <= 9 ? 1 : 0;
 }
 
-int rks2_create(rks2_ctx** out, int prec, int log2n, int ninst, const rks_tableau* d_tab, const rks_ctrl* d_ctl,
+int rks2_create(rks2_ctx** out, int prec, int variant, int log2n, int ninst, const rks_tableau* d_tab, const rks_ctrl* d_ctl,
                 rks_inst* d_inst, const rks_io* d_io, const void* d_tw, size_t off_cand0, size_t off_cand1,
                 size_t off_coef, size_t off_T) {
   *out = nullptr;
   rks2_ctx* c = new rks2_ctx();
   c->prec = prec;
+  c->variant = variant;
   c->log2n = log2n;
   c->ninst = ninst;
   c->M = rks2_modes(log2n);
   int ncg = 0, nnb = 0;
   hipError_t e = hipSuccess;
-  if (!with_engine(prec, log2n, [&](auto eng) {
+  if (!with_engine(prec, variant, log2n, [&](auto eng) {
         using E = decltype(eng);
         ncg = E::ncg();
         nnb = E::nnb();
@@ -184,7 +195,7 @@ static hipGraphExec_t attempt_graph(rks2_ctx* c, const rks_tableau& tb, int mode
     c->use_graph = false;
     return nullptr;
   }
-  with_engine(c->prec, c->log2n, [&](auto eng) { decltype(eng)::attempt(L, tb, c->cap); });
+  with_engine(c->prec, c->variant, c->log2n, [&](auto eng) { decltype(eng)::attempt(L, tb, c->cap); });
   hipGraph_t g = nullptr;
   if (hipStreamEndCapture(c->cap, &g) != hipSuccess || !g) {
     c->use_graph = false;
@@ -206,12 +217,12 @@ hipError_t rks2_run(rks2_ctx* c, const rks_tableau& tb, int mode, hipStream_t s)
   L.mode = mode;
   hipLaunchKernelGGL(k2_init, dim3(1), dim3(256), 0, s, L);
   if (mode == RKS_MODE_NL) {
-    with_engine(c->prec, c->log2n, [&](auto eng) { decltype(eng)::nl(L, s); });
+    with_engine(c->prec, c->variant, c->log2n, [&](auto eng) { decltype(eng)::nl(L, s); });
     return hipGetLastError();
   }
   // the caller's state into the internal layout (a resumed evolve keeps its own)
-  with_engine(c->prec, c->log2n, [&](auto eng) { decltype(eng)::in(L, s); });
-  if (mode == RKS_MODE_EVOLVE) with_engine(c->prec, c->log2n, [&](auto eng) { decltype(eng)::snap(L, s); });
+  with_engine(c->prec, c->variant, c->log2n, [&](auto eng) { decltype(eng)::in(L, s); });
+  if (mode == RKS_MODE_EVOLVE) with_engine(c->prec, c->variant, c->log2n, [&](auto eng) { decltype(eng)::snap(L, s); });
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   hipGraphExec_t g = attempt_graph(c, tb, mode);
@@ -222,7 +233,7 @@ hipError_t rks2_run(rks2_ctx* c, const rks_tableau& tb, int mode, hipStream_t s)
   for (long long it = 0;; it += K) {
     for (int k = 0; k < K; ++k) {
       if (g) e = hipGraphLaunch(g, s);
-      else with_engine(c->prec, c->log2n, [&](auto eng) { decltype(eng)::attempt(L, tb, s); });
+      else with_engine(c->prec, c->variant, c->log2n, [&](auto eng) { decltype(eng)::attempt(L, tb, s); });
       if (e == hipSuccess) e = hipGetLastError();
       if (e != hipSuccess) return e;
     }
@@ -232,7 +243,7 @@ hipError_t rks2_run(rks2_ctx* c, const rks_tableau& tb, int mode, hipStream_t s)
     if (*c->h_active == 0) break;
     if (it > cap) return hipErrorUnknown;
   }
-  with_engine(c->prec, c->log2n, [&](auto eng) { decltype(eng)::out(L, s); });
+  with_engine(c->prec, c->variant, c->log2n, [&](auto eng) { decltype(eng)::out(L, s); });
   return hipGetLastError();
 }
 

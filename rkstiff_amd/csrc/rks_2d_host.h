@@ -33,7 +33,8 @@ inline int rks2_imodes(int log2n) { return (1 << log2n) * rks2_istride(1 << log2
 //   complex values) at off_T;
 // NL slots, candidates and coefficient arrays have rks2_imodes elements each
 // (rows of rks2_istride).
-int rks2_create(rks2_ctx** out, int prec, int log2n, int ninst, const rks_tableau* d_tab, const rks_ctrl* d_ctl,
+// variant: the method whose kernels are compiled for it (real lin_op), or RKS_METH_ANY.
+int rks2_create(rks2_ctx** out, int prec, int variant, int log2n, int ninst, const rks_tableau* d_tab, const rks_ctrl* d_ctl,
                 rks_inst* d_inst, const rks_io* d_io, const void* d_tw, size_t off_cand0, size_t off_cand1,
                 size_t off_coef, size_t off_T);
 // One launch set: mode RKS_MODE_EVOLVE / RKS_MODE_STEP (attempts until every

@@ -157,10 +157,11 @@ typedef rks_kernel_entry KernelEntry;
 // Which stepping kernel runs a plan: the one compiled for its method where that exists, else
 // the one that reads the tableau.  ETD35 and IF34 are the methods of every workload; their
 // kernels are compiled for the coefficient storage that goes with the nonlinearity (real
-// lin_op with the advective term, complex with the cubic ones), so a complex lin_op with the
-// advective term (KdV) or a real one with a cubic term takes the general kernel.
+// lin_op with the advective and the rfft2 terms, complex with the cubic ones), so a complex
+// lin_op with the advective term (KdV) or a real one with a cubic term takes the general kernel.
 int method_variant(int method, int nlk, int coef_real) {
-  if ((nlk == RKS_NL_ADVECT_RFFT) != (coef_real != 0)) return RKS_METH_ANY;
+  const bool real = nlk == RKS_NL_ADVECT_RFFT || nlk == RKS_NL_AC2D_RFFT2;
+  if (real != (coef_real != 0)) return RKS_METH_ANY;
   if (method == RKS_M_ETD35) return method;
   if (method == RKS_M_IF34 && nlk != RKS_NL_HANKEL_CUBIC) return method;
   return RKS_METH_ANY;
@@ -515,7 +516,7 @@ int rks_plan_create(int method, int nl_kind, int precision, const rks_config* cf
     const size_t off_c1 = off_c0 + rks_align256(mw * p->esize);
     const size_t off_cf = off_c1 + rks_align256(mw * p->esize);
     const size_t off_T = off_cf + rks_align256(p->coef_bytes_per_mode * mw);
-    if (rks2_create(&p->c2, precision, l, ninst, p->d_tab, p->d_ctl, p->d_inst, p->d_io, p->d_tw[l], off_c0, off_c1,
+    if (rks2_create(&p->c2, precision, p->variant, l, ninst, p->d_tab, p->d_ctl, p->d_inst, p->d_io, p->d_tw[l], off_c0, off_c1,
                     off_cf, off_T)) {
       rks_plan_destroy(p);
       return fail(RKS_ERR_HIP, "2-D engine set-up failed");

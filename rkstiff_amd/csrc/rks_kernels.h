@@ -365,7 +365,9 @@ __device__ __forceinline__ void method_fracs(Get get, double h, int m, size_t M,
   }
 }
 
-template <typename TT, int F, typename RS, typename RN, int GS, typename CT>
+// One small mode's contour means by GS lanes, one node each: summed by a butterfly, or
+// (ORDERED) node by node in the order in which one thread sums them.
+template <typename TT, int F, typename RS, typename RN, int GS, bool ORDERED, typename CT>
 __device__ __forceinline__ void method_small(CT& ct, z64 z, int lane, double h, int m, size_t M,
                                              char* __restrict__ cbase) {
   if constexpr (F < TT::tab.nfrac) {
@@ -376,16 +378,33 @@ __device__ __forceinline__ void method_small(CT& ct, z64 z, int lane, double h, 
     if constexpr ((fmask & 14) != 0) {
       z64 acc[4];
       acc[1] = acc[2] = acc[3] = mkc(0.0, 0.0);
-      for (int j = lane; j < ct.contour_points; j += GS) {
-        const z64 nd = contour_node(ct.contour_points, ct.contour_radius, j);
-        frac_contour_add(fnum, fden, fmask, mkc(z.re + nd.re, z.im + nd.im), acc);
-      }
+      if constexpr (ORDERED) {
+        const int np = ct.contour_points;
+        for (int j0 = 0; j0 < np; j0 += GS) {
+          z64 p[4];
+          p[1] = p[2] = p[3] = mkc(0.0, 0.0);
+          const z64 nd = contour_node(np, ct.contour_radius, j0 + lane < np ? j0 + lane : 0);
+          frac_contour_add(fnum, fden, fmask, mkc(z.re + nd.re, z.im + nd.im), p);
+          for (int j = 0; j < GS && j0 + j < np; ++j) {
 #pragma unroll
-      for (int o = GS / 2; o >= 1; o >>= 1) {
+            for (int r = 1; r <= 3; ++r) {
+              acc[r].re += __shfl(p[r].re, j, GS);
+              acc[r].im += __shfl(p[r].im, j, GS);
+            }
+          }
+        }
+      } else {
+        for (int j = lane; j < ct.contour_points; j += GS) {
+          const z64 nd = contour_node(ct.contour_points, ct.contour_radius, j);
+          frac_contour_add(fnum, fden, fmask, mkc(z.re + nd.re, z.im + nd.im), acc);
+        }
 #pragma unroll
-        for (int r = 1; r <= 3; ++r) {
-          acc[r].re += __shfl_xor(acc[r].re, o, 64);
-          acc[r].im += __shfl_xor(acc[r].im, o, 64);
+        for (int o = GS / 2; o >= 1; o >>= 1) {
+#pragma unroll
+          for (int r = 1; r <= 3; ++r) {
+            acc[r].re += __shfl_xor(acc[r].re, o, 64);
+            acc[r].im += __shfl_xor(acc[r].im, o, 64);
+          }
         }
       }
 #pragma unroll
@@ -395,7 +414,7 @@ __device__ __forceinline__ void method_small(CT& ct, z64 z, int lane, double h, 
       v[0] = np_exp(frac_arg(z, fnum, fden, 1));
       coef_recipes<TT, F, RS, RN>(v, h, m, M, cbase, std::make_integer_sequence<int, TT::tab.ncoef>{});
     }
-    method_small<TT, F + 1, RS, RN, GS>(ct, z, lane, h, m, M, cbase);
+    method_small<TT, F + 1, RS, RN, GS, ORDERED>(ct, z, lane, h, m, M, cbase);
   }
 }
 
@@ -434,7 +453,7 @@ __device__ __attribute__((noinline)) void coef_update_method(const rks_ctrl& ct_
     const int g = t / GS, lane = t % GS;
     for (int idx = g; idx < nsmall; idx += T / GS) {
       const int m = list[idx];
-      method_small<TT, 0, RS, RN, GS>(ct, mode_z(L, LC, m, h), lane, h, m, (size_t)M, cbase);
+      method_small<TT, 0, RS, RN, GS, false>(ct, mode_z(L, LC, m, h), lane, h, m, (size_t)M, cbase);
     }
   }
   __syncthreads();
@@ -849,7 +868,7 @@ __host__ __device__ constexpr int rks_lds_bytes() {
 // line of its own), and the vector comes from LDS as broadcasts: the products are bound by
 // the 8 nr^2 bytes of yt per product that each trajectory streams from L2 (80 KB at nr = 100,
 // beyond the L1), with a thread per row so that all of a row's latency is spent once.  1024
-// beams, nr = 100, ETD35 FP64: RKS_HANKEL_FIGURES.
+// beams, nr = 100, ETD35 FP64, one evolve: 21.2 ms row by row with n/4 threads, 8.6 ms.
 // Arithmetic as the batched transform (rks_hankel.hip): f = (1/S) sum, |f|^2 f, then
 // i gamma (S sum).
 template <typename R, int LOG2N, int T, int MPT>
@@ -1139,25 +1158,6 @@ __device__ __forceinline__ double learned_after_accept(const rks_launch& P, cons
 // ---------------------------------------------------------------------------
 // one instance: evolve / step / nl
 // ---------------------------------------------------------------------------
-// Modes per chunk of the literal stage sums: what a chunk loads is in flight in registers
-// together (up to 12 values per mode), beside the stage value and the last NL value.
-template <typename R>
-__host__ __device__ constexpr int rks_sum_chunk() {
-  return sizeof(R) == 4 ? 8 : 4;
-}
-
-// Argument of stage s for a method known at compile time.
-template <typename TT, int S, typename RS, typename RN, int MPT, typename OW, typename SlotF>
-__device__ __forceinline__ void stage_switch(int s, cx<RS> (&acc)[MPT], const cx<RN> (&nv)[MPT], const cx<RS>* u,
-                                             const OW& ow, SlotF slotp, const char* cbase, size_t Mc, double h) {
-  if constexpr (S < TT::tab.nstage && TT::tab.st[S < TT::tab.nstage ? S : 0].has_nl) {
-    // the evaluation just before stage S > 0 is that of stage S - 1
-    constexpr int NEW = S > 0 ? TT::tab.st[S > 0 ? S - 1 : 0].nl_slot : -1;
-    if (s == S) stage_sum<TT, S, NEW, 0, rks_sum_chunk<RS>()>(acc, nv, u, ow, slotp, cbase, Mc, h);
-    else stage_switch<TT, S + 1>(s, acc, nv, u, ow, slotp, cbase, Mc, h);
-  }
-}
-
 // Returns nonzero (proposer variant only) when the evolve stopped after an
 // accepted step for the proposer: the state is in the instance record, and the
 // caller runs learned_between_steps and calls again with reenter set.
@@ -1354,7 +1354,7 @@ __device__ int run_instance(const rks_launch& P, int idx, cx<R>* buf, const cx<R
           load_modes(v, u);
         } else if constexpr (METHOD) {
           if (FUSED && last) break;
-          stage_switch<TT, 0>(s, v, nv, u, ow, slot, cbase, (size_t)Mc, h);
+          stage_switch<TT, 0, true>(s, v, nv, u, ow, slot, cbase, (size_t)Mc, h);
           if (!FUSED && last) {
 #pragma unroll
             for (int k = 0; k < MPT; ++k) {
