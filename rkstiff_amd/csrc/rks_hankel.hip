@@ -5,10 +5,8 @@
 // (transforms.py:172-240); its radial NLS demo (demos/nls.ipynb cell 8)
 // evaluates 1j gamma ht(|f|^2 f), f = iht(g), at every stage.
 //
-// Here one launch multiplies Y by a batch of vectors: out[b] = c Y in[b].
-// Tiles of 64 rows x 16 vectors with 32-wide K chunks staged in LDS, FP64
-// FMAs on the vector units (on MI355X the FP64 matrix-core rate equals the
-// FP64 vector rate, so MFMA would not add throughput here).  The epilogue
+// Here one launch multiplies Y by a batch of vectors: out[b] = c Y in[b], on
+// the FP64 matrix cores (hankel_gemm).  The epilogue
 // scales, or forms |f|^2 f (after the inverse), or multiplies by i gamma (after
 // the forward), so the radial NLS term is two launches.
 #include <hip/hip_runtime.h>
@@ -26,9 +24,9 @@ static __device__ __align__(256) double scratch[kScratchDoubles];
 
 namespace {
 
-constexpr int HB_M = 64;   // rows per tile
-constexpr int HB_B = 16;   // vectors per tile
 constexpr int HB_K = 32;   // K chunk
+constexpr int HB_B = 16;   // column pairs per tile: 16 complex or 32 real vectors
+constexpr int HB_CU = 256; // compute units
 
 enum { EPI_SCALE = 0, EPI_CUBIC = 1, EPI_TIMES_I = 2 };
 
@@ -37,77 +35,131 @@ int hfail(int code, const std::string& msg) {
   return code;
 }
 
+typedef double d4 __attribute__((ext_vector_type(4)));
+typedef double d2 __attribute__((ext_vector_type(2)));
+typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));  // two doubles at any double's address
+
 // out[b][i] = epi(c * sum_j Y[i][j] in[b][j]); complex vectors (CPLX) are
-// interleaved (re, im), real vectors are plain doubles.
-template <bool CPLX, int EPI>
+// interleaved (re, im), real vectors are plain doubles.  A column pair is one
+// complex vector's two parts, or real vectors b and b + 16 of a tile.
+//
+// V_MFMA_F64_16X16X4: lane l holds A[l % 16][l / 16], B[l / 16][l % 16] and
+// D[4 r + l / 16][l % 16], r < 4.  The vectors are A's rows, so a lane's results are one
+// row i of 4 vectors and 16 lanes store 16 consecutive i.  The four k of an instruction
+// need not be neighbours: lane group l / 16 takes a run of k of its own, read from LDS in
+// 16-byte pieces (row strides odd in those: no bank conflicts).  The matrix rate is the
+// vector units' FP64 rate, but an instruction of 2048 operations reads two LDS values per
+// lane where 32 FMAs of a 4 x 2 register tile read 24; those reads bounded the vector form.
+// The next chunk's global loads are in flight during a chunk's products, one barrier each.
+// nr = 251, 1024 complex vectors: 43.5 us by FMAs on a 4 x 2 register tile, now 10.4 (the
+// products alone take 3.3 us at 78 TFLOP/s).  ROWS 64: a wave has 16 rows of its own.  ROWS 16: the four waves share one tile and split
+// each chunk's k, so four times the workgroups; taken while 64-row tiles would leave CUs idle.
+template <bool CPLX, int EPI, int ROWS>
 __global__ __launch_bounds__(256) void hankel_gemm(const double* __restrict__ Y, int nr,
                                                    const double* __restrict__ in, double* __restrict__ out,
                                                    int batch, double c, double gamma) {
-  __shared__ double Ys[HB_M][HB_K + 1];
-  __shared__ double Xr[HB_K][HB_B];
-  __shared__ double Xi[HB_K][HB_B];
-  const int t = threadIdx.x;
-  const int tb = t % HB_B, ti = t / HB_B;  // 16 x 16 threads: vector, row group
-  const int i0 = blockIdx.x * HB_M, b0 = blockIdx.y * HB_B;
-  double ar[4] = {0.0, 0.0, 0.0, 0.0}, ai[4] = {0.0, 0.0, 0.0, 0.0};
-  for (int j0 = 0; j0 < nr; j0 += HB_K) {
+  constexpr bool SPLIT = ROWS == 16;
+  constexpr int YS = HB_K + 2, YE = ROWS * HB_K / 256, XE = HB_B * HB_K / 256;
+  __shared__ __align__(16) double Ys[2][ROWS][YS];
+  __shared__ __align__(16) d2 Xs[2][HB_B][HB_K + 1];
+  const int t = threadIdx.x, w = t / 64, l = t % 64, g = l / 16, n = l % 16;
+  const int i0 = blockIdx.x * ROWS, b0 = blockIdx.y * (CPLX ? HB_B : 2 * HB_B);
+  const int kt = t % HB_K, rt = t / HB_K;  // this thread's column of a chunk; rows rt + 8 e
+  double yr[YE];
+  d2 xr[XE];
+  auto load = [&](int k0) {
+    const int k = k0 + kt;
 #pragma unroll
-    for (int e = 0; e < HB_M * HB_K / 256; ++e) {
-      const int idx = t + 256 * e;
-      const int ii = idx / HB_K, jj = idx % HB_K;
-      const int i = i0 + ii, j = j0 + jj;
-      Ys[ii][jj] = (i < nr && j < nr) ? Y[(size_t)i * nr + j] : 0.0;
+    for (int e = 0; e < YE; ++e) {
+      const int i = i0 + rt + 8 * e;
+      yr[e] = (i < nr && k < nr) ? Y[(size_t)i * nr + k] : 0.0;
     }
 #pragma unroll
-    for (int e = 0; e < HB_K * HB_B / 256; ++e) {
-      const int idx = t + 256 * e;
-      const int bb = idx / HB_K, jj = idx % HB_K;
-      const int b = b0 + bb, j = j0 + jj;
-      const bool ok = b < batch && j < nr;
+    for (int e = 0; e < XE; ++e) {
+      const int b = b0 + rt + 8 * e;
+      d2 v = {0.0, 0.0};
       if (CPLX) {
-        Xr[jj][bb] = ok ? in[2 * ((size_t)b * nr + j)] : 0.0;
-        Xi[jj][bb] = ok ? in[2 * ((size_t)b * nr + j) + 1] : 0.0;
+        if (b < batch && k < nr) v = *(const d2u*)(in + 2 * ((size_t)b * nr + k));
       } else {
-        Xr[jj][bb] = ok ? in[(size_t)b * nr + j] : 0.0;
+        if (b < batch && k < nr) v.x = in[(size_t)b * nr + k];
+        if (b + HB_B < batch && k < nr) v.y = in[(size_t)(b + HB_B) * nr + k];
       }
+      xr[e] = v;
     }
-    __syncthreads();
-#pragma unroll 8
-    for (int jj = 0; jj < HB_K; ++jj) {
-      const double xr = Xr[jj][tb];
-      const double xi = CPLX ? Xi[jj][tb] : 0.0;
+  };
+  d4 a0 = {0.0, 0.0, 0.0, 0.0}, a1 = a0;
+  load(0);
+  for (int k0 = 0, buf = 0; k0 < nr; k0 += HB_K, buf ^= 1) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const double y = Ys[ti + 16 * r][jj];
-        ar[r] = fma(y, xr, ar[r]);
-        if (CPLX) ai[r] = fma(y, xi, ai[r]);
-      }
-    }
+    for (int e = 0; e < YE; ++e) Ys[buf][rt + 8 * e][kt] = yr[e];
+#pragma unroll
+    for (int e = 0; e < XE; ++e) Xs[buf][rt + 8 * e][kt] = xr[e];
+    if (k0 + HB_K < nr) load(k0 + HB_K);
     __syncthreads();
+    constexpr int S = SPLIT ? HB_K / 16 : HB_K / 4;  // k per lane group and chunk
+    const int kb = SPLIT ? w * (HB_K / 4) + g * S : g * S;
+    const double* yp = &Ys[buf][SPLIT ? n : w * 16 + n][kb];
+    const d2* xp = &Xs[buf][n][kb];
+#pragma unroll
+    for (int s = 0; s < S; s += 2) {
+      const d2 y = *(const d2*)(yp + s), x0 = xp[s], x1 = xp[s + 1];
+      a0 = __builtin_amdgcn_mfma_f64_16x16x4f64(x0.x, y.x, a0, 0, 0, 0);
+      a1 = __builtin_amdgcn_mfma_f64_16x16x4f64(x0.y, y.x, a1, 0, 0, 0);
+      a0 = __builtin_amdgcn_mfma_f64_16x16x4f64(x1.x, y.y, a0, 0, 0, 0);
+      a1 = __builtin_amdgcn_mfma_f64_16x16x4f64(x1.y, y.y, a1, 0, 0, 0);
+    }
   }
-  const int b = b0 + tb;
-  if (b >= batch) return;
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int i = i0 + ti + 16 * r;
-    if (i >= nr) continue;
-    double vr = c * ar[r], vi = c * ai[r];
+  const int i = i0 + (SPLIT ? n : w * 16 + n);
+  auto store = [&](int v, double vr, double vi) {
+    const int b = b0 + v;
+    vr *= c;
+    vi *= c;
+    if (i >= nr) return;
     if (EPI == EPI_CUBIC) {
       const double m2 = vr * vr + vi * vi;
       vr *= m2;
       vi *= m2;
     } else if (EPI == EPI_TIMES_I) {
-      const double w = vr;
+      const double q = vr;
       vr = -gamma * vi;
-      vi = gamma * w;
+      vi = gamma * q;
     }
     if (CPLX) {
-      out[2 * ((size_t)b * nr + i)] = vr;
-      out[2 * ((size_t)b * nr + i) + 1] = vi;
+      if (b < batch) {
+        d2u o = {vr, vi};
+        *(d2u*)(out + 2 * ((size_t)b * nr + i)) = o;
+      }
     } else {
-      out[(size_t)b * nr + i] = vr;
+      if (b < batch) out[(size_t)b * nr + i] = vr;
+      if (b + HB_B < batch) out[(size_t)(b + HB_B) * nr + i] = vi;
     }
+  };
+  if constexpr (SPLIT) {
+    // the four partial sums in wave order; wave w finishes the results r = w
+    __shared__ d2 part[4][4][64];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) part[w][r][l] = d2{a0[r], a1[r]};
+    __syncthreads();
+    d2 v = part[0][w][l];
+#pragma unroll
+    for (int q = 1; q < 4; ++q) v += part[q][w][l];
+    store(4 * w + g, v.x, v.y);
+  } else {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) store(4 * r + g, a0[r], a1[r]);
   }
+}
+
+template <bool CPLX, int EPI>
+void hankel_launch(const double* Y, int nr, const double* in, double* out, int batch, double c, double gamma,
+                   hipStream_t stream) {
+  const int nb = (batch + (CPLX ? HB_B : 2 * HB_B) - 1) / (CPLX ? HB_B : 2 * HB_B), ni = (nr + 63) / 64;
+  if (ni * nb >= HB_CU)
+    hipLaunchKernelGGL((hankel_gemm<CPLX, EPI, 64>), dim3(ni, nb), dim3(256), 0, stream, Y, nr, in, out, batch, c,
+                       gamma);
+  else
+    hipLaunchKernelGGL((hankel_gemm<CPLX, EPI, 16>), dim3((nr + 15) / 16, nb), dim3(256), 0, stream, Y, nr, in, out,
+                       batch, c, gamma);
 }
 
 // Allocation-free cubic term (rks_hankel_cubic_noalloc): its |f|^2 f intermediate
@@ -190,13 +242,10 @@ int rks_hankel_apply(rks_hankel* h, int inverse, const void* in, void* out, int 
   if (in == out) return hfail(RKS_ERR_INVALID, "in and out must not alias");
   if (batch == 0) return RKS_OK;
   const double c = inverse ? 1.0 / h->scale : h->scale;
-  dim3 grid((h->nr + HB_M - 1) / HB_M, (batch + HB_B - 1) / HB_B);
   if (cplx)
-    hipLaunchKernelGGL((hankel_gemm<true, EPI_SCALE>), grid, dim3(256), 0, stream, h->d_Y, h->nr,
-                       (const double*)in, (double*)out, batch, c, 0.0);
+    hankel_launch<true, EPI_SCALE>(h->d_Y, h->nr, (const double*)in, (double*)out, batch, c, 0.0, stream);
   else
-    hipLaunchKernelGGL((hankel_gemm<false, EPI_SCALE>), grid, dim3(256), 0, stream, h->d_Y, h->nr,
-                       (const double*)in, (double*)out, batch, c, 0.0);
+    hankel_launch<false, EPI_SCALE>(h->d_Y, h->nr, (const double*)in, (double*)out, batch, c, 0.0, stream);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return hfail(RKS_ERR_HIP, std::string("rks_hankel_apply: ") + hipGetErrorString(e));
   return RKS_OK;
@@ -217,11 +266,8 @@ int rks_hankel_cubic(rks_hankel* h, double gamma, const void* in, void* out, int
     if (e != hipSuccess) return hfail(RKS_ERR_HIP, std::string("rks_hankel_cubic: ") + hipGetErrorString(e));
     h->tmp_batch = batch;
   }
-  dim3 grid((h->nr + HB_M - 1) / HB_M, (batch + HB_B - 1) / HB_B);
-  hipLaunchKernelGGL((hankel_gemm<true, EPI_CUBIC>), grid, dim3(256), 0, stream, h->d_Y, h->nr,
-                     (const double*)in, h->d_tmp, batch, 1.0 / h->scale, 0.0);
-  hipLaunchKernelGGL((hankel_gemm<true, EPI_TIMES_I>), grid, dim3(256), 0, stream, h->d_Y, h->nr,
-                     (const double*)h->d_tmp, (double*)out, batch, h->scale, gamma);
+  hankel_launch<true, EPI_CUBIC>(h->d_Y, h->nr, (const double*)in, h->d_tmp, batch, 1.0 / h->scale, 0.0, stream);
+  hankel_launch<true, EPI_TIMES_I>(h->d_Y, h->nr, h->d_tmp, (double*)out, batch, h->scale, gamma, stream);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return hfail(RKS_ERR_HIP, std::string("rks_hankel_cubic: ") + hipGetErrorString(e));
   return RKS_OK;
@@ -240,11 +286,8 @@ int rks_hankel_cubic_noalloc(rks_hankel* h, double gamma, const void* in, void* 
                                       std::to_string(kScratchDoubles / 2) + " complex values");
   double* scr = scratch_for(h->device);
   if (!scr) return hfail(RKS_ERR_HIP, "rks_hankel_cubic_noalloc: no scratch address for the transform's device");
-  dim3 grid((h->nr + HB_M - 1) / HB_M, (batch + HB_B - 1) / HB_B);
-  hipLaunchKernelGGL((hankel_gemm<true, EPI_CUBIC>), grid, dim3(256), 0, stream, h->d_Y, h->nr,
-                     (const double*)in, scr, batch, 1.0 / h->scale, 0.0);
-  hipLaunchKernelGGL((hankel_gemm<true, EPI_TIMES_I>), grid, dim3(256), 0, stream, h->d_Y, h->nr,
-                     (const double*)scr, (double*)out, batch, h->scale, gamma);
+  hankel_launch<true, EPI_CUBIC>(h->d_Y, h->nr, (const double*)in, scr, batch, 1.0 / h->scale, 0.0, stream);
+  hankel_launch<true, EPI_TIMES_I>(h->d_Y, h->nr, scr, (double*)out, batch, h->scale, gamma, stream);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return hfail(RKS_ERR_HIP, std::string("rks_hankel_cubic_noalloc: ") + hipGetErrorString(e));
   return RKS_OK;
