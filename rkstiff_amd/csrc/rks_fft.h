@@ -274,10 +274,10 @@ __device__ __forceinline__ void chain(cx<R>* buf, const cx<R>* twl, int t) {
 // is called.  Without PP they are free again when it returns; with PP the buffer of the
 // last exchange, (BUF + exchanges - 1) % 2, may still be read by other threads.
 template <typename R, int P, int T, bool INV, int LOG2N, int MAXR, bool PP, int BUF, bool FENCE, typename Post>
-__device__ __forceinline__ void fft_reg(cx<R> (&v)[P / T], cx<R>* buf, const cx<R>* twl, Post post) {
+__device__ __forceinline__ void fft_reg(cx<R> (&v)[P / T], cx<R>* buf, const cx<R>* twl, int t, Post post) {
   static_assert((P & (P - 1)) == 0, "power of two");
   static_assert(P / T >= 2, "need at least two elements per thread");
-  chain_reg<R, P, T, 1, INV, LOG2N, (1 << LOG2N) / P, MAXR, PP, BUF, FENCE>(v, buf, twl, threadIdx.x, post);
+  chain_reg<R, P, T, 1, INV, LOG2N, (1 << LOG2N) / P, MAXR, PP, BUF, FENCE>(v, buf, twl, t, post);
 }
 
 // G independent P-point transforms by one workgroup of G*TG threads: threads

@@ -541,7 +541,7 @@ __device__ __forceinline__ ChunkIdx<CH> own_chunk(int c, const Own<N, M, T, NLK>
   ix.fold = ow.fold;
 #pragma unroll
   for (int i = 0; i < CH; ++i) {
-    const int x = (int)threadIdx.x + (c * CH + i) * T;
+    const int x = ow.t + (c * CH + i) * T;
     ix.ok[i] = x < ow.lim;
     ix.m[i] = ix.ok[i] ? x : 0;
   }
@@ -830,13 +830,13 @@ __device__ __forceinline__ void final_chunk(const rks_tableau& tb, const cx<RS>*
 // barriers.  Called by all threads; the LDS buffers are free at the call and at the
 // return.
 // ---------------------------------------------------------------------------
-// modes per chunk of the stage combination of the generic kernels
-#ifndef RKS_CHUNK
-#define RKS_CHUNK 8
-#endif
-template <int MPT>
+// Modes per chunk of the stage combination of the generic kernels.  Eight FP64 modes with
+// their NL values, coefficients and addresses spill (992 bytes of scratch per lane at n =
+// 8192, four: 352; an ETD34 step 213 us, four: 179).
+template <int MPT, int ES>
 struct Chunk {
-  static constexpr int CH = MPT < RKS_CHUNK ? MPT : RKS_CHUNK;
+  static constexpr int MAX = ES > 8 && MPT >= 8 ? 4 : 8;
+  static constexpr int CH = MPT < MAX ? MPT : MAX;
   static constexpr int NCH = (MPT + CH - 1) / CH;
 };
 
@@ -947,19 +947,24 @@ __device__ __forceinline__ void nl_regs(cx<R> (&v)[MPT], cx<R>* buf, const cx<R>
   constexpr int N = 1 << LOG2N;
   constexpr bool PP = rks_two_buffers<R, LOG2N, T, NLK>();
   constexpr int PS = rksfft::padded_size(N);
-  const int t = threadIdx.x;
+  // An opaque copy of the thread index, as in Own::fresh: the transforms' LDS addresses are
+  // formed here, at each call.  Hoisted out of the stage loop they were held (and spilled)
+  // through it: 448 bytes of scratch per lane at n = 8192 (advective IF34 FP64), now 128, and
+  // a step 122 -> 112 us; 640 -> 80 in FP32, the KS ensemble (2048) 23.8 -> 22.5 ms.
+  int t = threadIdx.x;
+  asm volatile("" : "+v"(t));
   const R inv = (R)1 / (R)N;
   if constexpr (NLK == NLK_HANKEL) {
     nl_hankel<R, LOG2N, T, MPT>(v, buf, coef, kx, nr, hs);
   } else if constexpr (NLK == NLK_CUBIC) {
     constexpr int X = rksfft::exchanges<N, T, RKS_MAXR>();
-    rksfft::fft_reg<R, N, T, true, LOG2N, RKS_MAXR, PP, 0, true>(v, buf, twl, [&](C w) {
+    rksfft::fft_reg<R, N, T, true, LOG2N, RKS_MAXR, PP, 0, true>(v, buf, twl, t, [&](C w) {
       const C v1 = inv * w;
       const R a = v1.re * v1.re + v1.im * v1.im;
       return a * v1;
     });
-    rksfft::fft_reg<R, N, T, false, LOG2N, RKS_MAXR, PP, X & 1, false>(v, buf, twl,
-                                                               [&](C w) { return mkc(-coef * w.im, coef * w.re); });
+    rksfft::fft_reg<R, N, T, false, LOG2N, RKS_MAXR, PP, X & 1, false>(
+        v, buf, twl, t, [&](C w) { return mkc(-coef * w.im, coef * w.re); });
     if constexpr (PP) __syncthreads();
   } else {
     // inverse transform of the spectrum of u + i u_x: Y[m] = U + iV, Y[N-m] = conj(U) +
@@ -998,7 +1003,7 @@ __device__ __forceinline__ void nl_regs(cx<R> (&v)[MPT], cx<R>* buf, const cx<R>
 #pragma unroll
     for (int k = 0; k < EH; ++k) y[EH + k] = buf[pad(t + k * T)];
     if constexpr (!PP) __syncthreads();
-    rksfft::fft_reg<R, N, T, true, LOG2N, RKS_MAXR, PP, 1, true>(y, buf, twl, [](C w) { return w; });
+    rksfft::fft_reg<R, N, T, true, LOG2N, RKS_MAXR, PP, 1, true>(y, buf, twl, t, [](C w) { return w; });
     // u u_x, a real sequence: complex element j of its half-length transform is the pair 2j, 2j+1
     constexpr int B2 = PP ? (1 + XI) & 1 : 0;
     C* const bp = buf + B2 * PS;
@@ -1013,7 +1018,7 @@ __device__ __forceinline__ void nl_regs(cx<R> (&v)[MPT], cx<R>* buf, const cx<R>
     for (int k = 0; k < EH; ++k) z[k] = bp[pad(t + k * T)];
     if constexpr (!PP) __syncthreads();
     constexpr int B3 = PP ? (B2 + 1) & 1 : 0;
-    rksfft::fft_reg<R, H, T, false, LOG2N, RKS_MAXR, PP, B3, true>(z, buf, twl, [](C w) { return w; });
+    rksfft::fft_reg<R, H, T, false, LOG2N, RKS_MAXR, PP, B3, true>(z, buf, twl, t, [](C w) { return w; });
     constexpr int B4 = PP ? (B3 + XF) & 1 : 0;
     C* const bm = buf + B4 * PS;
 #pragma unroll
@@ -1170,7 +1175,7 @@ __device__ int run_instance(const rks_launch& P, int idx, cx<R>* buf, const cx<R
   constexpr int M = (NLK == NLK_ADVECT) ? N / 2 + 1 : N;
   using OW = Own<N, M, T, NLK>;
   constexpr int MPT = OW::MPT;
-  constexpr int CH = Chunk<MPT>::CH;
+  constexpr int CH = Chunk<MPT, (int)sizeof(C)>::CH;
   constexpr bool METHOD = METH != RKS_METH_ANY;
   using TT = MethodTab<METHOD ? METH : 0, (int)sizeof(C), (int)sizeof(CN), NLK == NLK_ADVECT>;
   constexpr bool FUSED = TT::tab.st[TT::tab.nstage - 1].has_nl == 0;  // (METHOD) no NL in the last stage
@@ -1372,8 +1377,8 @@ __device__ int run_instance(const rks_launch& P, int idx, cx<R>* buf, const cx<R
           if (last && fused) {
             // per-mode |u_new| and |err|^2 (FP32 buffer: |err|) wait in the idle LDS buffer
 #pragma unroll 1
-            for (int c = 0; c < Chunk<MPT>::NCH; ++c) {
-              const ChunkIdx<CH> ix = own_chunk<N, M, T, NLK, CH>(c, ow);
+            for (int c = 0; c < Chunk<MPT, (int)sizeof(C)>::NCH; ++c) {
+              const ChunkIdx<CH> ix = own_chunk<N, M, T, NLK, CH>(c, ow.fresh());
               C acc[CH], ev[CH];
               final_chunk<R, RN, CH>(tb, u, slot, cbase, (size_t)Mc, ix, h, acc, ev);
 #pragma unroll
@@ -1396,8 +1401,8 @@ __device__ int run_instance(const rks_launch& P, int idx, cx<R>* buf, const cx<R
           // the stage argument through the thread's own places of the LDS buffer: the
           // run-time term loop stays rolled over the chunks
 #pragma unroll 1
-          for (int c = 0; c < Chunk<MPT>::NCH; ++c) {
-            const ChunkIdx<CH> ix = own_chunk<N, M, T, NLK, CH>(c, ow);
+          for (int c = 0; c < Chunk<MPT, (int)sizeof(C)>::NCH; ++c) {
+            const ChunkIdx<CH> ix = own_chunk<N, M, T, NLK, CH>(c, ow.fresh());
             C acc[CH];
             stage_chunk<R, RN, CH>(tb, S, u, slot, cbase, (size_t)Mc, ix, h, acc);
 #pragma unroll
@@ -1413,9 +1418,10 @@ __device__ int run_instance(const rks_launch& P, int idx, cx<R>* buf, const cx<R
           }
           if (!S.has_nl) continue;
 #pragma unroll
-          for (int k = 0; k < MPT; ++k) v[k] = buf[ow.m(k)];
+          for (int k = 0; k < MPT; ++k) v[k] = buf[of.m(k)];
           __syncthreads();
           ns = S.nl_slot;
+          const OW of = ow.fresh();
         }
         nl_regs<R, LOG2N, T, NLK>(v, buf, twl, nlc, kx, Mr, hs);
         ++nl_calls;
@@ -1508,7 +1514,7 @@ __device__ int run_instance(const rks_launch& P, int idx, cx<R>* buf, const cx<R
         constexpr int NCH = (NO::SLOTS + CH - 1) / CH;
 #pragma unroll 1
         for (int c = 0; c < NCH; ++c) {
-          ChunkIdx<CH> ix = own_chunk<N, M, T, NLK, CH>(c, ow);
+          ChunkIdx<CH> ix = own_chunk<N, M, T, NLK, CH>(c, ow.fresh());
 #pragma unroll
           for (int i = 0; i < CH; ++i) {
             ix.ok[i] = NO::ok(c * CH + i, ow.lim);
