@@ -25,7 +25,7 @@ EXPORTS = (
     "rks_mlp_gradient", "rks_mlp_infer_single", "rks_plan_set_proposer", "rks_set_records",
     "rks_read_records", "rks_hankel_create", "rks_hankel_destroy", "rks_hankel_apply", "rks_hankel_cubic",
     "rks_hankel_cubic_noalloc", "rks_dense_coeffs", "rks_dense_combine",
-    "rks_plan_buckets", "rks_plan_set_launch", "rks_plan_set_priority",
+    "rks_plan_buckets", "rks_plan_set_launch", "rks_plan_tiles", "rks_plan_set_priority",
 )
 
 # learned step-size proposer (include/rkstiff_amd.h)
@@ -162,6 +162,7 @@ def load(path=None):
         lib.rks_dense_combine.argtypes = [ip, ip, vp, ip, vp, vp]
         lib.rks_plan_buckets.argtypes = [vp, P(ip), P(ip), P(ip), P(ip), P(ip), ip]
         lib.rks_plan_set_launch.argtypes = [vp, ip, P(ip), P(ip), ip]
+        lib.rks_plan_tiles.argtypes = [vp, P(ip), ip]
         lib.rks_plan_set_priority.argtypes = [vp, P(dp)]
         lib.rks_last_error.restype = ctypes.c_char_p
         for name in EXPORTS:

@@ -93,7 +93,7 @@ def tune_launch(plan, u0, t0, tf, h, reps=2, min_gain=0.02):
             l2 = buckets[bucket][0]
             only = [tfs[i] if inst_l2[i] == l2 else t0s[i] for i in range(n)]
             sec = _timed(plan, u0, uf, t0s, only, hs, reps)
-        trials.append({"concurrent": conc, "wg_per_cu": list(wg), "tile": list(ti), "bucket": bucket,
+        trials.append({"concurrent": conc, "wg_per_cu": list(wg), "tile": plan.tiles(), "bucket": bucket,
                        "seconds": sec})
         return sec
 
@@ -142,7 +142,12 @@ def tune_launch(plan, u0, t0, tf, h, reps=2, min_gain=0.02):
             best, best_conc = sec, False
         if not best < default:
             best, best_conc, best_wg, best_ti = default, True, list(wg0), list(ti0)
-    plan.set_launch(best_conc, best_wg, best_ti)
+    # the tiles the library chooses by size (wider ones than can be set per bucket among them)
+    sec = trial(best_conc, best_wg, None)
+    own = best_ti
+    if sec < best:
+        best, own, best_ti = sec, None, plan.tiles()
+    plan.set_launch(best_conc, best_wg, own)
     # longest first: the attempts of a pilot over the whole ensemble estimate each
     # trajectory's cost
     plan.evolve(u0, uf, t0s, tfs, hs)
@@ -200,7 +205,7 @@ def tune_together(jobs, reps=2, min_gain=0.02, warm=True, uniform=False):
         la = plan.launch or {}
         shapes.append({"concurrent": la.get("concurrent", True),
                        "wg": list(la.get("wg_per_cu") or [0] * nb),
-                       "tile": list(la.get("tile") or [0] * nb)})
+                       "tile": [min(x, b[3] - 1) for x, b in zip(plan.tiles(), plan.buckets())]})
 
     def apply():
         for (plan, *_), sh in zip(runs, shapes):

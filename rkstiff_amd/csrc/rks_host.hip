@@ -108,6 +108,17 @@ __global__ void rks_transpose(const double* a, R* b, int n) {
     b[i] = (R)a[(i % n) * n + i / n];
 }
 
+// Per log2 n, the advective trajectories whose last mode is not damped at DAMPED times the rate at which a
+// field of unit size is advected across it (-Re L >= DAMPED |coef| k).
+constexpr double DAMPED = 100.0;
+__global__ void rks_count_undamped(const rks_inst* inst, int ninst, int* count) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= ninst) return;
+  const rks_inst& r = inst[i];
+  const int m = r.m - 1;
+  const double re = r.L_complex ? r.L[2 * m] : r.L[m];
+  if (!(-re >= DAMPED * fabs(r.nl_coef) * ((const double*)r.kx)[m])) atomicAdd(&count[32 - __clz(m)], 1);
+}
 
 // ===========================================================================
 // host side: plans and the C ABI
@@ -168,7 +179,7 @@ int method_variant(int method, int nlk, int coef_real) {
 }
 
 // learn: the proposer variant (a proposer or training records are attached);
-// tile: 0 the default tile, 1 twice the threads per trajectory (n = 2^9 .. 2^12)
+// tile: 0 the base tile (rks_threads), 1 twice and 2 four times the threads per trajectory
 bool lookup(int prec, int nlk, int variant, int log2n, bool learn, KernelEntry* e, int tile = 0) {
 #define RKS_PICK(p)                                                                                        \
   do {                                                                                                     \
@@ -189,6 +200,39 @@ bool lookup(int prec, int nlk, int variant, int log2n, bool learn, KernelEntry* 
   if (prec == RKS_MIXED) RKS_PICK(mix);
   RKS_PICK(f32);
 #undef RKS_PICK
+}
+
+// Tile of a bucket of `count` trajectories whose caller chose none.  A trajectory is a serial
+// chain of butterflies, exchanges and stage sums, so more waves with fewer modes each shorten
+// every link of it, until a transform takes more passes or a workgroup's registers and LDS
+// keep others off a loaded CU.  Measured per FP64 evolve, base tile / twice / four times
+// (MI355X):
+//   cubic ETD35  n = 512   x 1   3.49 / 2.21 ms          x 256   5.7 / 3.8 ms
+//                n = 1024  x 1   6.73 / 3.80 / 2.38      x 256  11.5 / 6.7 / 4.0
+//                n = 2048  x 1   6.68 / 4.09 / 3.24      x 256  13.2 / 7.8 / 5.3
+//                n = 4096  x 1   7.60 / 5.65 / 7.09      x 256  19.1 / 14.5 / 15.3
+//                n = 8192  x 1  12.04 / 12.77            x 256  30.2 / 27.0
+//   advect IF34  n = 512   x 1   1.85 / 1.60             x 256   2.8 / 2.5
+//                n = 1024  x 1   3.28 / 2.32 / 2.16      x 256   4.0 / 3.1 / 2.9
+//                n = 2048  x 1   4.08 / 2.80 / 3.06      x 256   6.1 / 4.0 / 4.1
+//                n = 4096  x 1   4.93 / 3.94 / 6.24      x 256   8.2 / 5.8 / 8.9
+//                n = 8192  x 1   7.91 / 9.71             x 256  12.7 / 16.7
+// FP32 and MIXED runs gain as much, but keep the base tile: a tile has its own order of
+// rounding, and in FP32 storage that moves the step sizes and with them the results (MIXED
+// soliton ensembles by 4e-9, FP32 KS by 3e-6), so there the caller chooses.  Likewise an
+// advective term on a grid whose last modes are not damped (rks_count_undamped): a spectrum
+// that reaches the grid's end amplifies rounding (viscosity 5e-4, n = 4096: 2e-3 of the
+// state; KS: 1e-13).  The proposer
+// counts accepted steps by the workgroup's size, so its kernels keep the base tile; so do
+// runs that log their attempts, whose logs compare with the proposer's attempt by attempt.
+int default_tile(int prec, int nlk, int log2n, int count, int cu, bool base_only) {
+  if (base_only || prec != RKS_F64 || nlk == RKS_NL_HANKEL_CUBIC || log2n < 9) return 0;
+  if (nlk == RKS_NL_CUBIC_FFT) {
+    if (log2n == 10 || log2n == 11) return 2;
+    return log2n == 13 ? 2 * count > cu : 1;
+  }
+  if (log2n == 10) return count <= cu ? 2 : 1;
+  return log2n == 13 ? 0 : 1;
 }
 
 int ilog2(int n) {
@@ -249,7 +293,8 @@ struct rks_plan {
   // cap on resident workgroups per CU per bucket (0: as many as fit)
   int concurrent = 1;
   std::vector<int> wg_per_cu;
-  std::vector<int> tile;  // per bucket: 0 default tile, 1 twice the threads
+  std::vector<int> undamped;  // per log2 n: trajectories whose rounding at the grid's end need not decay
+  std::vector<int> tile;  // per bucket: 0 base tile, 1 twice, 2 four times the threads, -1 by default_tile
   std::vector<hipStream_t> bstream;
   std::vector<hipEvent_t> bdone;
   hipEvent_t fork = nullptr;
@@ -541,8 +586,9 @@ int rks_plan_create(int method, int nl_kind, int precision, const rks_config* cf
       KernelEntry el;
       if (lookup(precision, nl_kind, p->variant, l, true, &el))
         HIPCHK(hipFuncSetAttribute(el.fn, hipFuncAttributeMaxDynamicSharedMemorySize, el.lds));
-      if (lookup(precision, nl_kind, p->variant, l, false, &el, 1))
-        HIPCHK(hipFuncSetAttribute(el.fn, hipFuncAttributeMaxDynamicSharedMemorySize, el.lds));
+      for (int tile = 1; tile <= 2; ++tile)
+        if (lookup(precision, nl_kind, p->variant, l, false, &el, tile))
+          HIPCHK(hipFuncSetAttribute(el.fn, hipFuncAttributeMaxDynamicSharedMemorySize, el.lds));
       if (hankel) continue;  // no transform tables
       const int N = 1 << l;
       HIPCHK(hipMalloc(&p->d_tw[l], (size_t)N * p->esize));
@@ -555,6 +601,13 @@ int rks_plan_create(int method, int nl_kind, int precision, const rks_config* cf
       HIPCHK(hipGetLastError());
     }
     HIPCHK(hipMemcpy(p->d_order, p->order.data(), sizeof(int) * ninst, hipMemcpyHostToDevice));
+    p->undamped.assign(14, 0);
+    if (nl_kind == RKS_NL_ADVECT_RFFT && precision == RKS_F64) {
+      hipLaunchKernelGGL(rks_zero_int, dim3(1), dim3(64), 0, 0, p->d_queue, 64);
+      hipLaunchKernelGGL(rks_count_undamped, dim3((ninst + 255) / 256), dim3(256), 0, 0, p->d_inst, ninst, p->d_queue);
+      HIPCHK(hipGetLastError());
+      HIPCHK(hipMemcpy(p->undamped.data(), p->d_queue, sizeof(int) * 14, hipMemcpyDeviceToHost));
+    }
     HIPCHK(hipDeviceSynchronize());
   }
   *out = p;
@@ -668,6 +721,13 @@ static char* inst_cbase(const rks_plan* p, int inst) {
          2 * rks_align256(M * p->esize);
 }
 
+// the tile that bucket b runs on: the caller's choice, else default_tile
+static int bucket_tile(const rks_plan* p, size_t b) {
+  if (b < p->tile.size() && p->tile[b] >= 0) return p->tile[b];
+  return default_tile(p->prec, p->nlk, p->bucket_log2[b], p->bucket_count[b], p->cu,
+                      p->undamped[p->bucket_log2[b]] || p->mlp.on || p->d_rec != nullptr || p->d_log != nullptr);
+}
+
 static int launch_all(rks_plan* p, int mode, double h_mode, hipStream_t stream) {
   if (p->c2) {
     const hipError_t e = rks2_run(p->c2, p->tab, mode, stream);
@@ -705,7 +765,7 @@ static int launch_all(rks_plan* p, int mode, double h_mode, hipStream_t stream) 
   for (size_t b = 0; b < nb; ++b) {
     KernelEntry e;
     const bool learn = p->mlp.on || p->d_rec != nullptr;
-    const int ti = b < p->tile.size() ? p->tile[b] : 0;
+    const int ti = bucket_tile(p, b);
     if (!lookup(p->prec, p->nlk, p->variant, p->bucket_log2[b], learn, &e, ti))
       return fail(RKS_ERR_INVALID, "no kernel for this grid size, variant and tile");
     L.order = p->d_order + p->bucket_start[b];
@@ -1026,7 +1086,7 @@ int rks_plan_buckets(rks_plan* p, int* nbucket, int* log2n, int* count, int* max
     if (count) count[b] = p->bucket_count[b];
     if (ntile) {
       KernelEntry e1;
-      ntile[b] = lookup(p->prec, p->nlk, p->variant, p->bucket_log2[b], false, &e1, 1) ? 2 : 1;
+      ntile[b] = lookup(p->prec, p->nlk, p->variant, p->bucket_log2[b], true, &e1, 1) ? 2 : 1;
     }
     if (max_wg_per_cu) {
       KernelEntry e;
@@ -1045,7 +1105,7 @@ int rks_plan_set_launch(rks_plan* p, int concurrent, const int* wg_per_cu, const
   if (p->c2) return fail(RKS_ERR_INVALID, "the 2-D engine has a fixed launch sequence");
   const int nb = (int)p->bucket_log2.size();
   if ((wg_per_cu || tile) && nbucket != nb) return fail(RKS_ERR_INVALID, "one value per size bucket needed");
-  std::vector<int> w(nb, 0), ti(nb, 0);
+  std::vector<int> w(nb, 0), ti(nb, -1);
   for (int b = 0; b < nb; ++b) {
     if (wg_per_cu) {
       if (wg_per_cu[b] < 0) return fail(RKS_ERR_INVALID, "wg_per_cu must be >= 0");
@@ -1053,7 +1113,8 @@ int rks_plan_set_launch(rks_plan* p, int concurrent, const int* wg_per_cu, const
     }
     if (tile) {
       KernelEntry e1;
-      if (tile[b] != 0 && !(tile[b] == 1 && lookup(p->prec, p->nlk, p->variant, p->bucket_log2[b], false, &e1, 1)))
+      // a chosen tile must have its proposer variant, which a caller may attach later
+      if (tile[b] != 0 && !(tile[b] == 1 && lookup(p->prec, p->nlk, p->variant, p->bucket_log2[b], true, &e1, 1)))
         return fail(RKS_ERR_INVALID, "tile 1 exists for n = 512 .. 4096 only");
       ti[b] = tile[b];
     }
@@ -1061,6 +1122,12 @@ int rks_plan_set_launch(rks_plan* p, int concurrent, const int* wg_per_cu, const
   p->concurrent = concurrent ? 1 : 0;
   p->wg_per_cu = w;
   p->tile = ti;
+  return RKS_OK;
+}
+
+int rks_plan_tiles(rks_plan* p, int* tile, int cap) {
+  if (!p || !tile) return fail(RKS_ERR_INVALID, "null argument");
+  for (size_t b = 0; b < p->bucket_log2.size() && (int)b < cap; ++b) tile[b] = bucket_tile(p, b);
   return RKS_OK;
 }
 

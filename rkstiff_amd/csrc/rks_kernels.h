@@ -840,12 +840,16 @@ struct Chunk {
   static constexpr int NCH = (MPT + CH - 1) / CH;
 };
 
+// exchange buffers must leave room for the twiddle tables and the reduction scratch (160 KB per CU)
+#define RKS_LDS_MAX (148 * 1024)
+
 // Two exchange buffers where they fit beside the register-bound number of waves: a
 // workgroup takes at most 512 threads x 16 elements x 8 bytes (padded, 70 KB) per
 // buffer then, and a one-wave workgroup has no barriers to save.
 template <typename R, int LOG2N, int T, int NLK>
 __host__ __device__ constexpr bool rks_two_buffers() {
-  return NLK != NLK_HANKEL && T > 64 && ((1 << LOG2N) / T) * (int)sizeof(cx<R>) <= 128;
+  return NLK != NLK_HANKEL && T > 64 && ((1 << LOG2N) / T) * (int)sizeof(cx<R>) <= 128 &&
+         2 * rksfft::padded_size(1 << LOG2N) * (int)sizeof(cx<R>) <= RKS_LDS_MAX;
 }
 
 // LDS elements of the exchange buffers
@@ -1417,11 +1421,11 @@ __device__ int run_instance(const rks_launch& P, int idx, cx<R>* buf, const cx<R
             }
           }
           if (!S.has_nl) continue;
+          const OW of = ow.fresh();
 #pragma unroll
           for (int k = 0; k < MPT; ++k) v[k] = buf[of.m(k)];
           __syncthreads();
           ns = S.nl_slot;
-          const OW of = ow.fresh();
         }
         nl_regs<R, LOG2N, T, NLK>(v, buf, twl, nlc, kx, Mr, hs);
         ++nl_calls;
@@ -1715,7 +1719,7 @@ template <typename R, typename RN, int LOG2N, int NLK, bool LEARN, int TILE, int
 __global__ __launch_bounds__(rks_threads(LOG2N, NLK) << TILE, rks_min_waves(LOG2N, (int)sizeof(R))) void rks_kernel(
     rks_launch P) {
   constexpr int T = rks_threads(LOG2N, NLK) << TILE;
-  static_assert(T <= 512 && (NLK == NLK_HANKEL || T <= (NLK == NLK_ADVECT ? (1 << LOG2N) / 4 : (1 << LOG2N) / 2)),
+  static_assert(T <= 1024 && (NLK == NLK_HANKEL || T <= (NLK == NLK_ADVECT ? (1 << LOG2N) / 4 : (1 << LOG2N) / 2)),
                 "tile too wide");
   extern __shared__ __align__(16) unsigned char rks_smem[];
   __shared__ double red[2 * (T / 64 + 1)];

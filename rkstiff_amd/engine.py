@@ -161,6 +161,14 @@ class Plan:
 
     def set_launch(self, concurrent=True, wg_per_cu=None, tile=None):
         def arr(v):
+    def tiles(self):
+        """The FFT tile each size bucket runs on: as set by ``set_launch``, else by size,
+        precision and number of trajectories (rks_plan_set_launch)."""
+        nb = len(self.buckets())
+        arr = (ctypes.c_int * max(nb, 1))()
+        _lib.check(self.lib.rks_plan_tiles(self.h, arr, nb))
+        return list(arr[:nb])
+
             return None if v is None else (ctypes.c_int * len(v))(*[int(x) for x in v])
         n = len(wg_per_cu) if wg_per_cu is not None else (len(tile) if tile is not None else 0)
         _lib.check(self.lib.rks_plan_set_launch(self.h, 1 if concurrent else 0, arr(wg_per_cu), arr(tile), n))
