@@ -308,6 +308,12 @@ int rks_hankel_cubic_noalloc(rks_hankel* h, double gamma, const void* in, void* 
  * after the work is done (its work buffers are released). */
 int rks_dense_coeffs(int method, int n, int batch, const void* L, const double* h, int contour_points,
                      double contour_radius, void* coeffs, hipStream_t stream);
+/* The same in the caller's work memory (device, 256-byte aligned, at least
+ * the *bytes of rks_dense_ws_bytes): the launches are queued on `stream` and ws
+ * must live until they are done. */
+int rks_dense_ws_bytes(int method, int n, int batch, int contour_points, size_t* bytes);
+int rks_dense_coeffs_ws(int method, int n, int batch, const void* L, const double* h, int contour_points,
+                        double contour_radius, void* coeffs, void* ws, size_t ws_bytes, hipStream_t stream);
 #define RKS_DENSE_MAX_TERMS 8
 /* One term of a stage sum: alpha * mat (x + s2 x2); mat NULL: the identity,
  * x2 NULL: no second vector. */

@@ -24,7 +24,8 @@ EXPORTS = (
     "rks_mlp_create", "rks_mlp_destroy", "rks_mlp_get_params", "rks_mlp_train", "rks_mlp_forward",
     "rks_mlp_gradient", "rks_mlp_infer_single", "rks_plan_set_proposer", "rks_set_records",
     "rks_read_records", "rks_hankel_create", "rks_hankel_destroy", "rks_hankel_apply", "rks_hankel_cubic",
-    "rks_hankel_cubic_noalloc", "rks_dense_coeffs", "rks_dense_combine",
+    "rks_hankel_cubic_noalloc", "rks_dense_coeffs", "rks_dense_ws_bytes", "rks_dense_coeffs_ws",
+    "rks_dense_combine",
     "rks_plan_buckets", "rks_plan_set_launch", "rks_plan_tiles", "rks_plan_set_priority",
 )
 
@@ -159,6 +160,8 @@ def load(path=None):
         lib.rks_hankel_cubic.argtypes = [vp, dp, vp, vp, ip, vp]
         lib.rks_hankel_cubic_noalloc.argtypes = [vp, dp, vp, vp, ip, vp]
         lib.rks_dense_coeffs.argtypes = [ip, ip, ip, vp, P(dp), ip, dp, vp, vp]
+        lib.rks_dense_ws_bytes.argtypes = [ip, ip, ip, ip, P(ctypes.c_size_t)]
+        lib.rks_dense_coeffs_ws.argtypes = [ip, ip, ip, vp, P(dp), ip, dp, vp, vp, ctypes.c_size_t, vp]
         lib.rks_dense_combine.argtypes = [ip, ip, vp, ip, vp, vp]
         lib.rks_plan_buckets.argtypes = [vp, P(ip), P(ip), P(ip), P(ip), P(ip), ip]
         lib.rks_plan_set_launch.argtypes = [vp, ip, P(ip), P(ip), ip]

@@ -44,9 +44,14 @@ def coefficients(method, L, h, etd_config=None):
     ncoef = _lib.tableau(method).ncoef
     out = torch.empty((B, ncoef, n, n), dtype=torch.complex128, device=L.device)
     harr = (ctypes.c_double * B)(*hs)
-    _lib.check(lib.rks_dense_coeffs(_lib.METHOD_IDS[method], n, B, ctypes.c_void_p(L.data_ptr()), harr,
-                                    int(etd.contour_points), float(etd.contour_radius),
-                                    ctypes.c_void_p(out.data_ptr()), _stream()))
+    mid, points = _lib.METHOD_IDS[method], int(etd.contour_points)
+    # work memory from torch's stream-ordered allocator: nothing to wait for before it is reused
+    nbytes = ctypes.c_size_t()
+    _lib.check(lib.rks_dense_ws_bytes(mid, n, B, points, ctypes.byref(nbytes)))
+    ws = torch.empty(nbytes.value, dtype=torch.uint8, device=L.device)
+    _lib.check(lib.rks_dense_coeffs_ws(mid, n, B, ctypes.c_void_p(L.data_ptr()), harr, points,
+                                       float(etd.contour_radius), ctypes.c_void_p(out.data_ptr()),
+                                       ctypes.c_void_p(ws.data_ptr()), ws.numel(), _stream()))
     return out
 
 
