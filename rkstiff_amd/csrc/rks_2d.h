@@ -9,8 +9,8 @@
 // attempt is a fixed sequence of kernels over all trajectories, each one pass
 // over HBM:
 //   col   forward column FFTs of the previous stage's transform buffer T
-//         -> NL slot; the next stage combination E u + sum C NL formed in
-//         registers; inverse column FFTs -> T (CG adjacent columns per
+//         -> NL slot; the next stage combination E u + sum C NL; inverse
+//         column FFTs -> T, all in registers (CG adjacent columns per
 //         workgroup, so every row segment read or written is contiguous)
 //   row   per pair of rows: one complex inverse FFT of both rows' half
 //         spectra, w - c w^3 on the real and imaginary parts, one forward
@@ -18,8 +18,8 @@
 //   norm  masked sums of the embedded error norm (solveras.py:449-455),
 //         FP64 partials per workgroup
 //   ctrl  FP64 accept/reject and dt per trajectory (solveras.py:384-410,
-//         457-554; evolve 605-650)
-// begin/ctrl/snap keep each trajectory's own controller state, so finished
+//         457-554; evolve 605-650), and the start of the next attempt
+// ctrl/snap keep each trajectory's own controller state, so finished
 // or rejected trajectories drop out of (or repeat) work per launch while the
 // others advance.  The host captures the sequence once into a hipGraph and
 // replays it until no trajectory is running.
@@ -66,10 +66,18 @@ struct Geo2 {
   // a column tile's row segments do not straddle cache lines
   static constexpr int TXS = rks2_t_stride(N, (int)sizeof(cx<R>));
   static constexpr int PS = rksfft::padded_size(N);
+  // column kernel: consecutive lanes hold the same element of CG columns, then the next
+  // element; a buffer stride of 4 modulo 32 (FP64: 2 modulo 16) elements spreads both over
+  // the banks
+  static constexpr int CBM = sizeof(R) == 4 ? 32 : 16, CBR = sizeof(R) == 4 ? 4 : 2;
+  static constexpr int CPS = PS + (CBM + CBR - PS % CBM) % CBM;
   static constexpr int TWS = rksfft::TwSplit<LOG2>::SIZE;
   // column kernel: CG columns of N points, CTG threads per column
   static constexpr int CG = sizeof(R) == 4 ? 16 : 8;
-  static constexpr int CTG = (N / 2 < 512 / CG) ? N / 2 : 512 / CG;
+  // At least four points a thread, for fewer passes on short columns: 8 x 64^2 ETD35 FP64 3.4 ms
+  // with two (radix 2 throughout), 2.7 with four, 3.1 with eight (too few waves); 128^2 3.37,
+  // 3.22, 3.38
+  static constexpr int CTG = (N / 4 < 512 / CG) ? N / 4 : 512 / CG;
   static constexpr int CT = CG * CTG;
   static constexpr int CEPT = N / CTG;  // tile elements per thread
   // modes per chunk of the stage combination: 4 in FP64 keeps the column
@@ -77,11 +85,11 @@ struct Geo2 {
   static constexpr int CCH_MAX = sizeof(R) == 4 ? 8 : 4;
   static constexpr int CCH = CEPT < CCH_MAX ? CEPT : CCH_MAX;
   static constexpr int NCG = (NXH + CG - 1) / CG;
-  static constexpr int COL_LDS = (CG * PS + TWS) * (int)sizeof(cx<R>);
+  static constexpr int COL_LDS = (CG * CPS + TWS) * (int)sizeof(cx<R>);
   // row kernel: RG complex transforms (2 RG rows), RTG threads each (N = 512:
   // 64 threads, 8 points each, three radix-8 passes)
   static constexpr int RG = 8;
-  static constexpr int RTG = (N / 2 < 512 / RG) ? N / 2 : 512 / RG;
+  static constexpr int RTG = (N / 4 < 512 / RG) ? N / 4 : 512 / RG;
   static constexpr int RT = RG * RTG;
   static constexpr int NRG = N / (2 * RG);
   static constexpr int ROW_LDS = (RG * PS + TWS) * (int)sizeof(cx<R>);
@@ -142,13 +150,19 @@ __device__ __forceinline__ void rks2_states(const rks2_launch& P, const rks_inst
 // idle at that point, for k2_norm_fused.  A separate instantiation, so the
 // other stages keep their register allocation (no spills at 4 waves per SIMD).
 // METH: the stage sums of one method as literals (rks_method.h), else the tableau.
-// A pass is bound by HBM once its loads are all in flight; the interpreted fused pass was not
-// (64 x 512^2 ETD35 FP32: 370 us for 0.8 GB).  The whole batch went 75.2 -> 61.2 ms with the
-// literal passes and coefficients, 8 x 128^2 FP64 10.3 -> 6.6 ms (there the coefficients were
-// 71 of 240 us an attempt: one thread summed a small mode's contour means).
+// A thread holds rows r0 + i CTG of one column from the load of T to its store: both
+// transforms take their first inputs from and leave their results in registers (chain_reg),
+// the NL values just formed enter the next stage sum without a trip to memory, and only the
+// exchanges between the transforms' passes go through LDS.  What bounds a pass then is HBM:
+// 64 x 512^2 ETD35 FP32, 0.5 GB for a middle stage.  Batches, one evolve, tableau read from
+// memory / literal sums with transforms from LDS to LDS / in registers:
+//   64 x 512^2 FP32, tf = 4    75.2 / 60.7 / 55.8 ms    8 x 128^2 FP64, tf = 4   10.3 / 6.6 / 5.4 ms
+//   32 x 512^2 FP64, tf = 2    41.3 / - / 23.5 ms
+// The generic kernels (METH = RKS_METH_ANY) form their stage sums over mirror row pairs and
+// pass them to the transform's rows through LDS.
 
-// The chunk's modes for the literal stage sums: mirror row pairs (slot 2j row q, slot
-// 2j + 1 row n - q), coefficients of the mirror row where L is mirror-symmetric.
+// Modes of the literal stage sums: slot k holds row row[k] of a column; coefficients of the
+// mirror row where L is mirror-symmetric.
 template <int N, int XS, int CH>
 struct OwnRows {
   int row[CH];
@@ -172,7 +186,7 @@ __global__ __launch_bounds__((Geo2<R, LOG2>::CT), 4) void k2_col(rks2_launch P, 
   using rksfft::pad;
   constexpr int N = G::N, NXH = G::NXH, XS = G::XS, MI = G::MI, CG = G::CG, CT = G::CT, CEPT = G::CEPT;
   // the fused last stage keeps the candidate and the error per mode: half the chunk
-  constexpr int CH = (FUSE && G::CCH >= 4) ? G::CCH / 2 : G::CCH, NCH = CEPT / CH, RS = CT / CG, PS = G::PS;
+  constexpr int CH = (FUSE && G::CCH >= 4) ? G::CCH / 2 : G::CCH, NCH = CEPT / CH, RS = CT / CG, PS = G::CPS;
   extern __shared__ __align__(16) unsigned char rks2_smem[];
   __shared__ double red[2 * (CT / 64 + 1)];
   const int inst = blockIdx.y;
@@ -203,120 +217,142 @@ __global__ __launch_bounds__((Geo2<R, LOG2>::CT), 4) void k2_col(rks2_launch P, 
   C* const bc = buf + c * PS;
   const C zero = mkc((R)0, (R)0);
   __syncthreads();
+  constexpr bool METHOD = METH != RKS_METH_ANY;
+  using TT = MethodTab<METHOD ? METH : 0, (int)sizeof(C), (int)sizeof(CN), true>;
+  // the last NL values of a method that recomputes NL1 are only read by this very pass
+  constexpr bool KEEP_LAST = !(FUSE && METHOD && TT::tab.nl1_policy == RKS_NL1_RECOMPUTE);
+  C w[CEPT];  // rows r0 + i RS: NL values, then the stage argument
+#pragma unroll
+  for (int i = 0; i < CEPT; ++i) w[i] = zero;
   if (fwd_slot >= 0 && (!fwd_need_nl1 || st.need_nl1)) {
 #pragma unroll
-    for (int i = 0; i < CEPT; ++i) {
-      const int r = r0 + i * RS;
-      bc[pad(r)] = valid ? Tb[r * G::TXS + col] : zero;
-    }
-    __syncthreads();
-    rksfft::fft_multi<R, N, G::CTG, CG, false, LOG2, RKS_MAXR>(buf, twl);
+    for (int i = 0; i < CEPT; ++i) w[i] = valid ? Tb[(r0 + i * RS) * G::TXS + col] : zero;
+    rksfft::chain_reg<R, N, G::CTG, 1, false, LOG2, 1, RKS_MAXR, false, 0, true>(w, bc, twl, r0, [](C z) { return z; });
     if (valid) {
       if (P.mode == RKS_MODE_NL) {
         C* dst = (C*)io.u_out;
 #pragma unroll
-        for (int i = 0; i < CEPT; ++i) {
-          const int r = r0 + i * RS;
-          dst[r * NXH + col] = bc[pad(r)];
-        }
-      } else {
+        for (int i = 0; i < CEPT; ++i) dst[(r0 + i * RS) * NXH + col] = w[i];
+      } else if (KEEP_LAST) {
         CN* dst = slot(fwd_slot);
 #pragma unroll
-        for (int i = 0; i < CEPT; ++i) {
-          const int r = r0 + i * RS;
-          dst[r * XS + col] = cvt<RN>(bc[pad(r)]);
-        }
+        for (int i = 0; i < CEPT; ++i) gstore(dst, (r0 + i * RS) * XS + col, cvt<RN>(w[i]));
       }
     }
-    __syncthreads();
   }
   if (arg < -1) return;
+  if constexpr (!METHOD) __syncthreads();  // the rows below are other threads'
   const bool has_nl = arg < 0 || tb.st[arg].has_nl;
   const bool last = arg >= 0 && arg == tb.nstage - 1;
   const int sym = in->coef_sym;
   const size_t Mc = sym ? G::MSYM : MI;
   const bool fused = FUSE && last;
-  constexpr bool METHOD = METH != RKS_METH_ANY;
-  using TT = MethodTab<METHOD ? METH : 0, (int)sizeof(C), (int)sizeof(CN), true>;
   double mx = 0.0;
-  // stage combination over mirror row pairs: slot 2j row q = r0 + (ch CH/2 + j) RS,
-  // slot 2j + 1 row n - q (n/2 for q = 0), so a mirror-symmetric L shares coefficients
-#pragma unroll 1
-  for (int ch = 0; ch < NCH; ++ch) {
-    ChunkIdx<CH> ix;
-    int row[CH];
-    ix.sym = sym;
-    ix.lim = G::MGEN_SYM_I;
-    ix.anyq = 0;
-    ix.fold = 0;
+  if constexpr (METHOD) {
+    // the thread's own rows r0 + i RS, whose NL values of the stage before are still in w
+    CN nv[CEPT];
 #pragma unroll
-    for (int j = 0; j < CH / 2; ++j) {
-      const int q = r0 + (ch * (CH / 2) + j) * RS;
-      row[2 * j] = q;
-      row[2 * j + 1] = q == 0 ? N / 2 : N - q;
-      ix.m[2 * j] = valid ? row[2 * j] * XS + col : 0;
-      ix.m[2 * j + 1] = valid ? row[2 * j + 1] * XS + col : 0;
-      ix.ok[2 * j] = ix.ok[2 * j + 1] = valid;
-    }
-    C acc[CH];
-    if constexpr (METHOD) {
-      OwnRows<N, XS, CH> ow;
+    for (int i = 0; i < CEPT; ++i) nv[i] = cvt<RN>(w[i]);
+    if constexpr (FUSE) {
+      constexpr int NEW = TT::tab.st[TT::tab.nstage > 1 ? TT::tab.nstage - 2 : 0].nl_slot;
 #pragma unroll
-      for (int i = 0; i < CH; ++i) ow.row[i] = row[i];
-      ow.col = col;
-      ow.sym = sym;
-      ow.valid = valid;
-      CN none[CH];  // no NL values kept in registers between kernels
+      for (int ch = 0; ch < NCH; ++ch) {
+        OwnRows<N, XS, CH> ow;
+        CN nc[CH];
 #pragma unroll
-      for (int i = 0; i < CH; ++i) none[i] = mkc((RN)0, (RN)0);
-      if (fused) {
-        if constexpr (FUSE) {
-          double a[CH], e[CH];
-          final_sum<TT, -1, 0, CH, false>(a, e, cand, none, u, ow, slot, cbase, Mc, h);
-#pragma unroll
-          for (int i = 0; i < CH; ++i) {
-            if (!valid) continue;
-            gstore(Tb, row[i] * G::TXS + col, mkc((R)a[i], (R)e[i]));
-            mx = nanmax(mx, a[i]);
-          }
+        for (int i = 0; i < CH; ++i) {
+          ow.row[i] = r0 + (ch * CH + i) * RS;
+          nc[i] = nv[ch * CH + i];
         }
-        continue;
-      }
-      if (arg < 0) {
+        ow.col = col;
+        ow.sym = sym;
+        ow.valid = valid;
+        double a[CH], e[CH];
+        final_sum<TT, NEW, 0, CH, false>(a, e, cand, nc, u, ow, slot, cbase, Mc, h);
 #pragma unroll
-        for (int i = 0; i < CH; ++i) acc[i] = valid ? gload(u, row[i] * ustride + col) : zero;
-      } else {
-        stage_switch<TT, 0, false>(arg, acc, none, u, ow, slot, cbase, Mc, h);
+        for (int i = 0; i < CH; ++i) {
+          if (!valid) continue;
+          gstore(Tb, ow.row[i] * G::TXS + col, mkc((R)a[i], (R)e[i]));
+          mx = nanmax(mx, a[i]);
+        }
       }
     } else if (arg < 0) {
 #pragma unroll
-      for (int i = 0; i < CH; ++i) acc[i] = valid ? u[row[i] * ustride + col] : zero;
-    } else if (fused) {
-      if constexpr (FUSE) {
-        C ev[CH];
-        final_chunk<R, RN, CH>(tb, u, slot, cbase, Mc, ix, h, acc, ev);
+      for (int i = 0; i < CEPT; ++i) w[i] = valid ? gload(u, (r0 + i * RS) * ustride + col) : zero;
+    } else {
+      OwnRows<N, XS, CEPT> ow;
 #pragma unroll
-        for (int i = 0; i < CH; ++i) {
-          if (valid) {
-            const double a = hypot((double)acc[i].re, (double)acc[i].im);
-            const double er = (double)ev[i].re, ei = (double)ev[i].im;
-            if constexpr (sizeof(R) == sizeof(double))
-              Tb[row[i] * G::TXS + col] = mkc((R)a, (R)(er * er + ei * ei));
-            else
-              Tb[row[i] * G::TXS + col] = mkc((R)a, (R)hypot(er, ei));
+      for (int i = 0; i < CEPT; ++i) ow.row[i] = r0 + i * RS;
+      ow.col = col;
+      ow.sym = sym;
+      ow.valid = valid;
+      stage_switch<TT, 0, true, G::CCH>(arg, w, nv, u, ow, slot, cbase, Mc, h);
+#pragma unroll
+      for (int i = 0; i < CEPT; ++i) {
+        if (last && valid) {
+          gstore(cand, ow.m(i), w[i]);
+          mx = nanmax(mx, hypot((double)w[i].re, (double)w[i].im));
+        }
+        if (!valid) w[i] = zero;
+      }
+    }
+  } else {
+    // over mirror row pairs: slot 2j row q = r0 + (ch CH/2 + j) RS, slot 2j + 1 row n - q
+    // (n/2 for q = 0), so a mirror-symmetric L shares coefficients
+#pragma unroll 1
+    for (int ch = 0; ch < NCH; ++ch) {
+      ChunkIdx<CH> ix;
+      int row[CH];
+      ix.sym = sym;
+      ix.lim = G::MGEN_SYM_I;
+      ix.anyq = 0;
+      ix.fold = 0;
+#pragma unroll
+      for (int j = 0; j < CH / 2; ++j) {
+        const int q = r0 + (ch * (CH / 2) + j) * RS;
+        row[2 * j] = q;
+        row[2 * j + 1] = q == 0 ? N / 2 : N - q;
+        ix.m[2 * j] = valid ? row[2 * j] * XS + col : 0;
+        ix.m[2 * j + 1] = valid ? row[2 * j + 1] * XS + col : 0;
+        ix.ok[2 * j] = ix.ok[2 * j + 1] = valid;
+      }
+      C acc[CH];
+      if (arg < 0) {
+#pragma unroll
+        for (int i = 0; i < CH; ++i) acc[i] = valid ? u[row[i] * ustride + col] : zero;
+      } else if (fused) {
+        if constexpr (FUSE) {
+          C ev[CH];
+          final_chunk<R, RN, CH>(tb, u, slot, cbase, Mc, ix, h, acc, ev);
+#pragma unroll
+          for (int i = 0; i < CH; ++i) {
+            if (valid) {
+              const double a = hypot((double)acc[i].re, (double)acc[i].im);
+              const double er = (double)ev[i].re, ei = (double)ev[i].im;
+              if constexpr (sizeof(R) == sizeof(double))
+                Tb[row[i] * G::TXS + col] = mkc((R)a, (R)(er * er + ei * ei));
+              else
+                Tb[row[i] * G::TXS + col] = mkc((R)a, (R)hypot(er, ei));
+            }
           }
         }
+      } else {
+        stage_chunk<R, RN, CH>(tb, tb.st[arg], u, slot, cbase, Mc, ix, h, acc);
       }
-    } else {
-      stage_chunk<R, RN, CH>(tb, tb.st[arg], u, slot, cbase, Mc, ix, h, acc);
-    }
 #pragma unroll
-    for (int i = 0; i < CH; ++i) {
-      if (last && valid) {
-        cand[ix.m[i]] = acc[i];
-        mx = nanmax(mx, hypot((double)acc[i].re, (double)acc[i].im));
+      for (int i = 0; i < CH; ++i) {
+        if (last && valid) {
+          cand[ix.m[i]] = acc[i];
+          mx = nanmax(mx, hypot((double)acc[i].re, (double)acc[i].im));
+        }
+        if (has_nl) bc[pad(row[i])] = valid ? acc[i] : zero;
       }
-      if (has_nl) bc[pad(row[i])] = valid ? acc[i] : zero;
+    }
+    if (has_nl) {
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < CEPT; ++i) w[i] = bc[pad(r0 + i * RS)];
+      __syncthreads();
     }
   }
   if (last && tb.adaptive) {
@@ -324,14 +360,10 @@ __global__ __launch_bounds__((Geo2<R, LOG2>::CT), 4) void k2_col(rks2_launch P, 
     if (t == 0) P.pmax[inst * P.ncg + blockIdx.x] = mx;
   }
   if (has_nl) {
-    __syncthreads();
-    rksfft::fft_multi<R, N, G::CTG, CG, true, LOG2, RKS_MAXR>(buf, twl);
+    rksfft::chain_reg<R, N, G::CTG, 1, true, LOG2, 1, RKS_MAXR, false, 0, true>(w, bc, twl, r0, [](C z) { return z; });
     if (valid) {
 #pragma unroll
-      for (int i = 0; i < CEPT; ++i) {
-        const int r = r0 + i * RS;
-        Tb[r * G::TXS + col] = bc[pad(r)];
-      }
+      for (int i = 0; i < CEPT; ++i) gstore(Tb, (r0 + i * RS) * G::TXS + col, w[i]);
     }
   }
 }
@@ -375,16 +407,23 @@ __global__ __launch_bounds__((Geo2<R, LOG2>::RT)) void k2_row(rks2_launch P, int
     }
   }
   __syncthreads();
-  rksfft::fft_multi<R, N, G::RTG, RG, true, LOG2, RKS_MAXR>(buf, twl);
-  for (int e = t; e < RG * N; e += RT) {
-    const int g = e / N, j = e - g * N;
-    C* bg = buf + g * PS;
-    const C z = bg[pad(j)];
-    const R w1 = z.re * inv, w2 = z.im * inv;
-    bg[pad(j)] = mkc(w1 - c3 * (w1 * w1 * w1), w2 - c3 * (w2 * w2 * w2));
-  }
+  // both transforms and the pointwise term between them in registers (chain_reg): an exchange
+  // through LDS per pass but the last, instead of one per pass and two around the term
+  constexpr int RTG = G::RTG, EPT = N / RTG;
+  const int q = t % RTG;
+  C* const bq = buf + (t / RTG) * PS;
+  C v[EPT];
+#pragma unroll
+  for (int k = 0; k < EPT; ++k) v[k] = bq[pad(q + k * RTG)];
   __syncthreads();
-  rksfft::fft_multi<R, N, G::RTG, RG, false, LOG2, RKS_MAXR>(buf, twl);
+  rksfft::chain_reg<R, N, RTG, 1, true, LOG2, 1, RKS_MAXR, false, 0, true>(v, bq, twl, q, [&](C z) {
+    const R w1 = z.re * inv, w2 = z.im * inv;
+    return mkc(w1 - c3 * (w1 * w1 * w1), w2 - c3 * (w2 * w2 * w2));
+  });
+  rksfft::chain_reg<R, N, RTG, 1, false, LOG2, 1, RKS_MAXR, false, 0, true>(v, bq, twl, q, [](C z) { return z; });
+#pragma unroll
+  for (int k = 0; k < EPT; ++k) bq[pad(q + k * RTG)] = v[k];
+  __syncthreads();
   for (int e = t; e < RG * NXH; e += RT) {
     const int g = e / NXH, k = e - g * NXH;
     const C* bg = buf + g * PS;
@@ -404,6 +443,7 @@ template <typename R, typename RN, int LOG2, int METH>
 __global__ __launch_bounds__(256) void k2_coef(rks2_launch P) {
   using G = Geo2<R, LOG2>;
   const int inst = blockIdx.y;
+  if (inst == 0 && blockIdx.x == 0 && threadIdx.x == 0) *P.active_count = 0;  // k2_ctrl counts anew
   const rks2_state st = P.st[inst];
   if (!st.active || !st.need_coef) return;
   const rks_inst* in = P.inst + inst;
@@ -459,6 +499,17 @@ __global__ __launch_bounds__(256) void k2_coef(rks2_launch P) {
 }
 
 
+// Largest of the n partial maxima, the same in every lane: a lane per partial (one load, not
+// n in a row).
+__device__ __forceinline__ double rks2_max(const double* p, int n) {
+  const int lane = threadIdx.x & 63;
+  double mx = p[lane < n ? lane : 0];
+  for (int j = lane + 64; j < n; j += 64) mx = nanmax(mx, p[j]);
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) mx = nanmax(mx, __shfl_xor(mx, o, 64));
+  return mx;
+}
+
 // ---------------------------------------------------------------------------
 // norm: masked sums |u_new|^2, |err|^2 over modes with |u_new|/max > cutoff
 // ---------------------------------------------------------------------------
@@ -482,9 +533,7 @@ __global__ __launch_bounds__(256) void k2_norm(rks2_launch P) {
   const C* u;
   C* cand;
   rks2_states<R>(P, in, io, &u, &cand);
-  const double* pm = P.pmax + (size_t)inst * P.ncg;
-  double mx = pm[0];
-  for (int j = 1; j < P.ncg; ++j) mx = nanmax(mx, pm[j]);
+  const double mx = rks2_max(P.pmax + (size_t)inst * P.ncg, P.ncg);
   const int t = threadIdx.x;
   // NE/2 mirror row pairs per thread: pair p = (q, col) holds rows q and n - q (n/2 for q = 0)
   constexpr int N = G::N, NXH = G::NXH, XS = G::XS;
@@ -541,9 +590,7 @@ __global__ __launch_bounds__(256) void k2_norm_fused(rks2_launch P) {
   if (!st.active) return;
   const rks_inst* in = P.inst + inst;
   const C* Tb = (const C*)((const char*)in->ws + P.off_T);
-  const double* pm = P.pmax + (size_t)inst * P.ncg;
-  double mx = pm[0];
-  for (int j = 1; j < P.ncg; ++j) mx = nanmax(mx, pm[j]);
+  const double mx = rks2_max(P.pmax + (size_t)inst * P.ncg, P.ncg);
   const double cut = P.ctl->adapt_cutoff;
   const int t = threadIdx.x;
   double su = 0.0, se = 0.0;
@@ -574,7 +621,7 @@ __global__ __launch_bounds__(256) void k2_norm_fused(rks2_launch P) {
 }
 
 // ---------------------------------------------------------------------------
-// per-trajectory control (one block; a thread per trajectory)
+// per-trajectory control
 // ---------------------------------------------------------------------------
 // set-up of a launch: evolve / resume / step (run_instance's set-up)
 __global__ void k2_init(rks2_launch P) {
@@ -618,128 +665,147 @@ __global__ void k2_init(rks2_launch P) {
     }
     in.numloops = 0;
   }
+  if (threadIdx.x == 0) *P.active_count = 0;
 }
 
-// start of an attempt: who runs, coefficient and NL1 needs, FSAL slot swap
-__global__ void k2_begin(rks2_launch P) {
-  __shared__ int cnt[4];
+// Start of an attempt of trajectory i, by one thread: who runs, coefficient and NL1 needs,
+// FSAL slot swap.
+__device__ __forceinline__ void rks2_begin(const rks2_launch& P, rks_inst& in, rks2_state& st) {
   const rks_tableau& tb = *P.tab;
-  int n_active = 0;
-  for (int i = threadIdx.x; i < P.ninst; i += blockDim.x) {
-    rks2_state& st = P.st[i];
-    rks_inst& in = P.inst[i];
-    st.store = 0;
-    int active = 0;
-    if (in.status == RKS_ST_RUNNING) {
-      const bool evolve = P.mode == RKS_MODE_EVOLVE;
-      if (evolve && !(in.tc < in.tf)) in.status = RKS_ST_OK;
-      else if (evolve && in.store_freq > 0 && in.snap_count >= in.snap_cap) in.status = RKS_ST_PAUSED;
-      else active = 1;
-    }
-    st.active = active;
-    st.need_nl1 = 0;
-    st.need_coef = 0;
-    if (!active) continue;
-    ++n_active;
-    if (in.h != in.h_coeff) {
-      st.need_coef = 1;
-      in.h_coeff = in.h;
-      ++in.coef_updates;
-    }
-    if (!in.started) {
-      st.need_nl1 = 1;
-      in.started = 1;
-    } else if (in.accept || !tb.adaptive) {
-      if (tb.nl1_policy == RKS_NL1_RECOMPUTE) {
-        st.need_nl1 = 1;
-      } else {
-        const int f = tb.fsal_slot, a = in.slot_map[0];
-        in.slot_map[0] = in.slot_map[f];
-        in.slot_map[f] = a;
-      }
-    }
-    int nl = st.need_nl1;
-    for (int s = 0; s < tb.nstage; ++s) nl += tb.st[s].has_nl ? 1 : 0;
-    in.nl_calls += nl;
+  int active = 0;
+  if (in.status == RKS_ST_RUNNING) {
+    const bool evolve = P.mode == RKS_MODE_EVOLVE;
+    if (evolve && !(in.tc < in.tf)) in.status = RKS_ST_OK;
+    else if (evolve && in.store_freq > 0 && in.snap_count >= in.snap_cap) in.status = RKS_ST_PAUSED;
+    else active = 1;
   }
-  // block sum of n_active (blockDim.x = 256)
-  for (int o = 32; o >= 1; o >>= 1) n_active += __shfl_xor(n_active, o, 64);
-  if ((threadIdx.x & 63) == 0) cnt[threadIdx.x >> 6] = n_active;
-  __syncthreads();
-  if (threadIdx.x == 0) *P.active_count = cnt[0] + cnt[1] + cnt[2] + cnt[3];
+  st.active = active;
+  st.need_nl1 = 0;
+  st.need_coef = 0;
+  if (!active) return;
+  atomicAdd(P.active_count, 1);
+  if (in.h != in.h_coeff) {
+    st.need_coef = 1;
+    in.h_coeff = in.h;
+    ++in.coef_updates;
+  }
+  if (!in.started) {
+    st.need_nl1 = 1;
+    in.started = 1;
+  } else if (in.accept || !tb.adaptive) {
+    if (tb.nl1_policy == RKS_NL1_RECOMPUTE) {
+      st.need_nl1 = 1;
+    } else {
+      const int f = tb.fsal_slot, a = in.slot_map[0];
+      in.slot_map[0] = in.slot_map[f];
+      in.slot_map[f] = a;
+    }
+  }
+  int nl = st.need_nl1;
+  for (int s = 0; s < tb.nstage; ++s) nl += tb.st[s].has_nl ? 1 : 0;
+  in.nl_calls += nl;
 }
 
-// end of an attempt: error ratio, accept/reject, dt, time, snapshots
-__global__ void k2_ctrl(rks2_launch P) {
+// the first attempt's start (the others': k2_ctrl); one block per trajectory, as k2_ctrl
+__global__ void k2_begin(rks2_launch P) {
+  if (threadIdx.x == 0) rks2_begin(P, P.inst[blockIdx.x], P.st[blockIdx.x]);
+}
+
+// End of an attempt of a trajectory, by one thread: error ratio from the sums, accept/reject,
+// dt, time, snapshots.
+__device__ __forceinline__ void rks2_end(const rks2_launch& P, rks_inst& in, rks2_state& st, int i, double su,
+                                         double se) {
   const rks_tableau& tb = *P.tab;
   const rks_ctrl& ct = *P.ctl;
-  for (int i = threadIdx.x; i < P.ninst; i += blockDim.x) {
-    rks2_state& st = P.st[i];
-    if (!st.active) continue;
-    rks_inst& in = P.inst[i];
-    const double h = in.h;
-    double h_suggest = h;
-    if (tb.adaptive) {
-      double su = 0.0, se = 0.0;
-      const double* ps = P.psum + 2 * (size_t)i * P.nnb;
-      for (int b = 0; b < P.nnb; ++b) {
-        su += ps[2 * b];
-        se += ps[2 * b + 1];
-      }
-      const double sv = rks_error_ratio(su, se, ct.epsilon, ct.safety_f, tb.q, P.lowp != 0);
-      ++in.attempts;
-      if (in.log_count < in.log_cap) {
-        in.log[2 * in.log_count] = h;
-        in.log[2 * in.log_count + 1] = sv;
-      }
-      ++in.log_count;
-      if (isinf(sv) || isnan(sv) || sv < 1.0) {  // reject (solveras.py:490-506)
-        in.accept = 0;
-        ++in.rejects;
-        double hn;
-        if (isinf(sv) || isnan(sv)) {
-          hn = ct.min_s * h;
-        } else {
-          double sc = sv > ct.min_s ? sv : ct.min_s;
-          sc = sc < ct.decr_f ? sc : ct.decr_f;
-          hn = sc * h;
-        }
-        in.h = hn;
-        ++in.numloops;
-        if (in.numloops > ct.max_loops) in.status = RKS_ST_MAXLOOPS;
-        else if (hn < ct.minh) in.status = RKS_ST_MINSTEP;
-        continue;
-      }
-      in.accept = 1;  // accept (solveras.py:543-554)
-      const double sc = sv < ct.max_s ? sv : ct.max_s;
-      h_suggest = (sc > ct.incr_f) ? sc * h : h;
-    } else {
-      in.accept = 1;
+  const double h = in.h;
+  double h_suggest = h;
+  if (tb.adaptive) {
+    const double sv = rks_error_ratio(su, se, ct.epsilon, ct.safety_f, tb.q, P.lowp != 0);
+    ++in.attempts;
+    if (in.log_count < in.log_cap) {
+      in.log[2 * in.log_count] = h;
+      in.log[2 * in.log_count + 1] = sv;
     }
-    in.numloops = 0;
-    in.h_used = h;
-    in.h_next = h_suggest;
-    if (P.mode != RKS_MODE_EVOLVE) {
-      in.status = RKS_ST_OK;
-      ++in.steps;
-      continue;
+    ++in.log_count;
+    if (isinf(sv) || isnan(sv) || sv < 1.0) {  // reject (solveras.py:490-506)
+      in.accept = 0;
+      ++in.rejects;
+      double hn;
+      if (isinf(sv) || isnan(sv)) {
+        hn = ct.min_s * h;
+      } else {
+        double sc = sv > ct.min_s ? sv : ct.min_s;
+        sc = sc < ct.decr_f ? sc : ct.decr_f;
+        hn = sc * h;
+      }
+      in.h = hn;
+      ++in.numloops;
+      if (in.numloops > ct.max_loops) in.status = RKS_ST_MAXLOOPS;
+      else if (hn < ct.minh) in.status = RKS_ST_MINSTEP;
+      return;
     }
-    in.ubuf = in.ubuf == 0 ? 1 : 0;
-    const double tprev = in.tc;
-    in.tc += h;
+    in.accept = 1;  // accept (solveras.py:543-554)
+    const double sc = sv < ct.max_s ? sv : ct.max_s;
+    h_suggest = (sc > ct.incr_f) ? sc * h : h;
+  } else {
+    in.accept = 1;
+  }
+  in.numloops = 0;
+  in.h_used = h;
+  in.h_next = h_suggest;
+  if (P.mode != RKS_MODE_EVOLVE) {
+    in.status = RKS_ST_OK;
     ++in.steps;
-    if (!(in.tc > tprev)) {  // h below the resolution of tc
-      in.status = RKS_ST_MINSTEP;
-      continue;
-    }
-    if (tb.adaptive) in.h = (in.tc + h_suggest > in.tf) ? in.tf - in.tc : h_suggest;  // solveras.py:638-641
-    if (in.store_freq > 0 && (in.steps % in.store_freq) == 0) {
-      st.store = 1;
-      st.snap_idx = in.snap_count;
-      in.snap_t[in.snap_count] = in.tc;
-      ++in.snap_count;
+    return;
+  }
+  in.ubuf = in.ubuf == 0 ? 1 : 0;
+  const double tprev = in.tc;
+  in.tc += h;
+  ++in.steps;
+  if (!(in.tc > tprev)) {  // h below the resolution of tc
+    in.status = RKS_ST_MINSTEP;
+    return;
+  }
+  if (tb.adaptive) in.h = (in.tc + h_suggest > in.tf) ? in.tf - in.tc : h_suggest;  // solveras.py:638-641
+  if (in.store_freq > 0 && (in.steps % in.store_freq) == 0) {
+    st.store = 1;
+    st.snap_idx = in.snap_count;
+    in.snap_t[in.snap_count] = in.tc;
+    ++in.snap_count;
+  }
+}
+
+// Between two attempts: the end of one and the start of the next, a wave per trajectory.  The
+// partial sums are loaded a lane each and added in order by one lane from LDS; loaded one after
+// the other by a thread per trajectory they took 23 us at n = 512 (65 partials).
+__global__ __launch_bounds__(64) void k2_ctrl(rks2_launch P) {
+  __shared__ double part[2 * 64];
+  const int i = blockIdx.x, t = threadIdx.x;
+  rks_inst& in = P.inst[i];
+  rks2_state& st = P.st[i];
+  double su = 0.0, se = 0.0;
+  const bool active = st.active != 0;
+  if (active && P.tab->adaptive) {
+    const double* ps = P.psum + 2 * (size_t)i * P.nnb;
+    for (int b0 = 0; b0 < P.nnb; b0 += 64) {
+      const int nb = P.nnb - b0 < 64 ? P.nnb - b0 : 64;
+      __syncthreads();
+      if (t < nb) {
+        part[2 * t] = ps[2 * (b0 + t)];
+        part[2 * t + 1] = ps[2 * (b0 + t) + 1];
+      }
+      __syncthreads();
+      if (t == 0)
+        for (int b = 0; b < nb; ++b) {
+          su += part[2 * b];
+          se += part[2 * b + 1];
+        }
     }
   }
+  if (t != 0) return;
+  st.store = 0;
+  if (active) rks2_end(P, in, st, i, su, se);
+  rks2_begin(P, in, st);
 }
 
 // The caller's u0 (rfft2 layout, row stride NXH) into cand0 (row stride XS):

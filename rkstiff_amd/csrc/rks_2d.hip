@@ -15,8 +15,8 @@ struct rks2_ctx {
   int* d_active = nullptr;
   int* h_active = nullptr;  // pinned
   hipStream_t cap = nullptr;
-  hipGraph_t graph[2] = {nullptr, nullptr};  // evolve, step
-  hipGraphExec_t exec[2] = {nullptr, nullptr};
+  hipGraph_t graph[3] = {nullptr, nullptr, nullptr};  // evolve, step, evolve with snapshots
+  hipGraphExec_t exec[3] = {nullptr, nullptr, nullptr};
   bool use_graph = true;
 };
 
@@ -57,9 +57,8 @@ struct Eng2 {
   static void out(const rks2_launch& L, hipStream_t s) {
     hipLaunchKernelGGL((k2_out<R, LOG2>), dim3(copy_blocks(), L.ninst), dim3(256), 0, s, L);
   }
-  // one attempt of every running trajectory
-  static void attempt(const rks2_launch& L, const rks_tableau& tb, hipStream_t s) {
-    hipLaunchKernelGGL(k2_begin, dim3(1), dim3(256), 0, s, L);
+  // one attempt of every running trajectory (store: one may keep snapshots)
+  static void attempt(const rks2_launch& L, const rks_tableau& tb, bool store, hipStream_t s) {
     // a mode per thread until there are 8 workgroups for every CU, then several
     const int one = (G::M + 255) / 256, cap = 2048 / L.ninst > one / 8 ? 2048 / L.ninst : one / 8 + 1;
     hipLaunchKernelGGL((k2_coef<R, RN, LOG2, METH>), dim3(one < cap ? one : cap, L.ninst), dim3(256), 0, s, L);
@@ -84,8 +83,8 @@ struct Eng2 {
       hipLaunchKernelGGL((k2_norm_fused<R, LOG2>), dim3(G::NNB, L.ninst), dim3(G::NT), 0, s, L);
     else if (tb.adaptive)
       hipLaunchKernelGGL((k2_norm<R, RN, LOG2>), dim3(G::NNB, L.ninst), dim3(G::NT), 0, s, L);
-    hipLaunchKernelGGL(k2_ctrl, dim3(1), dim3(256), 0, s, L);
-    snap(L, s);
+    hipLaunchKernelGGL(k2_ctrl, dim3(L.ninst), dim3(64), 0, s, L);
+    if (store) snap(L, s);
   }
   static void nl(const rks2_launch& L, hipStream_t s) {
     col(L, s, -1, 0, -1, 1);
@@ -182,8 +181,8 @@ int rks2_create(rks2_ctx** out, int prec, int variant, int log2n, int ninst, con
 }
 
 // the attempt sequence of `mode`, captured once
-static hipGraphExec_t attempt_graph(rks2_ctx* c, const rks_tableau& tb, int mode) {
-  const int gi = mode == RKS_MODE_EVOLVE ? 0 : 1;
+static hipGraphExec_t attempt_graph(rks2_ctx* c, const rks_tableau& tb, int mode, bool store) {
+  const int gi = mode != RKS_MODE_EVOLVE ? 1 : (store ? 2 : 0);
   if (c->exec[gi] || !c->use_graph) return c->exec[gi];
   if (!c->cap && hipStreamCreateWithFlags(&c->cap, hipStreamNonBlocking) != hipSuccess) {
     c->use_graph = false;
@@ -195,7 +194,7 @@ static hipGraphExec_t attempt_graph(rks2_ctx* c, const rks_tableau& tb, int mode
     c->use_graph = false;
     return nullptr;
   }
-  with_engine(c->prec, c->variant, c->log2n, [&](auto eng) { decltype(eng)::attempt(L, tb, c->cap); });
+  with_engine(c->prec, c->variant, c->log2n, [&](auto eng) { decltype(eng)::attempt(L, tb, store, c->cap); });
   hipGraph_t g = nullptr;
   if (hipStreamEndCapture(c->cap, &g) != hipSuccess || !g) {
     c->use_graph = false;
@@ -212,7 +211,8 @@ static hipGraphExec_t attempt_graph(rks2_ctx* c, const rks_tableau& tb, int mode
   return x;
 }
 
-hipError_t rks2_run(rks2_ctx* c, const rks_tableau& tb, int mode, hipStream_t s) {
+hipError_t rks2_run(rks2_ctx* c, const rks_tableau& tb, int mode, bool store, hipStream_t s) {
+  store = store && mode == RKS_MODE_EVOLVE;
   rks2_launch L = c->L;
   L.mode = mode;
   hipLaunchKernelGGL(k2_init, dim3(1), dim3(256), 0, s, L);
@@ -222,10 +222,11 @@ hipError_t rks2_run(rks2_ctx* c, const rks_tableau& tb, int mode, hipStream_t s)
   }
   // the caller's state into the internal layout (a resumed evolve keeps its own)
   with_engine(c->prec, c->variant, c->log2n, [&](auto eng) { decltype(eng)::in(L, s); });
-  if (mode == RKS_MODE_EVOLVE) with_engine(c->prec, c->variant, c->log2n, [&](auto eng) { decltype(eng)::snap(L, s); });
+  if (store) with_engine(c->prec, c->variant, c->log2n, [&](auto eng) { decltype(eng)::snap(L, s); });
+  hipLaunchKernelGGL(k2_begin, dim3(c->ninst), dim3(64), 0, s, L);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipGraphExec_t g = attempt_graph(c, tb, mode);
+  hipGraphExec_t g = attempt_graph(c, tb, mode, store);
   // every attempt either advances tc (bounded by tf and the resolution guard)
   // or counts towards max_loops, so the loop ends; the cap only guards bugs
   const long long cap = 200000000LL;
@@ -233,7 +234,7 @@ hipError_t rks2_run(rks2_ctx* c, const rks_tableau& tb, int mode, hipStream_t s)
   for (long long it = 0;; it += K) {
     for (int k = 0; k < K; ++k) {
       if (g) e = hipGraphLaunch(g, s);
-      else with_engine(c->prec, c->variant, c->log2n, [&](auto eng) { decltype(eng)::attempt(L, tb, s); });
+      else with_engine(c->prec, c->variant, c->log2n, [&](auto eng) { decltype(eng)::attempt(L, tb, store, s); });
       if (e == hipSuccess) e = hipGetLastError();
       if (e != hipSuccess) return e;
     }
@@ -249,7 +250,7 @@ hipError_t rks2_run(rks2_ctx* c, const rks_tableau& tb, int mode, hipStream_t s)
 
 void rks2_destroy(rks2_ctx* c) {
   if (!c) return;
-  for (int i = 0; i < 2; ++i) {
+  for (int i = 0; i < 3; ++i) {
     if (c->exec[i]) (void)hipGraphExecDestroy(c->exec[i]);
     if (c->graph[i]) (void)hipGraphDestroy(c->graph[i]);
   }

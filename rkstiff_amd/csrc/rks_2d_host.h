@@ -38,6 +38,7 @@ int rks2_create(rks2_ctx** out, int prec, int variant, int log2n, int ninst, con
                 rks_inst* d_inst, const rks_io* d_io, const void* d_tw, size_t off_cand0, size_t off_cand1,
                 size_t off_coef, size_t off_T);
 // One launch set: mode RKS_MODE_EVOLVE / RKS_MODE_STEP (attempts until every
-// trajectory has finished) or RKS_MODE_NL.  Synchronises `stream`.
-hipError_t rks2_run(rks2_ctx* c, const rks_tableau& tab, int mode, hipStream_t stream);
+// trajectory has finished) or RKS_MODE_NL; store: trajectories keep snapshots.
+// Synchronises `stream`.
+hipError_t rks2_run(rks2_ctx* c, const rks_tableau& tab, int mode, bool store, hipStream_t stream);
 void rks2_destroy(rks2_ctx* c);

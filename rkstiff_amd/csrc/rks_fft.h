@@ -1,13 +1,10 @@
-// LDS-resident Stockham FFT for one workgroup.
-//
-// The transform of P = 2^k complex points lives in LDS (natural order in and
-// out).  Each pass (NS, RAD) is done by all T threads: a thread loads the
-// RAD*NB elements of its NB butterflies into registers, the workgroup
-// synchronises, then each butterfly is twiddled, transformed in registers and
-// written back in Stockham autosort order:
-//   read  buf[j + r*P/RAD]                          (r < RAD, j < P/RAD)
+// Stockham FFT of P = 2^k complex points by T threads of one workgroup, the elements in
+// registers and exchanged through LDS between its passes.  Pass (NS, RAD): a thread
+// twiddles and transforms its E / RAD butterflies, then writes them in Stockham autosort
+// order, and the next pass's come from there:
+//   inputs  element j + r*P/RAD                     (r < RAD, j < P/RAD)
 //   twiddle by W_{NS*RAD}^{r*(j mod NS)}
-//   write buf[(j/NS)*NS*RAD + (j mod NS) + r*NS]
+//   outputs element (j/NS)*NS*RAD + (j mod NS) + r*NS
 // Layout and twiddles:
 //   * element x lives at LDS index pad(x) = x + x/16: one spare element every
 //     16 makes the stride-RAD writes of the first pass and all later passes
@@ -151,34 +148,6 @@ __device__ __forceinline__ void apply_twiddles(cx<R> (&v)[RAD], const cx<R>* twl
   }
 }
 
-// One Stockham pass.  Twiddle W_{NS*RAD}^{r k} = W_N^{r k (P/(NS RAD)) TSCALE}, where
-// TSCALE = N / P maps a P-point transform onto the N-point table.
-// t: the thread's index among the T threads working on this transform.
-template <typename R, int P, int T, int NS, int RAD, bool INV, int LOG2N, int TSCALE>
-__device__ __forceinline__ void pass(cx<R>* buf, const cx<R>* twl, int t) {
-  constexpr int NB = P / (RAD * T);
-  static_assert(NB >= 1, "too few elements per thread");
-  cx<R> v[NB][RAD];
-#pragma unroll
-  for (int b = 0; b < NB; ++b) {
-    const int j = t + b * T;
-#pragma unroll
-    for (int r = 0; r < RAD; ++r) v[b][r] = buf[pad(j + r * (P / RAD))];
-  }
-  __syncthreads();
-#pragma unroll
-  for (int b = 0; b < NB; ++b) {
-    const int j = t + b * T;
-    const int k = j & (NS - 1);
-    if (NS > 1) apply_twiddles<RAD, INV, LOG2N>(v[b], twl, k * (P / (NS * RAD)) * TSCALE);
-    dft_small<RAD, INV>(v[b]);
-    const int base = (j - k) * RAD + k;
-#pragma unroll
-    for (int r = 0; r < RAD; ++r) buf[pad(base + r * NS)] = v[b][r];
-  }
-  __syncthreads();
-}
-
 // Register-resident transform: v[k] holds element t + k T (k < E = P / T) on entry
 // and on exit, for every radix sequence, because both the first pass's inputs
 // j + r P / RAD and the last pass's outputs j + r NS (NS = P / RAD) of the
@@ -258,19 +227,7 @@ constexpr int exchanges() {
   return n - 1;
 }
 
-template <typename R, int P, int T, int NS, bool INV, int LOG2N, int TSCALE, int MAXR>
-__device__ __forceinline__ void chain(cx<R>* buf, const cx<R>* twl, int t) {
-  if constexpr (NS < P) {
-    constexpr int E = P / T;
-    constexpr int R0 = pick_radix<E, MAXR>::v;
-    constexpr int REM = P / NS;
-    constexpr int RAD = (R0 <= REM) ? R0 : REM;
-    pass<R, P, T, NS, RAD, INV, LOG2N, TSCALE>(buf, twl, t);
-    chain<R, P, T, NS * RAD, INV, LOG2N, TSCALE, MAXR>(buf, twl, t);
-  }
-}
-
-// Full P-point register-resident transform (chain_reg).  The buffers are free when it
+// Full P-point register-resident transform (chain_reg) by the threads t.  The buffers are free when it
 // is called.  Without PP they are free again when it returns; with PP the buffer of the
 // last exchange, (BUF + exchanges - 1) % 2, may still be read by other threads.
 template <typename R, int P, int T, bool INV, int LOG2N, int MAXR, bool PP, int BUF, bool FENCE, typename Post>
@@ -278,17 +235,6 @@ __device__ __forceinline__ void fft_reg(cx<R> (&v)[P / T], cx<R>* buf, const cx<
   static_assert((P & (P - 1)) == 0, "power of two");
   static_assert(P / T >= 2, "need at least two elements per thread");
   chain_reg<R, P, T, 1, INV, LOG2N, (1 << LOG2N) / P, MAXR, PP, BUF, FENCE>(v, buf, twl, t, post);
-}
-
-// G independent P-point transforms by one workgroup of G*TG threads: threads
-// [g*TG, (g+1)*TG) transform the padded buffer buf + g*padded_size(P).  Every
-// pass synchronises the whole workgroup, so all threads must call this.
-template <typename R, int P, int TG, int G, bool INV, int LOG2N, int MAXR = 32>
-__device__ __forceinline__ void fft_multi(cx<R>* buf, const cx<R>* twl) {
-  static_assert((P & (P - 1)) == 0, "power of two");
-  static_assert(P / TG >= 2, "need at least two elements per thread");
-  const int g = threadIdx.x / TG;
-  chain<R, P, TG, 1, INV, LOG2N, (1 << LOG2N) / P, MAXR>(buf + g * padded_size(P), twl, threadIdx.x % TG);
 }
 
 }  // namespace rksfft

@@ -730,7 +730,7 @@ static int bucket_tile(const rks_plan* p, size_t b) {
 
 static int launch_all(rks_plan* p, int mode, double h_mode, hipStream_t stream) {
   if (p->c2) {
-    const hipError_t e = rks2_run(p->c2, p->tab, mode, stream);
+    const hipError_t e = rks2_run(p->c2, p->tab, mode, p->store_freq > 0, stream);
     if (e != hipSuccess) return fail(RKS_ERR_HIP, std::string("2-D engine: ") + hipGetErrorString(e));
     return RKS_OK;
   }

@@ -216,19 +216,20 @@ __host__ __device__ constexpr int rks_sum_chunk() {
   return sizeof(R) == 4 ? 8 : 4;
 }
 
-// Argument of stage s (uniform).  KEEP: the NL values of the stage before are in nv.
-template <typename TT, int S, bool KEEP, typename RS, typename RN, int MPT, typename OW, typename SlotF>
+// Argument of stage s (uniform), CH modes at a time (0: rks_sum_chunk).  KEEP: the NL values
+// of the stage before are in nv.
+template <typename TT, int S, bool KEEP, int CH = 0, typename RS, typename RN, int MPT, typename OW, typename SlotF>
 __device__ __forceinline__ void stage_switch(int s, cx<RS> (&acc)[MPT], const cx<RN> (&nv)[MPT], const cx<RS>* u,
                                              const OW& ow, SlotF slotp, const char* cbase, size_t Mc, double h) {
   constexpr int LAST = TT::tab.nstage - (TT::tab.st[TT::tab.nstage - 1].has_nl ? 1 : 2);
   constexpr int NEW = (KEEP && S > 0) ? TT::tab.st[S > 0 ? S - 1 : 0].nl_slot : -1;
   if constexpr (S < LAST) {
     if (s != S) {
-      stage_switch<TT, S + 1, KEEP>(s, acc, nv, u, ow, slotp, cbase, Mc, h);
+      stage_switch<TT, S + 1, KEEP, CH>(s, acc, nv, u, ow, slotp, cbase, Mc, h);
       return;
     }
   }
-  stage_sum<TT, S, NEW, 0, rks_sum_chunk<RS>()>(acc, nv, u, ow, slotp, cbase, Mc, h);
+  stage_sum<TT, S, NEW, 0, CH != 0 ? CH : rks_sum_chunk<RS>()>(acc, nv, u, ow, slotp, cbase, Mc, h);
 }
 
 // embedded error estimate at slots K0 .. K0 + CH - 1
