@@ -197,14 +197,8 @@ def tableau(method):
 
 
 def ptr_array(ptrs):
-    arr = (ctypes.c_void_p * len(ptrs))()
-    for i, p in enumerate(ptrs):
-        arr[i] = p
-    return arr
+    return (ctypes.c_void_p * len(ptrs))(*ptrs)
 
 
 def dbl_array(vals):
-    arr = (ctypes.c_double * len(vals))()
-    for i, v in enumerate(vals):
-        arr[i] = float(v)
-    return arr
+    return (ctypes.c_double * len(vals))(*vals)

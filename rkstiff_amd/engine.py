@@ -14,6 +14,8 @@ from .config import ETDConfig, SolverConfig
 
 STATUS_NAMES = {0: "OK", 3: "MAXLOOPS", 4: "MINSTEP", 5: "PAUSED", 6: "RUNNING"}
 
+_STATS = np.dtype(_lib.Stats)
+
 
 def _stream():
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
@@ -159,8 +161,6 @@ class Plan:
         _lib.check(self.lib.rks_plan_buckets(self.h, ctypes.byref(nb), l2, cnt, mx, nt, cap))
         return [(l2[b], cnt[b], mx[b], nt[b]) for b in range(nb.value)]
 
-    def set_launch(self, concurrent=True, wg_per_cu=None, tile=None):
-        def arr(v):
     def tiles(self):
         """The FFT tile each size bucket runs on: as set by ``set_launch``, else by size,
         precision and number of trajectories (rks_plan_set_launch)."""
@@ -169,6 +169,8 @@ class Plan:
         _lib.check(self.lib.rks_plan_tiles(self.h, arr, nb))
         return list(arr[:nb])
 
+    def set_launch(self, concurrent=True, wg_per_cu=None, tile=None):
+        def arr(v):
             return None if v is None else (ctypes.c_int * len(v))(*[int(x) for x in v])
         n = len(wg_per_cu) if wg_per_cu is not None else (len(tile) if tile is not None else 0)
         _lib.check(self.lib.rks_plan_set_launch(self.h, 1 if concurrent else 0, arr(wg_per_cu), arr(tile), n))
@@ -186,11 +188,12 @@ class Plan:
 
     # -- launches --------------------------------------------------------------
     def _check_state(self, tensors):
+        dtype, modes = self.dtype, self.modes
         for i, t in enumerate(tensors):
-            if t.dtype != self.dtype or not t.is_cuda or not t.is_contiguous():
-                raise ValueError(f"state {i}: expected contiguous {self.dtype} on the device")
-            if t.numel() != self.modes[i]:
-                raise ValueError(f"state {i}: expected {self.modes[i]} modes, got {t.numel()}")
+            if t.dtype is not dtype or not t.is_cuda or not t.is_contiguous():
+                raise ValueError(f"state {i}: expected contiguous {dtype} on the device")
+            if t.numel() != modes[i]:
+                raise ValueError(f"state {i}: expected {modes[i]} modes, got {t.numel()}")
 
     def evolve(self, u0, uf, t0, tf, h):
         self._check_state(u0)
@@ -244,7 +247,8 @@ class Plan:
     def stats(self):
         arr = (_lib.Stats * self.ninst)()
         _lib.check(self.lib.rks_get_stats(self.h, arr, _stream()))
-        return [{f: getattr(a, f) for f, _ in _lib.Stats._fields_} for a in arr]
+        names = [f for f, _ in _lib.Stats._fields_]
+        return [dict(zip(names, row)) for row in np.frombuffer(arr, dtype=_STATS).tolist()]
 
     def attempt_log(self, inst, count):
         count = min(count, self.storage[2])
