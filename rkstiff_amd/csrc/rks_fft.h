@@ -157,7 +157,8 @@ __device__ __forceinline__ void apply_twiddles(cx<R> (&v)[RAD], const cx<R>* twl
 // LDS-to-LDS form exchanges p times and is filled and drained once more.
 // PP: two buffers (buf and, padded_size(2^LOG2N) further, the other) used in turn, so an
 // exchange takes one barrier instead of two; BUF is the one that the next exchange writes.
-// post(x): applied to each output.
+// post(x): applied to each output.  on: the thread takes part (every thread calls, for the
+// barriers).
 //
 // Which product of a sum of two the compiler fuses hangs on the order in which it sees the
 // operands, and on which loads it finds equal.  leaf() makes the first pass's inputs opaque
@@ -171,7 +172,8 @@ __device__ __forceinline__ void leaf(cx<R>& v) {
 }
 
 template <typename R, int P, int T, int NS, bool INV, int LOG2N, int TSCALE, int MAXR, bool PP, int BUF, bool FENCE, typename Post>
-__device__ __forceinline__ void chain_reg(cx<R> (&v)[P / T], cx<R>* buf, const cx<R>* twl, int t, Post post) {
+__device__ __forceinline__ void chain_reg(cx<R> (&v)[P / T], cx<R>* buf, const cx<R>* twl, int t, Post post,
+                                          bool on = true) {
   constexpr int E = P / T;
   constexpr int R0 = pick_radix<E, MAXR>::v;
   constexpr int REM = P / NS;
@@ -181,37 +183,41 @@ __device__ __forceinline__ void chain_reg(cx<R> (&v)[P / T], cx<R>* buf, const c
   constexpr int PREV = PP ? 1 - BUF : 0;  // the buffer of the exchange before this pass
   constexpr int BS = padded_size(1 << LOG2N);
   cx<R> w[NB][RAD];
+  if (on) {
 #pragma unroll
-  for (int b = 0; b < NB; ++b) {
-    const int j = t + b * T;
+    for (int b = 0; b < NB; ++b) {
+      const int j = t + b * T;
 #pragma unroll
-    for (int r = 0; r < RAD; ++r) {
-      if constexpr (NS == 1) {
-        w[b][r] = v[b + r * NB];
-        leaf(w[b][r]);
-      } else {
-        w[b][r] = buf[PREV * BS + pad(j + r * (P / RAD))];
+      for (int r = 0; r < RAD; ++r) {
+        if constexpr (NS == 1) {
+          w[b][r] = v[b + r * NB];
+          leaf(w[b][r]);
+        } else {
+          w[b][r] = buf[PREV * BS + pad(j + r * (P / RAD))];
+        }
       }
     }
   }
   if constexpr (NS > 1 && !PP) __syncthreads();
+  if (on) {
 #pragma unroll
-  for (int b = 0; b < NB; ++b) {
-    const int j = t + b * T;
-    const int k = j & (NS - 1);
-    if constexpr (NS > 1) apply_twiddles<RAD, INV, LOG2N>(w[b], twl, k * (P / (NS * RAD)) * TSCALE);
-    dft_small<RAD, INV>(w[b]);
-    const int base = (j - k) * RAD + k;
+    for (int b = 0; b < NB; ++b) {
+      const int j = t + b * T;
+      const int k = j & (NS - 1);
+      if constexpr (NS > 1) apply_twiddles<RAD, INV, LOG2N>(w[b], twl, k * (P / (NS * RAD)) * TSCALE);
+      dft_small<RAD, INV>(w[b]);
+      const int base = (j - k) * RAD + k;
 #pragma unroll
-    for (int r = 0; r < RAD; ++r) {
-      if constexpr (LAST) v[b + r * NB] = post(w[b][r]);
-      else buf[(PP ? BUF : 0) * BS + pad(base + r * NS)] = w[b][r];
+      for (int r = 0; r < RAD; ++r) {
+        if constexpr (LAST) v[b + r * NB] = post(w[b][r]);
+        else buf[(PP ? BUF : 0) * BS + pad(base + r * NS)] = w[b][r];
+      }
+      if constexpr (LAST && FENCE && NB > 1) asm volatile("" ::: "memory");
     }
-    if constexpr (LAST && FENCE && NB > 1) asm volatile("" ::: "memory");
   }
   if constexpr (!LAST) {
     __syncthreads();
-    chain_reg<R, P, T, NS * RAD, INV, LOG2N, TSCALE, MAXR, PP, PP ? 1 - BUF : 0, FENCE>(v, buf, twl, t, post);
+    chain_reg<R, P, T, NS * RAD, INV, LOG2N, TSCALE, MAXR, PP, PP ? 1 - BUF : 0, FENCE>(v, buf, twl, t, post, on);
   }
 }
 
@@ -231,10 +237,11 @@ constexpr int exchanges() {
 // is called.  Without PP they are free again when it returns; with PP the buffer of the
 // last exchange, (BUF + exchanges - 1) % 2, may still be read by other threads.
 template <typename R, int P, int T, bool INV, int LOG2N, int MAXR, bool PP, int BUF, bool FENCE, typename Post>
-__device__ __forceinline__ void fft_reg(cx<R> (&v)[P / T], cx<R>* buf, const cx<R>* twl, int t, Post post) {
+__device__ __forceinline__ void fft_reg(cx<R> (&v)[P / T], cx<R>* buf, const cx<R>* twl, int t, Post post,
+                                        bool on = true) {
   static_assert((P & (P - 1)) == 0, "power of two");
   static_assert(P / T >= 2, "need at least two elements per thread");
-  chain_reg<R, P, T, 1, INV, LOG2N, (1 << LOG2N) / P, MAXR, PP, BUF, FENCE>(v, buf, twl, t, post);
+  chain_reg<R, P, T, 1, INV, LOG2N, (1 << LOG2N) / P, MAXR, PP, BUF, FENCE>(v, buf, twl, t, post, on);
 }
 
 }  // namespace rksfft

@@ -213,7 +213,7 @@ bool lookup(int prec, int nlk, int variant, int log2n, bool learn, KernelEntry* 
 //                n = 4096  x 1   7.60 / 5.65 / 7.09      x 256  19.1 / 14.5 / 15.3
 //                n = 8192  x 1  12.04 / 12.77            x 256  30.2 / 27.0
 //   advect IF34  n = 512   x 1   1.85 / 1.60             x 256   2.8 / 2.5
-//                n = 1024  x 1   3.28 / 2.32 / 2.16      x 256   4.0 / 3.1 / 2.9
+//                n = 1024  x 1   3.28 / 2.26 / 2.03      x 256   4.0 / 3.0 / 2.8
 //                n = 2048  x 1   4.08 / 2.80 / 3.06      x 256   6.1 / 4.0 / 4.1
 //                n = 4096  x 1   4.93 / 3.94 / 6.24      x 256   8.2 / 5.8 / 8.9
 //                n = 8192  x 1   7.91 / 9.71             x 256  12.7 / 16.7
