@@ -742,9 +742,32 @@ static int launch_all(rks_plan* p, int mode, double h_mode, hipStream_t stream) 
   L.io = p->d_io;
   L.mode = mode;
   L.h_mode = h_mode;
-  hipLaunchKernelGGL(rks_zero_int, dim3(1), dim3(64), 0, stream, p->d_queue, 64);
-  HIPCHK(hipGetLastError());
   const size_t nb = p->bucket_log2.size();
+  const bool learn = p->mlp.on || p->d_rec != nullptr;
+  std::vector<KernelEntry> kern(nb);
+  std::vector<int> grid(nb);
+  bool queued = false;
+  for (size_t b = 0; b < nb; ++b) {
+    KernelEntry& e = kern[b];
+    if (!lookup(p->prec, p->nlk, p->variant, p->bucket_log2[b], learn, &e, bucket_tile(p, b)))
+      return fail(RKS_ERR_INVALID, "no kernel for this grid size, variant and tile");
+    grid[b] = p->bucket_count[b];
+    if (grid[b] <= p->cu) continue;  // a CU holds at least one workgroup
+    int per_cu = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, e.fn, e.threads, e.lds) != hipSuccess || per_cu < 1)
+      per_cu = 1;
+    if (b < p->wg_per_cu.size() && p->wg_per_cu[b] > 0 && p->wg_per_cu[b] < per_cu) per_cu = p->wg_per_cu[b];
+    if (grid[b] > per_cu * p->cu) {
+      grid[b] = per_cu * p->cu;
+      queued = true;
+    }
+  }
+  // the queue's counters, where a launch has more trajectories than workgroups: a launch of its
+  // own, 3 us of a single step (62 -> 59)
+  if (queued) {
+    hipLaunchKernelGGL(rks_zero_int, dim3(1), dim3(64), 0, stream, p->d_queue, 64);
+    HIPCHK(hipGetLastError());
+  }
   const bool conc = p->concurrent && nb > 1;
   if (conc) {
     // fork: every bucket stream waits for the caller's stream (queue counters cleared)
@@ -763,28 +786,18 @@ static int launch_all(rks_plan* p, int mode, double h_mode, hipStream_t stream) 
     HIPCHK(hipEventRecord(p->fork, stream));
   }
   for (size_t b = 0; b < nb; ++b) {
-    KernelEntry e;
-    const bool learn = p->mlp.on || p->d_rec != nullptr;
-    const int ti = bucket_tile(p, b);
-    if (!lookup(p->prec, p->nlk, p->variant, p->bucket_log2[b], learn, &e, ti))
-      return fail(RKS_ERR_INVALID, "no kernel for this grid size, variant and tile");
+    const KernelEntry& e = kern[b];
     L.order = p->d_order + p->bucket_start[b];
     L.count = p->bucket_count[b];
-    L.queue = p->d_queue + b;
+    L.queue = grid[b] < L.count ? p->d_queue + b : nullptr;
     L.tw = p->d_tw[p->bucket_log2[b]];
-    int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, e.fn, e.threads, e.lds) != hipSuccess || per_cu < 1)
-      per_cu = 1;
-    if (b < p->wg_per_cu.size() && p->wg_per_cu[b] > 0 && p->wg_per_cu[b] < per_cu) per_cu = p->wg_per_cu[b];
-    int grid = per_cu * p->cu;
-    if (grid > L.count) grid = L.count;
     void* args[] = {&L};
     hipStream_t st = stream;
     if (conc) {
       st = p->bstream[b];
       HIPCHK(hipStreamWaitEvent(st, p->fork, 0));
     }
-    HIPCHK(hipLaunchKernel(e.fn, dim3(grid), dim3(e.threads), args, (size_t)e.lds, st));
+    HIPCHK(hipLaunchKernel(e.fn, dim3(grid[b]), dim3(e.threads), args, (size_t)e.lds, st));
     if (conc) HIPCHK(hipEventRecord(p->bdone[b], st));
   }
   // join after every bucket is queued: a wait on the caller's stream is a

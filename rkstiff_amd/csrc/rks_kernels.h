@@ -44,7 +44,7 @@ struct rks_launch {
   const int* order;
   int count;
   int mode;
-  int* queue;
+  int* queue;      // next item, or null where the grid has a workgroup per trajectory
   const void* tw;  // exp(-2 pi i x / N), x < N, engine precision
   double h_mode;   // RKS_MODE_COEFFS
   rks_mlp_dev mlp; // learned step-size proposer (mlp.on = 0: the reference's controller only)
@@ -1746,11 +1746,14 @@ __global__ __launch_bounds__(rks_threads(LOG2N, NLK) << TILE, rks_min_waves(LOG2
   cx<R>* twl = buf + rks_buf_elems<R, LOG2N, T, NLK>();
   float* scr = kScrInBuf ? (float*)rks_smem : s_scr;
   if constexpr (NLK != NLK_HANKEL) rksfft::load_twiddles<R, LOG2N, T>(twl, (const cx<R>*)P.tw);
-  for (;;) {
-    if (threadIdx.x == 0) s_item = atomicAdd(P.queue, 1);
-    __syncthreads();
-    const int item = uni(s_item);
-    __syncthreads();
+  for (bool first = true;; first = false) {
+    int item = first ? (int)blockIdx.x : P.count;  // without a queue: a workgroup per trajectory
+    if (P.queue != nullptr) {
+      if (threadIdx.x == 0) s_item = atomicAdd(P.queue, 1);
+      __syncthreads();
+      item = uni(s_item);
+      __syncthreads();
+    }
     if (item >= P.count) break;
     const int idx = uni(P.order[item]);
     if constexpr (LEARN && T >= 64) {
