@@ -57,20 +57,23 @@ struct Eng2 {
   static void out(const rks2_launch& L, hipStream_t s) {
     hipLaunchKernelGGL((k2_out<R, LOG2>), dim3(copy_blocks(), L.ninst), dim3(256), 0, s, L);
   }
-  // one attempt of every running trajectory (store: one may keep snapshots)
-  static void attempt(const rks2_launch& L, const rks_tableau& tb, bool store, hipStream_t s) {
+  // one attempt of every running trajectory (nl1: one may need NL1 = nl(u) first; store: one
+  // may keep snapshots)
+  static void attempt(const rks2_launch& L, const rks_tableau& tb, bool nl1, bool store, hipStream_t s) {
     // a mode per thread until there are 8 workgroups for every CU, then several
     const int one = (G::M + 255) / 256, cap = 2048 / L.ninst > one / 8 ? 2048 / L.ninst : one / 8 + 1;
     hipLaunchKernelGGL((k2_coef<R, RN, LOG2, METH>), dim3(one < cap ? one : cap, L.ninst), dim3(256), 0, s, L);
     // NL1 = nl(u) where needed (start; after an accept for RECOMPUTE methods)
-    col(L, s, -1, 0, -1, 1);
-    row(L, s, 1);
+    if (nl1) {
+      col(L, s, -1, 0, -1, 1);
+      row(L, s, 1);
+    }
     // the last stage forms the error estimate with the candidate where the method allows
     const bool fused = rks_fused_final(tb);
     for (int k = 0; k < tb.nstage; ++k) {
       int fwd = -1, cond = 0;
       if (k == 0) {
-        fwd = 0;
+        fwd = nl1 ? 0 : -1;
         cond = 1;
       } else if (tb.st[k - 1].has_nl) {
         fwd = tb.st[k - 1].nl_slot;
@@ -180,7 +183,12 @@ int rks2_create(rks2_ctx** out, int prec, int variant, int log2n, int ninst, con
   return 0;
 }
 
-// the attempt sequence of `mode`, captured once
+// Whether an attempt after the first of a launch can need NL1 anew: only where the method
+// recomputes it.  The others (FSAL: IF34, ETD34) take it from a slot, and two launches of each
+// attempt would start only to find nothing to do.
+static bool rks2_nl1_again(const rks_tableau& tb) { return tb.nl1_policy == RKS_NL1_RECOMPUTE; }
+
+// the attempt sequence of `mode` (after the first of a launch), captured once
 static hipGraphExec_t attempt_graph(rks2_ctx* c, const rks_tableau& tb, int mode, bool store) {
   const int gi = mode != RKS_MODE_EVOLVE ? 1 : (store ? 2 : 0);
   if (c->exec[gi] || !c->use_graph) return c->exec[gi];
@@ -194,7 +202,7 @@ static hipGraphExec_t attempt_graph(rks2_ctx* c, const rks_tableau& tb, int mode
     c->use_graph = false;
     return nullptr;
   }
-  with_engine(c->prec, c->variant, c->log2n, [&](auto eng) { decltype(eng)::attempt(L, tb, store, c->cap); });
+  with_engine(c->prec, c->variant, c->log2n, [&](auto eng) { decltype(eng)::attempt(L, tb, rks2_nl1_again(tb), store, c->cap); });
   hipGraph_t g = nullptr;
   if (hipStreamEndCapture(c->cap, &g) != hipSuccess || !g) {
     c->use_graph = false;
@@ -233,8 +241,9 @@ hipError_t rks2_run(rks2_ctx* c, const rks_tableau& tb, int mode, bool store, hi
   const int K = 4;  // attempts between completion checks
   for (long long it = 0;; it += K) {
     for (int k = 0; k < K; ++k) {
-      if (g) e = hipGraphLaunch(g, s);
-      else with_engine(c->prec, c->variant, c->log2n, [&](auto eng) { decltype(eng)::attempt(L, tb, store, s); });
+      const bool nl1 = (it == 0 && k == 0) || rks2_nl1_again(tb);
+      if (g && nl1 == rks2_nl1_again(tb)) e = hipGraphLaunch(g, s);
+      else with_engine(c->prec, c->variant, c->log2n, [&](auto eng) { decltype(eng)::attempt(L, tb, nl1, store, s); });
       if (e == hipSuccess) e = hipGetLastError();
       if (e != hipSuccess) return e;
     }
