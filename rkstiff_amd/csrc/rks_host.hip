@@ -108,16 +108,19 @@ __global__ void rks_transpose(const double* a, R* b, int n) {
     b[i] = (R)a[(i % n) * n + i / n];
 }
 
-// Per log2 n, the advective trajectories whose last mode is not damped at DAMPED times the rate at which a
-// field of unit size is advected across it (-Re L >= DAMPED |coef| k).
+// Whether the last mode is damped at DAMPED times the rate at which a field of unit size is
+// advected across it: -Re L >= DAMPED |coef| k.
 constexpr double DAMPED = 100.0;
+__host__ __device__ inline bool rks_damped(double re, double coef, double k) { return -re >= DAMPED * fabs(coef) * k; }
+
+// Per log2 n, the advective trajectories whose last mode is not.
 __global__ void rks_count_undamped(const rks_inst* inst, int ninst, int* count) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= ninst) return;
   const rks_inst& r = inst[i];
   const int m = r.m - 1;
-  const double re = r.L_complex ? r.L[2 * m] : r.L[m];
-  if (!(-re >= DAMPED * fabs(r.nl_coef) * ((const double*)r.kx)[m])) atomicAdd(&count[32 - __clz(m)], 1);
+  if (!rks_damped(r.L_complex ? r.L[2 * m] : r.L[m], r.nl_coef, ((const double*)r.kx)[m]))
+    atomicAdd(&count[32 - __clz(m)], 1);
 }
 
 // ===========================================================================
@@ -220,7 +223,7 @@ bool lookup(int prec, int nlk, int variant, int log2n, bool learn, KernelEntry* 
 // FP32 and MIXED runs gain as much, but keep the base tile: a tile has its own order of
 // rounding, and in FP32 storage that moves the step sizes and with them the results (MIXED
 // soliton ensembles by 4e-9, FP32 KS by 3e-6), so there the caller chooses.  Likewise an
-// advective term on a grid whose last modes are not damped (rks_count_undamped): a spectrum
+// advective term on a grid whose last modes are not damped (rks_damped): a spectrum
 // that reaches the grid's end amplifies rounding (viscosity 5e-4, n = 4096: 2e-3 of the
 // state; KS: 1e-13).  The proposer
 // counts accepted steps by the workgroup's size, so its kernels keep the base tile; so do
@@ -602,7 +605,16 @@ int rks_plan_create(int method, int nl_kind, int precision, const rks_config* cf
     }
     HIPCHK(hipMemcpy(p->d_order, p->order.data(), sizeof(int) * ninst, hipMemcpyHostToDevice));
     p->undamped.assign(14, 0);
-    if (nl_kind == RKS_NL_ADVECT_RFFT && precision == RKS_F64) {
+    if (nl_kind == RKS_NL_ADVECT_RFFT && precision == RKS_F64 && ninst <= 4) {
+      // a few: from the caller's arrays, without a launch and a read back
+      for (int i = 0; i < ninst; ++i) {
+        const int m = p->modes[i] - 1;
+        double re = 0.0, k = 0.0;
+        HIPCHK(hipMemcpy(&re, (const double*)desc[i].L + (desc[i].L_is_complex ? 2 * m : m), sizeof(double), hipMemcpyDefault));
+        HIPCHK(hipMemcpy(&k, (const double*)desc[i].kx + m, sizeof(double), hipMemcpyDefault));
+        p->undamped[ilog2(desc[i].n)] += !rks_damped(re, desc[i].nl_coef, k);
+      }
+    } else if (nl_kind == RKS_NL_ADVECT_RFFT && precision == RKS_F64) {
       hipLaunchKernelGGL(rks_zero_int, dim3(1), dim3(64), 0, 0, p->d_queue, 64);
       hipLaunchKernelGGL(rks_count_undamped, dim3((ninst + 255) / 256), dim3(256), 0, 0, p->d_inst, ninst, p->d_queue);
       HIPCHK(hipGetLastError());

@@ -6,7 +6,7 @@
 // (add_terms, coef_update in rks_kernels.h), each term is a run of uniform branches with
 // its own wait, about 90 dependent round trips per n = 8192 ETD35 attempt, and the
 // allocator spills around them (1104 bytes of scratch per lane in FP64).  Only the methods
-// and storage kinds that the workloads run are compiled this way: rks_method_kernel.
+// and storage kinds that the workloads run are compiled this way (method_variant, rks_host.hip).
 #pragma once
 #include <utility>
 
@@ -251,7 +251,8 @@ __device__ __forceinline__ void error_sum(cx<RS> (&ev)[CH], const cx<RN> (&nv)[M
 
 // Last stage and error estimate, then the values of the masked norm per mode (FP64): |u_new|
 // and |err|^2 where the last stage has no NL (FP32: |u_new| and |err|, rounded to FP32; a
-// square would flush to zero below ~1e-19), else |u_new|^2 and |err|^2.  A method whose last stage has no NL (ETD35) forms both from the same NL values;
+// square would flush to zero below ~1e-19), else |u_new|^2 and |err|^2.  A method whose last
+// stage has no NL (ETD35) forms both from the same NL values;
 // LAST_NL: the candidate is already stored (it went through the last NL evaluation).
 template <typename TT, int NEW, int K0, int CHMAX, bool LAST_NL, typename RS, typename RN, int MPT, typename OW,
           typename SlotF>
