@@ -6,9 +6,9 @@
 //   * coefficient arrays are regenerated in FP64 when h changes
 //     (exact compare, etd35.py:851-852), stored in engine precision;
 //   * every stage is one pass over the modes: k = E u + sum C NL is formed in
-//     registers and written straight into the LDS FFT buffer, the nonlinear
-//     term is evaluated in LDS (inverse FFT, pointwise product, forward FFT)
-//     and the new NL array is written once;
+//     registers, the nonlinear term takes it from there (inverse FFT, pointwise
+//     product, forward FFT, exchanging through LDS) and the new NL array is
+//     written once;
 //   * the embedded error norm (solveras.py:449-455) is a workgroup reduction
 //     accumulated in FP64, and the accept/reject dt controller
 //     (solveras.py:457-554) runs in FP64 on the device.
@@ -873,8 +873,9 @@ __host__ __device__ constexpr int rks_lds_bytes() {
 // the 8 nr^2 bytes of yt per product that each trajectory streams from L2 (80 KB at nr = 100,
 // beyond the L1), with a thread per row so that all of a row's latency is spent once.  1024
 // beams, nr = 100, ETD35 FP64, one evolve: 21.2 ms row by row with n/4 threads, 8.6 ms.
-// Arithmetic as the batched transform (rks_hankel.hip): f = (1/S) sum, |f|^2 f, then
-// i gamma (S sum).
+// Values as the batched transform's (rks_hankel.hip): f = (1/S) sum, |f|^2 f, then
+// i gamma (S sum).  Batches of 10 columns: 16 (7.6 -> 8.9 ms) and 32 (9.6) were slower, also
+// with the next batch prefetched (9.6).
 template <typename R, int LOG2N, int T, int MPT>
 __device__ __forceinline__ void hankel_rows(cx<R> (&v)[MPT], const cx<R>* x, const R* __restrict__ yt, int nr) {
 #pragma unroll
