@@ -170,12 +170,13 @@ typedef rks_kernel_entry KernelEntry;
 
 // Which stepping kernel runs a plan: the one compiled for its method where that exists, else
 // the one that reads the tableau.  ETD35 and IF34 are the methods of every workload; their
-// kernels are compiled for the coefficient storage that goes with the nonlinearity (real
-// lin_op with the advective and the rfft2 terms, complex with the cubic ones), so a complex
-// lin_op with the advective term (KdV) or a real one with a cubic term takes the general kernel.
-int method_variant(int method, int nlk, int coef_real) {
+// kernels are compiled for lin_ops of one kind (real with the advective and the rfft2 terms,
+// complex with the cubic ones) and read every L of the plan so.  A complex lin_op with the
+// advective term (KdV), a real one with a cubic term, or a plan that holds both kinds takes the
+// general kernel, which reads each trajectory's kind.
+int method_variant(int method, int nlk, int n_complex, int ninst) {
   const bool real = nlk == RKS_NL_ADVECT_RFFT || nlk == RKS_NL_AC2D_RFFT2;
-  if (real != (coef_real != 0)) return RKS_METH_ANY;
+  if (n_complex != (real ? 0 : ninst)) return RKS_METH_ANY;
   if (method == RKS_M_ETD35) return method;
   if (method == RKS_M_IF34 && nlk != RKS_NL_HANKEL_CUBIC) return method;
   return RKS_METH_ANY;
@@ -379,11 +380,12 @@ int rks_plan_create(int method, int nl_kind, int precision, const rks_config* cf
   // contour means, whose nodes come in conjugate pairs.  The generic path (no built-in term) keeps the
   // reference's complex arrays.
   {
-    bool real = nl_kind != RKS_NL_NONE;
-    for (int i = 0; i < ninst && real; ++i) real = !desc[i].L_is_complex;
+    int n_complex = 0;
+    for (int i = 0; i < ninst; ++i) n_complex += desc[i].L_is_complex ? 1 : 0;
+    const bool real = nl_kind != RKS_NL_NONE && n_complex == 0;
     p->coef_real = real ? 1 : 0;
     p->coef_bytes_per_mode = (size_t)rks_tab::layout(p->tab, p->esize, p->nsize, real);
-    p->variant = method_variant(method, nl_kind, p->coef_real);
+    p->variant = method_variant(method, nl_kind, n_complex, ninst);
   }
   fill_ctrl(&p->ctl, cfg);
   if (cfg->contour_points < 2) {

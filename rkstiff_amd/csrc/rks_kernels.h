@@ -420,6 +420,8 @@ __device__ __forceinline__ void method_small(CT& ct, z64 z, int lane, double h, 
 
 // coef_update of one method.  The generator was bound by the tableau it walked: per mode,
 // every fraction searched the whole coefficient list and divided by run-time constants.
+// Whether L is complex is a literal (LC): the host picks these kernels only for plans whose
+// lin_ops are all of that kind.
 template <typename TT, typename RS, typename RN, int T, int MPT>
 __device__ __attribute__((noinline)) void coef_update_method(const rks_ctrl& ct_in, const double* __restrict__ L,
                                                              int M, int Mg, double h, char* __restrict__ cbase,
