@@ -205,7 +205,7 @@ class FamilyRun:
         la = self.plan.launch
         if self.tuned is None or la is None:
             return None
-        return {"concurrent_buckets": la["concurrent"], "wg_per_cu": la["wg_per_cu"], "fft_tile": la["tile"]}
+        return {"concurrent_buckets": la["concurrent"], "wg_per_cu": la["wg_per_cu"], "fft_tile": self.plan.tiles()}
 
 
 def tune_batch(runs, streams, whole=False):

@@ -165,12 +165,14 @@ int rks_error_s(rks_plan* p, int inst, const void* u_new, const void* err, doubl
  * private streams forked from and joined back to the caller's stream, so a
  * bucket's tail overlaps the others; 0 launches them in order on the caller's
  * stream.  wg_per_cu[b] (NULL: all 0) caps bucket b's resident workgroups per
- * CU, 0 = as many as fit; tile[b] picks bucket b's FFT tile (the proposer
- * variant too; NULL, as before the first call: chosen by size, precision and
- * number of trajectories, the base tile with a proposer, records or an attempt
- * log).  Results do not depend on the shape or, beyond rounding, the tile.
- * rks_plan_tiles: the tile each bucket (up to cap) runs on now: 0, 1, or 2 (four
- * times the threads). */
+ * CU, 0 = as many as fit; tile[b] picks bucket b's FFT tile: 0 the base tile, 1
+ * twice its threads (n = 512 .. 4096; without a proposer or records also the cubic
+ * n = 8192), 2 four times (n = 1024 and the cubic n = 2048, without a proposer or
+ * records; these, attached later, bring the base tile back), -1 (also tile NULL, as
+ * before the first call) the library's choice by size, precision and number of
+ * trajectories: the base tile with a proposer, records or an attempt log.  Results
+ * do not depend on the shape or, beyond rounding, the tile.
+ * rks_plan_tiles: the tile each bucket (up to cap) runs on now (0, 1 or 2). */
 int rks_plan_buckets(rks_plan* p, int* nbucket, int* log2n, int* count, int* max_wg_per_cu, int* ntile, int cap);
 int rks_plan_set_launch(rks_plan* p, int concurrent, const int* wg_per_cu, const int* tile, int nbucket);
 int rks_plan_tiles(rks_plan* p, int* tile, int cap);

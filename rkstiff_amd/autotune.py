@@ -11,7 +11,8 @@ per bucket.  Two launch choices change throughput and not results:
   trajectories share a CU's caches and LDS bandwidth with fewer others);
 * the FFT tile of each bucket where a second one exists (n = 512 .. 4096):
   twice the threads per trajectory, half the modes per thread in the stage
-  passes and transforms.
+  passes and transforms.  A bucket starts on the tile that the library
+  chooses for it (-1, ``Plan.tiles`` says which).
 
 ``tune_launch`` times short pilot evolves of the plan's own trajectories and
 keeps the fastest shape.  Finally each bucket's trajectories are ordered by
@@ -64,12 +65,18 @@ def _bucket_log2(plan, n):
     return int(n).bit_length() - 1
 
 
+def _other_tile(tile):
+    """The tile tried against ``tile``: the second one, or the base tile against that."""
+    return 0 if tile == 1 else 1
+
+
 def tune_launch(plan, u0, t0, tf, h, reps=2, min_gain=0.02):
     """Tune ``plan``'s launch shape on pilot evolves over [t0, tf] from ``u0``.
 
     u0: list of device state tensors (the plan's dtype), one per trajectory;
     t0/tf/h: scalars or per-trajectory sequences (h: first step).
-    Returns {"concurrent", "wg_per_cu", "tile", "seconds", "trials", "buckets"}.
+    Returns {"concurrent", "wg_per_cu", "tile", "seconds", "trials", "buckets"}; the first
+    three are what ``Plan.set_launch`` takes (tile -1: the library's choice).
     """
     n = plan.ninst
     t0s = np.broadcast_to(np.asarray(t0, dtype=np.float64), (n,)).tolist()
@@ -93,13 +100,14 @@ def tune_launch(plan, u0, t0, tf, h, reps=2, min_gain=0.02):
             l2 = buckets[bucket][0]
             only = [tfs[i] if inst_l2[i] == l2 else t0s[i] for i in range(n)]
             sec = _timed(plan, u0, uf, t0s, only, hs, reps)
-        trials.append({"concurrent": conc, "wg_per_cu": list(wg), "tile": plan.tiles(), "bucket": bucket,
+        trials.append({"concurrent": conc, "wg_per_cu": list(wg), "tile": list(ti), "bucket": bucket,
                        "seconds": sec})
         return sec
 
     nb = len(buckets)
-    wg0, ti0 = [0] * nb, [0] * nb
+    wg0, ti0 = [0] * nb, [-1] * nb
     default = trial(True, wg0, ti0)  # the plan's default shape
+    own = plan.tiles()
     best_wg, best_ti, whole = list(wg0), list(ti0), default
 
     def consider(b, base, wg, ti):
@@ -122,12 +130,12 @@ def tune_launch(plan, u0, t0, tf, h, reps=2, min_gain=0.02):
         base = trial(True, best_wg, best_ti, b) if nb > 1 else default
         if ntile > 1:
             ti = list(best_ti)
-            ti[b] = 1
+            ti[b] = _other_tile(own[b])
             sec = consider(b, base, best_wg, ti)
             if sec is not None:
                 base, best_ti = sec, ti
         plan.set_launch(True, best_wg, best_ti)
-        if best_ti[b] == 0:
+        if plan.tiles()[b] == 0:
             mx = plan.buckets()[b][2]
             for v in sorted({mx // 2, mx // 4} - {0, mx}, reverse=True):
                 wg = list(best_wg)
@@ -142,12 +150,7 @@ def tune_launch(plan, u0, t0, tf, h, reps=2, min_gain=0.02):
             best, best_conc = sec, False
         if not best < default:
             best, best_conc, best_wg, best_ti = default, True, list(wg0), list(ti0)
-    # the tiles the library chooses by size (wider ones than can be set per bucket among them)
-    sec = trial(best_conc, best_wg, None)
-    own = best_ti
-    if sec < best:
-        best, own, best_ti = sec, None, plan.tiles()
-    plan.set_launch(best_conc, best_wg, own)
+    plan.set_launch(best_conc, best_wg, best_ti)
     # longest first: the attempts of a pilot over the whole ensemble estimate each
     # trajectory's cost
     plan.evolve(u0, uf, t0s, tfs, hs)
@@ -187,12 +190,12 @@ def tune_together(jobs, reps=2, min_gain=0.02, warm=True, uniform=False):
     all plans).  The buckets with a second tile are flipped in turn, largest (trajectories
     x n) first over all plans, and a flip is kept when the joint launch is faster by more
     than ``min_gain``.  With ``uniform`` the flips start from the best combination of
-    each plan's own tuning, the second tile on every bucket that has one, and the first
-    tile everywhere (single flips miss combinations that only pay together: on the
+    each plan's own tuning, the library's own choice, the second tile on every bucket that has
+    one, and the first tile everywhere (single flips miss combinations that only pay together: on the
     mixed batch the KS family's second tiles gain most when the NLS family's buckets
     keep the first).  Resident-workgroup
     limits, bucket concurrency and trajectory order stay as tuned.  Returns {"tiles":
-    per-plan tiles, "seconds": the best joint launch, "trials": [...]}.
+    per-plan tiles as ``Plan.set_launch`` takes them, "seconds": the best joint launch, "trials": [...]}.
     """
     runs = []
     for plan, u0, t0, tf, h, stream in jobs:
@@ -205,26 +208,35 @@ def tune_together(jobs, reps=2, min_gain=0.02, warm=True, uniform=False):
         la = plan.launch or {}
         shapes.append({"concurrent": la.get("concurrent", True),
                        "wg": list(la.get("wg_per_cu") or [0] * nb),
-                       "tile": [min(x, b[3] - 1) for x, b in zip(plan.tiles(), plan.buckets())]})
+                       "tile": list(la.get("tile") or [-1] * nb)})
 
     def apply():
         for (plan, *_), sh in zip(runs, shapes):
             if plan.buckets():
                 plan.set_launch(sh["concurrent"], sh["wg"], sh["tile"])
 
+    def effective(plan, tile):
+        """The tiles that ``tile`` stands for (every launch below sets its own shape first)."""
+        if plan.buckets():
+            plan.set_launch(True, None, tile)
+        return plan.tiles()
+
     apply()
     best = _timed_together(runs, reps, warm)
     trials = [{"tiles": [list(sh["tile"]) for sh in shapes], "seconds": best}]
     if uniform:
-        # every combination of (own tuning, second tile everywhere, first tile everywhere)
-        # over the plans (at most three plans; more: one plan at a time)
+        # every combination of (own tuning, the library's choice, second tile everywhere, first
+        # tile everywhere) over the plans, each shape once (at most three plans; more: one plan
+        # at a time)
         opts = []
         for j, (plan, *_) in enumerate(runs):
             nt = [b[3] for b in plan.buckets()]
-            o = [list(shapes[j]["tile"])]
-            for cand in ([1 if t > 1 else 0 for t in nt], [0] * len(nt)):
-                if cand not in o:
+            o, seen = [], []
+            for cand in (list(shapes[j]["tile"]), [-1] * len(nt), [1 if t > 1 else 0 for t in nt], [0] * len(nt)):
+                runs_on = effective(plan, cand)
+                if runs_on not in seen:
                     o.append(cand)
+                    seen.append(runs_on)
             opts.append(o)
         combos = list(itertools.product(*opts)) if len(runs) <= 3 else \
             [tuple(o[k] if i == j else o[0] for i, o in enumerate(opts)) for j in range(len(opts))
@@ -247,7 +259,7 @@ def tune_together(jobs, reps=2, min_gain=0.02, warm=True, uniform=False):
              for b, (l2, cnt, _mx, ntile) in enumerate(plan.buckets()) if ntile > 1]
     for _, j, b in sorted(flips, reverse=True):
         old = shapes[j]["tile"][b]
-        shapes[j]["tile"][b] = 1 - old
+        shapes[j]["tile"][b] = _other_tile(runs[j][0].tiles()[b])
         apply()
         sec = _timed_together(runs, reps, warm)
         trials.append({"tiles": [list(sh["tile"]) for sh in shapes], "seconds": sec})

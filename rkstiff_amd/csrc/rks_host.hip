@@ -735,11 +735,18 @@ static char* inst_cbase(const rks_plan* p, int inst) {
          2 * rks_align256(M * p->esize);
 }
 
-// the tile that bucket b runs on: the caller's choice, else default_tile
+// the proposer variant runs: a proposer or training records are attached
+static bool learns(const rks_plan* p) { return p->mlp.on || p->d_rec != nullptr; }
+
+// the tile that bucket b runs on: the caller's choice (a tile without a proposer variant gives
+// way to the base tile when a proposer or records are attached after it), else default_tile
 static int bucket_tile(const rks_plan* p, size_t b) {
-  if (b < p->tile.size() && p->tile[b] >= 0) return p->tile[b];
+  if (b < p->tile.size() && p->tile[b] >= 0) {
+    KernelEntry e;
+    return lookup(p->prec, p->nlk, p->variant, p->bucket_log2[b], learns(p), &e, p->tile[b]) ? p->tile[b] : 0;
+  }
   return default_tile(p->prec, p->nlk, p->bucket_log2[b], p->bucket_count[b], p->cu,
-                      p->undamped[p->bucket_log2[b]] || p->mlp.on || p->d_rec != nullptr || p->d_log != nullptr);
+                      p->undamped[p->bucket_log2[b]] || learns(p) || p->d_log != nullptr);
 }
 
 static int launch_all(rks_plan* p, int mode, double h_mode, hipStream_t stream) {
@@ -757,7 +764,7 @@ static int launch_all(rks_plan* p, int mode, double h_mode, hipStream_t stream) 
   L.mode = mode;
   L.h_mode = h_mode;
   const size_t nb = p->bucket_log2.size();
-  const bool learn = p->mlp.on || p->d_rec != nullptr;
+  const bool learn = learns(p);
   std::vector<KernelEntry> kern(nb);
   std::vector<int> grid(nb);
   bool queued = false;
@@ -1118,7 +1125,7 @@ int rks_plan_buckets(rks_plan* p, int* nbucket, int* log2n, int* count, int* max
     if (max_wg_per_cu) {
       KernelEntry e;
       int per_cu = 0;
-      if (!lookup(p->prec, p->nlk, p->variant, p->bucket_log2[b], p->mlp.on || p->d_rec != nullptr, &e) ||
+      if (!lookup(p->prec, p->nlk, p->variant, p->bucket_log2[b], learns(p), &e) ||
           hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, e.fn, e.threads, e.lds) != hipSuccess || per_cu < 1)
         per_cu = 1;
       max_wg_per_cu[b] = per_cu;
@@ -1139,10 +1146,11 @@ int rks_plan_set_launch(rks_plan* p, int concurrent, const int* wg_per_cu, const
       w[b] = wg_per_cu[b];
     }
     if (tile) {
+      // -1: default_tile's choice; else a tile that the plan can run on as it is
       KernelEntry e1;
-      // a chosen tile must have its proposer variant, which a caller may attach later
-      if (tile[b] != 0 && !(tile[b] == 1 && lookup(p->prec, p->nlk, p->variant, p->bucket_log2[b], true, &e1, 1)))
-        return fail(RKS_ERR_INVALID, "tile 1 exists for n = 512 .. 4096 only");
+      if (tile[b] < -1 || (tile[b] > 0 && !lookup(p->prec, p->nlk, p->variant, p->bucket_log2[b], learns(p), &e1, tile[b])))
+        return fail(RKS_ERR_INVALID, "tile 1 exists for n = 512 .. 4096; without a proposer or records also tile 1 for "
+                                     "the cubic n = 8192, tile 2 for n = 1024 and the cubic n = 2048");
       ti[b] = tile[b];
     }
   }

@@ -170,6 +170,8 @@ class Plan:
         return list(arr[:nb])
 
     def set_launch(self, concurrent=True, wg_per_cu=None, tile=None):
+        """Launch shape: buckets overlapped or in order, a cap on workgroups per CU and the FFT
+        tile of each bucket (any that ``tiles`` reports; -1: the library's choice)."""
         def arr(v):
             return None if v is None else (ctypes.c_int * len(v))(*[int(x) for x in v])
         n = len(wg_per_cu) if wg_per_cu is not None else (len(tile) if tile is not None else 0)
