@@ -113,14 +113,13 @@ __global__ void rks_transpose(const double* a, R* b, int n) {
 constexpr double DAMPED = 100.0;
 __host__ __device__ inline bool rks_damped(double re, double coef, double k) { return -re >= DAMPED * fabs(coef) * k; }
 
-// Per log2 n, the advective trajectories whose last mode is not.
-__global__ void rks_count_undamped(const rks_inst* inst, int ninst, int* count) {
+// Marks the advective trajectories whose last mode is not.
+__global__ void rks_mark_undamped(const rks_inst* inst, int ninst, int* undamped) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= ninst) return;
   const rks_inst& r = inst[i];
   const int m = r.m - 1;
-  if (!rks_damped(r.L_complex ? r.L[2 * m] : r.L[m], r.nl_coef, ((const double*)r.kx)[m]))
-    atomicAdd(&count[32 - __clz(m)], 1);
+  undamped[i] = rks_damped(r.L_complex ? r.L[2 * m] : r.L[m], r.nl_coef, ((const double*)r.kx)[m]) ? 0 : 1;
 }
 
 // ===========================================================================
@@ -206,21 +205,34 @@ bool lookup(int prec, int nlk, int variant, int log2n, bool learn, KernelEntry* 
 #undef RKS_PICK
 }
 
-// Tile of a bucket of `count` trajectories whose caller chose none.  A trajectory is a serial
+// Tile of a trajectory whose caller chose none: by its size, method and precision, and not by
+// what else is in the plan, so that its FP64 result is the same alone and in a batch.  A
+// trajectory is a serial
 // chain of butterflies, exchanges and stage sums, so more waves with fewer modes each shorten
 // every link of it, until a transform takes more passes or a workgroup's registers and LDS
 // keep others off a loaded CU.  Measured per FP64 evolve, base tile / twice / four times
-// (MI355X):
+// (MI355X; another interval for x 1000, ETD34 for the methods that read their tableau):
 //   cubic ETD35  n = 512   x 1   3.49 / 2.21 ms          x 256   5.7 / 3.8 ms
-//                n = 1024  x 1   6.73 / 3.80 / 2.38      x 256  11.5 / 6.7 / 4.0
-//                n = 2048  x 1   6.68 / 4.09 / 3.24      x 256  13.2 / 7.8 / 5.3
-//                n = 4096  x 1   7.60 / 5.65 / 7.09      x 256  19.1 / 14.5 / 15.3
-//                n = 8192  x 1  12.04 / 12.77            x 256  30.2 / 27.0
-//   advect IF34  n = 512   x 1   1.85 / 1.60             x 256   2.8 / 2.5
-//                n = 1024  x 1   3.28 / 2.26 / 2.03      x 256   4.0 / 3.0 / 2.8
-//                n = 2048  x 1   4.08 / 2.80 / 3.06      x 256   6.1 / 4.0 / 4.1
-//                n = 4096  x 1   4.93 / 3.94 / 6.24      x 256   8.2 / 5.8 / 8.9
+//                n = 1024  x 1   6.73 / 3.80 / 2.38      x 256  11.5 / 6.7 / 4.0     x 1000  6.0 / 3.7 / 2.8 ms
+//                n = 2048  x 1   6.68 / 4.09 / 3.24      x 256  13.2 / 7.8 / 5.3     x 1000  6.3 / 4.9 / 4.4
+//                n = 4096  x 1   7.60 / 5.65 / 7.09      x 256  19.1 / 14.5 / 15.3   x 1000  9.7 / 8.1
+//                n = 8192  x 1  12.04 / 12.77            x 256  30.2 / 27.0          x 1000 18.6 / 16.3
+//         ETD34  n = 1024  x 1   1.97 / 1.11 / 0.65                                  x 1000  5.4 / 3.3 / 3.0
+//                n = 2048  x 1   1.40 / 0.84 / 0.61                                  x 1000  5.6 / 3.9 / 4.0
+//                n = 8192  x 1   1.34 / 1.65                                         x 1000 10.1 / 13.5
+//         IF34   n = 1024  x 1   0.35 / 0.23 / 0.17                                  x 1000  1.55 / 1.23 / 1.15
+//                n = 2048  x 1   0.37 / 0.26 / 0.24                                  x 1000  2.00 / 1.84 / 2.11
+//                n = 8192  x 1   0.71 / 0.77                                         x 1000  6.9 / 7.0
+//   advect IF34  n = 512   x 1   1.85 / 1.60             x 256   2.8 / 2.5           x 1000  1.03 / 1.00
+//                n = 1024  x 1   3.28 / 2.26 / 2.03      x 256   4.0 / 3.0 / 2.8     x 1000  1.54 / 1.24 / 1.21
+//                n = 2048  x 1   4.08 / 2.80 / 3.06      x 256   6.1 / 4.0 / 4.1     x 1000  1.88 / 1.64
+//                n = 4096  x 1   4.93 / 3.94 / 6.24      x 256   8.2 / 5.8 / 8.9     x 1000  2.70 / 2.73
 //                n = 8192  x 1   7.91 / 9.71             x 256  12.7 / 16.7
+//         ETD35  n = 1024  x 1   0.62 / 0.38 / 0.29      x 256   1.37 / 0.85 / 0.68  x 1000  2.06 / 1.47 / 1.59
+//                n = 4096  x 1   0.64 / 0.52             x 256   1.72 / 1.28         x 1000  4.32 / 3.93
+//         ETD34  n = 1024  x 1   0.90 / 0.53 / 0.38      x 256   1.30 / 0.84 / 0.66  x 1000  2.15 / 1.57 / 1.68
+//                n = 2048  x 1   0.83 / 0.50             x 256   1.39 / 0.93         x 1000  2.40 / 2.23
+//                n = 4096  x 1   0.83 / 0.59             x 256   1.53 / 1.13         x 1000  3.49 / 3.64
 // FP32 and MIXED runs gain as much, but keep the base tile: a tile has its own order of
 // rounding, and in FP32 storage that moves the step sizes and with them the results (MIXED
 // soliton ensembles by 4e-9, FP32 KS by 3e-6), so there the caller chooses.  Likewise an
@@ -229,14 +241,10 @@ bool lookup(int prec, int nlk, int variant, int log2n, bool learn, KernelEntry* 
 // state; KS: 1e-13).  The proposer
 // counts accepted steps by the workgroup's size, so its kernels keep the base tile; so do
 // runs that log their attempts, whose logs compare with the proposer's attempt by attempt.
-int default_tile(int prec, int nlk, int log2n, int count, int cu, bool base_only) {
-  if (base_only || prec != RKS_F64 || nlk == RKS_NL_HANKEL_CUBIC || log2n < 9) return 0;
-  if (nlk == RKS_NL_CUBIC_FFT) {
-    if (log2n == 10 || log2n == 11) return 2;
-    return log2n == 13 ? 2 * count > cu : 1;
-  }
-  if (log2n == 10) return count <= cu ? 2 : 1;
-  return log2n == 13 ? 0 : 1;
+int default_tile(int prec, int nlk, int variant, int log2n, bool base_only) {
+  if (base_only || prec != RKS_F64 || nlk == RKS_NL_HANKEL_CUBIC || log2n < 9 || log2n == 13) return 0;
+  if (log2n == 10 || (nlk == RKS_NL_CUBIC_FFT && log2n == 11 && variant != RKS_M_IF34)) return 2;
+  return 1;
 }
 
 int ilog2(int n) {
@@ -297,7 +305,8 @@ struct rks_plan {
   // cap on resident workgroups per CU per bucket (0: as many as fit)
   int concurrent = 1;
   std::vector<int> wg_per_cu;
-  std::vector<int> undamped;  // per log2 n: trajectories whose rounding at the grid's end need not decay
+  std::vector<int> undamped;        // per trajectory: its rounding at the grid's end need not decay
+  std::vector<int> bucket_undamped;  // per bucket: how many are
   std::vector<int> tile;  // per bucket: 0 base tile, 1 twice, 2 four times the threads, -1 by default_tile
   std::vector<hipStream_t> bstream;
   std::vector<hipEvent_t> bdone;
@@ -305,6 +314,7 @@ struct rks_plan {
 };
 
 static void fill_ctrl(rks_ctrl* c, const rks_config* cfg);
+static hipError_t upload_order(rks_plan* p);
 
 // L[r][c] == L[(rows - r) mod rows][c] bitwise for every mode of a rows x cols
 // lin_op in device memory (1-D: cols = 1): the ETD/IF coefficients of a mode
@@ -493,7 +503,7 @@ int rks_plan_create(int method, int nl_kind, int precision, const rks_config* cf
   HIPCHK(hipMalloc(&p->d_L, L_total * sizeof(double)));
   HIPCHK(hipMalloc(&p->d_kx, kx_total * (p->esize / 2)));
   HIPCHK(hipMalloc(&p->d_queue, sizeof(int) * 64));
-  HIPCHK(hipMalloc(&p->d_order, sizeof(int) * ninst));
+  HIPCHK(hipMalloc(&p->d_order, sizeof(int) * 2 * ninst));
   HIPCHK(hipMemcpy(p->d_tab, &p->tab, sizeof(rks_tableau), hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(p->d_ctl, &p->ctl, sizeof(rks_ctrl), hipMemcpyHostToDevice));
   HIPCHK(hipMemset(p->d_ws, 0, ws_total));
@@ -605,8 +615,7 @@ int rks_plan_create(int method, int nl_kind, int precision, const rks_config* cf
                            (cx<float>*)p->d_tw[l], N);
       HIPCHK(hipGetLastError());
     }
-    HIPCHK(hipMemcpy(p->d_order, p->order.data(), sizeof(int) * ninst, hipMemcpyHostToDevice));
-    p->undamped.assign(14, 0);
+    p->undamped.assign(ninst, 0);
     if (nl_kind == RKS_NL_ADVECT_RFFT && precision == RKS_F64 && ninst <= 4) {
       // a few: from the caller's arrays, without a launch and a read back
       for (int i = 0; i < ninst; ++i) {
@@ -614,14 +623,19 @@ int rks_plan_create(int method, int nl_kind, int precision, const rks_config* cf
         double re = 0.0, k = 0.0;
         HIPCHK(hipMemcpy(&re, (const double*)desc[i].L + (desc[i].L_is_complex ? 2 * m : m), sizeof(double), hipMemcpyDefault));
         HIPCHK(hipMemcpy(&k, (const double*)desc[i].kx + m, sizeof(double), hipMemcpyDefault));
-        p->undamped[ilog2(desc[i].n)] += !rks_damped(re, desc[i].nl_coef, k);
+        p->undamped[i] = rks_damped(re, desc[i].nl_coef, k) ? 0 : 1;
       }
     } else if (nl_kind == RKS_NL_ADVECT_RFFT && precision == RKS_F64) {
-      hipLaunchKernelGGL(rks_zero_int, dim3(1), dim3(64), 0, 0, p->d_queue, 64);
-      hipLaunchKernelGGL(rks_count_undamped, dim3((ninst + 255) / 256), dim3(256), 0, 0, p->d_inst, ninst, p->d_queue);
+      hipLaunchKernelGGL(rks_mark_undamped, dim3((ninst + 255) / 256), dim3(256), 0, 0, p->d_inst, ninst, p->d_order);
       HIPCHK(hipGetLastError());
-      HIPCHK(hipMemcpy(p->undamped.data(), p->d_queue, sizeof(int) * 14, hipMemcpyDeviceToHost));
+      HIPCHK(hipMemcpy(p->undamped.data(), p->d_order, sizeof(int) * ninst, hipMemcpyDeviceToHost));
     }
+    for (size_t b = 0; b < p->bucket_start.size(); ++b) {
+      int n = 0;
+      for (int k = 0; k < p->bucket_count[b]; ++k) n += p->undamped[p->order[p->bucket_start[b] + k]];
+      p->bucket_undamped.push_back(n);
+    }
+    HIPCHK(upload_order(p));
     HIPCHK(hipDeviceSynchronize());
   }
   *out = p;
@@ -641,6 +655,18 @@ static void fill_ctrl(rks_ctrl* c, const rks_config* cfg) {
   c->contour_points = cfg->contour_points;
   c->modecutoff = cfg->modecutoff;
   c->contour_radius = cfg->contour_radius;
+}
+
+// d_order: every bucket's trajectories in the order in which its workgroups take them, then
+// every bucket's once more with those that keep the base tile (undamped) behind the others.
+static hipError_t upload_order(rks_plan* p) {
+  std::vector<int> o(p->order);
+  o.insert(o.end(), p->order.begin(), p->order.end());
+  for (size_t b = 0; b < p->bucket_start.size(); ++b) {
+    auto first = o.begin() + p->ninst + p->bucket_start[b];
+    std::stable_partition(first, first + p->bucket_count[b], [&](int i) { return !p->undamped[i]; });
+  }
+  return hipMemcpy(p->d_order, o.data(), sizeof(int) * o.size(), hipMemcpyHostToDevice);
 }
 
 int rks_set_config(rks_plan* p, const rks_config* cfg, hipStream_t stream) {
@@ -738,15 +764,37 @@ static char* inst_cbase(const rks_plan* p, int inst) {
 // the proposer variant runs: a proposer or training records are attached
 static bool learns(const rks_plan* p) { return p->mlp.on || p->d_rec != nullptr; }
 
-// the tile that bucket b runs on: the caller's choice (a tile without a proposer variant gives
-// way to the base tile when a proposer or records are attached after it), else default_tile
-static int bucket_tile(const rks_plan* p, size_t b) {
+// the tile of bucket b's trajectories (those with damped, or undamped, last modes): the caller's
+// choice (a tile without a proposer variant gives way to the base tile when a proposer or records
+// are attached after it), else default_tile
+static int bucket_tile(const rks_plan* p, size_t b, bool undamped) {
   if (b < p->tile.size() && p->tile[b] >= 0) {
     KernelEntry e;
     return lookup(p->prec, p->nlk, p->variant, p->bucket_log2[b], learns(p), &e, p->tile[b]) ? p->tile[b] : 0;
   }
-  return default_tile(p->prec, p->nlk, p->bucket_log2[b], p->bucket_count[b], p->cu,
-                      p->undamped[p->bucket_log2[b]] || learns(p) || p->d_log != nullptr);
+  return default_tile(p->prec, p->nlk, p->variant, p->bucket_log2[b], undamped || learns(p) || p->d_log != nullptr);
+}
+
+// The launches of a plan: a bucket each, or two where its trajectories run on different tiles.
+struct LaunchPart {
+  size_t bucket;
+  const int* order;
+  int count, tile;
+};
+
+static std::vector<LaunchPart> launch_parts(const rks_plan* p) {
+  std::vector<LaunchPart> v;
+  for (size_t b = 0; b < p->bucket_log2.size(); ++b) {
+    const int n = p->bucket_count[b], nu = p->bucket_undamped[b], start = p->bucket_start[b];
+    const int td = bucket_tile(p, b, false), tu = bucket_tile(p, b, true);
+    if (nu == 0 || nu == n || td == tu) {
+      v.push_back({b, p->d_order + start, n, nu == n ? tu : td});
+    } else {
+      v.push_back({b, p->d_order + p->ninst + start, n - nu, td});
+      v.push_back({b, p->d_order + p->ninst + start + n - nu, nu, tu});
+    }
+  }
+  return v;
 }
 
 static int launch_all(rks_plan* p, int mode, double h_mode, hipStream_t stream) {
@@ -763,23 +811,25 @@ static int launch_all(rks_plan* p, int mode, double h_mode, hipStream_t stream) 
   L.io = p->d_io;
   L.mode = mode;
   L.h_mode = h_mode;
-  const size_t nb = p->bucket_log2.size();
+  const std::vector<LaunchPart> parts = launch_parts(p);
+  const size_t np = parts.size();
   const bool learn = learns(p);
-  std::vector<KernelEntry> kern(nb);
-  std::vector<int> grid(nb);
+  std::vector<KernelEntry> kern(np);
+  std::vector<int> grid(np);
   bool queued = false;
-  for (size_t b = 0; b < nb; ++b) {
-    KernelEntry& e = kern[b];
-    if (!lookup(p->prec, p->nlk, p->variant, p->bucket_log2[b], learn, &e, bucket_tile(p, b)))
+  for (size_t i = 0; i < np; ++i) {
+    KernelEntry& e = kern[i];
+    const size_t b = parts[i].bucket;
+    if (!lookup(p->prec, p->nlk, p->variant, p->bucket_log2[b], learn, &e, parts[i].tile))
       return fail(RKS_ERR_INVALID, "no kernel for this grid size, variant and tile");
-    grid[b] = p->bucket_count[b];
-    if (grid[b] <= p->cu) continue;  // a CU holds at least one workgroup
+    grid[i] = parts[i].count;
+    if (grid[i] <= p->cu) continue;  // a CU holds at least one workgroup
     int per_cu = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, e.fn, e.threads, e.lds) != hipSuccess || per_cu < 1)
       per_cu = 1;
     if (b < p->wg_per_cu.size() && p->wg_per_cu[b] > 0 && p->wg_per_cu[b] < per_cu) per_cu = p->wg_per_cu[b];
-    if (grid[b] > per_cu * p->cu) {
-      grid[b] = per_cu * p->cu;
+    if (grid[i] > per_cu * p->cu) {
+      grid[i] = per_cu * p->cu;
       queued = true;
     }
   }
@@ -789,13 +839,13 @@ static int launch_all(rks_plan* p, int mode, double h_mode, hipStream_t stream) 
     hipLaunchKernelGGL(rks_zero_int, dim3(1), dim3(64), 0, stream, p->d_queue, 64);
     HIPCHK(hipGetLastError());
   }
-  const bool conc = p->concurrent && nb > 1;
+  const bool conc = p->concurrent && np > 1;
   if (conc) {
-    // fork: every bucket stream waits for the caller's stream (queue counters cleared)
-    if (p->bstream.size() < nb) {
+    // fork: every launch's stream waits for the caller's stream (queue counters cleared)
+    if (p->bstream.size() < np) {
       HIPCHK(hipDeviceSynchronize());
       if (!p->fork) HIPCHK(hipEventCreateWithFlags(&p->fork, hipEventDisableTiming));
-      while (p->bstream.size() < nb) {
+      while (p->bstream.size() < np) {
         hipStream_t st;
         hipEvent_t ev;
         HIPCHK(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
@@ -806,26 +856,26 @@ static int launch_all(rks_plan* p, int mode, double h_mode, hipStream_t stream) 
     }
     HIPCHK(hipEventRecord(p->fork, stream));
   }
-  for (size_t b = 0; b < nb; ++b) {
-    const KernelEntry& e = kern[b];
-    L.order = p->d_order + p->bucket_start[b];
-    L.count = p->bucket_count[b];
-    L.queue = grid[b] < L.count ? p->d_queue + b : nullptr;
-    L.tw = p->d_tw[p->bucket_log2[b]];
+  for (size_t i = 0; i < np; ++i) {
+    const KernelEntry& e = kern[i];
+    L.order = parts[i].order;
+    L.count = parts[i].count;
+    L.queue = grid[i] < L.count ? p->d_queue + i : nullptr;
+    L.tw = p->d_tw[p->bucket_log2[parts[i].bucket]];
     void* args[] = {&L};
     hipStream_t st = stream;
     if (conc) {
-      st = p->bstream[b];
+      st = p->bstream[i];
       HIPCHK(hipStreamWaitEvent(st, p->fork, 0));
     }
-    HIPCHK(hipLaunchKernel(e.fn, dim3(grid[b]), dim3(e.threads), args, (size_t)e.lds, st));
-    if (conc) HIPCHK(hipEventRecord(p->bdone[b], st));
+    HIPCHK(hipLaunchKernel(e.fn, dim3(grid[i]), dim3(e.threads), args, (size_t)e.lds, st));
+    if (conc) HIPCHK(hipEventRecord(p->bdone[i], st));
   }
-  // join after every bucket is queued: a wait on the caller's stream is a
+  // join after every launch is queued: a wait on the caller's stream is a
   // barrier in the hardware queue that stream maps to, and a bucket stream
-  // sharing that queue would otherwise start only when the earlier buckets end
+  // sharing that queue would otherwise start only when the earlier ones end
   if (conc)
-    for (size_t b = 0; b < nb; ++b) HIPCHK(hipStreamWaitEvent(stream, p->bdone[b], 0));
+    for (size_t i = 0; i < np; ++i) HIPCHK(hipStreamWaitEvent(stream, p->bdone[i], 0));
   return RKS_OK;
 }
 
@@ -1108,7 +1158,7 @@ int rks_plan_set_priority(rks_plan* p, const double* cost) {
     std::stable_sort(first, first + p->bucket_count[b], [&](int a, int c) { return cost[a] > cost[c]; });
   }
   HIPCHK(hipDeviceSynchronize());
-  HIPCHK(hipMemcpy(p->d_order, p->order.data(), sizeof(int) * p->ninst, hipMemcpyHostToDevice));
+  HIPCHK(upload_order(p));
   return RKS_OK;
 }
 
@@ -1162,7 +1212,8 @@ int rks_plan_set_launch(rks_plan* p, int concurrent, const int* wg_per_cu, const
 
 int rks_plan_tiles(rks_plan* p, int* tile, int cap) {
   if (!p || !tile) return fail(RKS_ERR_INVALID, "null argument");
-  for (size_t b = 0; b < p->bucket_log2.size() && (int)b < cap; ++b) tile[b] = bucket_tile(p, b);
+  for (size_t b = 0; b < p->bucket_log2.size() && (int)b < cap; ++b)
+    tile[b] = bucket_tile(p, b, p->bucket_undamped[b] == p->bucket_count[b]);
   return RKS_OK;
 }
 

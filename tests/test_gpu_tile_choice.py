@@ -66,3 +66,41 @@ def test_tuning_starts_from_the_plans_own_tiles():
         shapes.append(plan.tiles())
     assert shapes[0] == own and [0] in shapes and [1] in shapes
     plan.set_launch(True, None, joint["tiles"][0])
+
+
+@pytest.mark.parametrize("kind,n", [("advect", 1024), ("cubic", 8192)])
+def test_result_does_not_depend_on_the_rest_of_the_plan(kind, n):
+    """A trajectory alone, among 299 like it, and beside one whose last modes are not damped (and
+    that one alone): the same bits, in any order of the bucket."""
+    from rkstiff_amd import _lib
+    from rkstiff_amd.engine import Plan
+    from rkstiff_amd.nonlinear import AdvectiveNL, CubicNL
+    if kind == "advect":
+        x, k = np.arange(n) * (32 * np.pi / n), 2 * np.pi * np.fft.rfftfreq(n, d=32 * np.pi / n)
+        nl, u, tf = AdvectiveNL(torch.as_tensor(k), -1.0), np.fft.rfft(np.cos(x / 16) * (1 + np.sin(x / 16))), 2.0
+        ops = [k**2 * (1 - k**2), -0.05 * k**2]
+    else:
+        x, k = -16.0 + np.arange(n) * (32.0 / n), 2 * np.pi * np.fft.fftfreq(n, d=32.0 / n)
+        nl, u, tf = CubicNL(n, 1.0), np.fft.fft(1.5 / np.cosh(1.5 * x)), 0.05
+        ops = [-0.5j * k**2, -0.4j * k**2]
+    ut = torch.as_tensor(u).cuda()
+
+    def run(which, cost=None):
+        plan = Plan("ETD35", nl, _lib.F64, None, None, [nl.descriptor(torch.as_tensor(ops[w])) for w in which])
+        if cost is not None:
+            plan.set_priority(cost)
+        uf, m = [torch.empty_like(ut) for _ in which], len(which)
+        plan.evolve([ut] * m, uf, [0.0] * m, [tf] * m, [tf / 50] * m)
+        assert all(s["status"] == _lib.RKS_OK for s in plan.stats())
+        return uf, plan.tiles()
+
+    (a,), own = run([0])
+    (b,), other = run([1])
+    print(kind, n, "tiles", own, other, flush=True)
+    many, tiles = run([0] * 300)
+    assert tiles == own and all(torch.equal(x, a) for x in many)
+    which = [0, 1] * 150
+    for cost in (None, np.arange(300.0)):
+        mixed, tiles = run(which, cost)
+        assert tiles == own
+        assert all(torch.equal(x, b if w else a) for x, w in zip(mixed, which))
