@@ -51,11 +51,16 @@ typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));  // two doub
 // vector units' FP64 rate, but an instruction of 2048 operations reads two LDS values per
 // lane where 32 FMAs of a 4 x 2 register tile read 24; those reads bounded the vector form.
 // The next chunk's global loads are in flight during a chunk's products, one barrier each.
-// nr = 251, 1024 complex vectors: 43.5 us by FMAs on a 4 x 2 register tile, now 10.4 (the
-// products alone take 3.3 us at 78 TFLOP/s).  ROWS 64: a wave has 16 rows of its own.  ROWS 16: the four waves share one tile and split
-// each chunk's k, so four times the workgroups; taken while 64-row tiles would leave CUs idle.
+// ROWS 64: a wave has 16 rows of its own.  ROWS 16: the four waves share one tile, so four times
+// the workgroups; taken while 64-row tiles would leave CUs idle.  There wave w takes the quarter
+// w of each chunk's k; with 64 rows a wave keeps the four quarters' sums apart and adds them in
+// the same order, so a vector's result does not depend on the batch it is in.  Two waves per
+// SIMD (256 registers) keep the sums out of the accumulation registers, to and from which each
+// chunk would copy them (12.0 us).
+// nr = 251, 1024 complex vectors: 43.5 us by FMAs on a 4 x 2 register tile, now 10.2 (the
+// products alone take 3.3 us at 78 TFLOP/s; with one sum per wave 10.4).
 template <bool CPLX, int EPI, int ROWS>
-__global__ __launch_bounds__(256) void hankel_gemm(const double* __restrict__ Y, int nr,
+__global__ __launch_bounds__(256, 2) void hankel_gemm(const double* __restrict__ Y, int nr,
                                                    const double* __restrict__ in, double* __restrict__ out,
                                                    int batch, double c, double gamma) {
   constexpr bool SPLIT = ROWS == 16;
@@ -87,7 +92,10 @@ __global__ __launch_bounds__(256) void hankel_gemm(const double* __restrict__ Y,
       xr[e] = v;
     }
   };
-  d4 a0 = {0.0, 0.0, 0.0, 0.0}, a1 = a0;
+  constexpr int NP = SPLIT ? 1 : 4;  // quarters of a chunk per wave
+  d4 a0[NP], a1[NP];
+#pragma unroll
+  for (int q = 0; q < NP; ++q) a0[q] = a1[q] = d4{0.0, 0.0, 0.0, 0.0};
   load(0);
   for (int k0 = 0, buf = 0; k0 < nr; k0 += HB_K, buf ^= 1) {
 #pragma unroll
@@ -96,17 +104,15 @@ __global__ __launch_bounds__(256) void hankel_gemm(const double* __restrict__ Y,
     for (int e = 0; e < XE; ++e) Xs[buf][rt + 8 * e][kt] = xr[e];
     if (k0 + HB_K < nr) load(k0 + HB_K);
     __syncthreads();
-    constexpr int S = SPLIT ? HB_K / 16 : HB_K / 4;  // k per lane group and chunk
-    const int kb = SPLIT ? w * (HB_K / 4) + g * S : g * S;
-    const double* yp = &Ys[buf][SPLIT ? n : w * 16 + n][kb];
-    const d2* xp = &Xs[buf][n][kb];
 #pragma unroll
-    for (int s = 0; s < S; s += 2) {
-      const d2 y = *(const d2*)(yp + s), x0 = xp[s], x1 = xp[s + 1];
-      a0 = __builtin_amdgcn_mfma_f64_16x16x4f64(x0.x, y.x, a0, 0, 0, 0);
-      a1 = __builtin_amdgcn_mfma_f64_16x16x4f64(x0.y, y.x, a1, 0, 0, 0);
-      a0 = __builtin_amdgcn_mfma_f64_16x16x4f64(x1.x, y.y, a0, 0, 0, 0);
-      a1 = __builtin_amdgcn_mfma_f64_16x16x4f64(x1.y, y.y, a1, 0, 0, 0);
+    for (int q = 0; q < NP; ++q) {
+      const int kb = (SPLIT ? w : q) * (HB_K / 4) + 2 * g;
+      const d2 y = *(const d2*)&Ys[buf][SPLIT ? n : w * 16 + n][kb];
+      const d2 x0 = Xs[buf][n][kb], x1 = Xs[buf][n][kb + 1];
+      a0[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(x0.x, y.x, a0[q], 0, 0, 0);
+      a1[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(x0.y, y.x, a1[q], 0, 0, 0);
+      a0[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(x1.x, y.y, a0[q], 0, 0, 0);
+      a1[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(x1.y, y.y, a1[q], 0, 0, 0);
     }
   }
   const int i = i0 + (SPLIT ? n : w * 16 + n);
@@ -116,7 +122,7 @@ __global__ __launch_bounds__(256) void hankel_gemm(const double* __restrict__ Y,
     vi *= c;
     if (i >= nr) return;
     if (EPI == EPI_CUBIC) {
-      const double m2 = vr * vr + vi * vi;
+      const double m2 = fma(vr, vr, vi * vi);
       vr *= m2;
       vi *= m2;
     } else if (EPI == EPI_TIMES_I) {
@@ -134,11 +140,12 @@ __global__ __launch_bounds__(256) void hankel_gemm(const double* __restrict__ Y,
       if (b + HB_B < batch) out[(size_t)(b + HB_B) * nr + i] = vi;
     }
   };
+  // the four partial sums in order
   if constexpr (SPLIT) {
-    // the four partial sums in wave order; wave w finishes the results r = w
+    // wave w finishes the results r = w
     __shared__ d2 part[4][4][64];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) part[w][r][l] = d2{a0[r], a1[r]};
+    for (int r = 0; r < 4; ++r) part[w][r][l] = d2{a0[0][r], a1[0][r]};
     __syncthreads();
     d2 v = part[0][w][l];
 #pragma unroll
@@ -146,7 +153,8 @@ __global__ __launch_bounds__(256) void hankel_gemm(const double* __restrict__ Y,
     store(4 * w + g, v.x, v.y);
   } else {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) store(4 * r + g, a0[r], a1[r]);
+    for (int r = 0; r < 4; ++r)
+      store(4 * r + g, a0[0][r] + a0[1][r] + a0[2][r] + a0[3][r], a1[0][r] + a1[1][r] + a1[2][r] + a1[3][r]);
   }
 }
 

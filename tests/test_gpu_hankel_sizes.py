@@ -29,3 +29,20 @@ def test_hankel_products_at_tile_edges(nr, batch, cplx):
     for got, c in ((ht.ht(ft), S), (ht.iht(ft), 1.0 / S)):
         bound = 4 * (nr + 8) * EPS * abs(c) * (np.abs(f) @ np.abs(Y).T)
         assert np.all(np.abs(got.cpu().numpy() - c * (f @ Y.T)) <= bound)
+
+
+@pytest.mark.parametrize("nr", [17, 100, 251])
+@pytest.mark.parametrize("cplx", [False, True])
+def test_hankel_products_do_not_depend_on_the_batch(nr, cplx):
+    """A profile transformed alone and among others: the same bits, whichever row tile runs."""
+    from rkstiff_amd.transforms import HankelTransform
+    ht = HankelTransform(nr, 5.0)
+    rng = np.random.default_rng(nr)
+    f = rng.standard_normal((6000, nr))
+    if cplx:
+        f = f + 1j * rng.standard_normal(f.shape)
+    ft = torch.as_tensor(f).cuda()
+    for op in (ht.ht, ht.iht) + ((ht.cubic_nl(2.0),) if cplx else ()):
+        many = op(ft) if op in (ht.ht, ht.iht) else torch.stack([op(x) for x in ft[:40]])
+        for i in (0, 15, 16, 39):
+            assert torch.equal(op(ft[i]), many[i])
