@@ -306,7 +306,6 @@ __global__ __launch_bounds__((Geo2<R, LOG2>::CT), 4) void k2_col(rks2_launch P, 
       ix.sym = sym;
       ix.lim = G::MGEN_SYM_I;
       ix.anyq = 0;
-      ix.fold = 0;
 #pragma unroll
       for (int j = 0; j < CH / 2; ++j) {
         const int q = r0 + (ch * (CH / 2) + j) * RS;
@@ -542,7 +541,6 @@ __global__ __launch_bounds__(256) void k2_norm(rks2_launch P) {
   ix.sym = sym;
   ix.lim = G::MGEN_SYM_I;
   ix.anyq = 1;
-  ix.fold = 0;
 #pragma unroll
   for (int j = 0; j < NE / 2; ++j) {
     const int p = blockIdx.x * NT * (NE / 2) + t + j * NT;

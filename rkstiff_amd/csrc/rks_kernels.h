@@ -487,9 +487,8 @@ struct ChunkIdx {
   int sym;   // slots are mirror pairs sharing coefficients
   int lim;   // first mode without stored coefficients (sym only)
   int anyq;  // any odd slot may lie below lim (else only slot 1)
-  int fold;  // 1-D: mode m > fold / 2 reads the coefficient of fold - m (0: every mode its own)
   __device__ __forceinline__ ChunkIdx() {}
-  __device__ __forceinline__ ChunkIdx(int m0, int T, int mlim) : sym(0), lim(0), anyq(0), fold(0) {
+  __device__ __forceinline__ ChunkIdx(int m0, int T, int mlim) : sym(0), lim(0), anyq(0) {
 #pragma unroll
     for (int i = 0; i < CH; ++i) {
       const int x = m0 + i * T;
@@ -534,18 +533,36 @@ struct Own {
   }
 };
 
+// Modes of the general kernel's stage passes, chunk c.  fft layout: the mirror pairs q = t + jT
+// (slot 2j) and N - q (slot 2j + 1; N/2 for q = 0), as in the norm (NormOrder), so a pair shares
+// one load of each coefficient of a mirror-symmetric L; by the thread's own modes every mode
+// loads its own.  One FP32 evolve, n = 8192, own modes / pairs: ETD34 1.31 / 1.20 ms, ETD5 5.01 /
+// 4.35, IF45DP 288 / 245; n = 4096 1.11 / 1.04, 3.63 / 3.28, 205 / 183.  Else the thread's own
+// modes.
 template <int N, int M, int T, int NLK, int CH>
-__device__ __forceinline__ ChunkIdx<CH> own_chunk(int c, const Own<N, M, T, NLK>& ow) {
+__device__ __forceinline__ ChunkIdx<CH> pass_chunk(int c, const Own<N, M, T, NLK>& ow) {
   ChunkIdx<CH> ix;
-  ix.sym = 0;
-  ix.lim = 0;
   ix.anyq = 0;
-  ix.fold = ow.fold;
+  if constexpr (M == N && NLK != NLK_HANKEL) {
+    static_assert(CH % 2 == 0 && N % (2 * T) == 0, "whole mirror pairs per chunk");
+    ix.sym = ow.fold != 0;
+    ix.lim = N / 2 + 1;
 #pragma unroll
-  for (int i = 0; i < CH; ++i) {
-    const int x = ow.t + (c * CH + i) * T;
-    ix.ok[i] = x < ow.lim;
-    ix.m[i] = ix.ok[i] ? x : 0;
+    for (int j = 0; j < CH / 2; ++j) {
+      const int q = ow.t + (c * (CH / 2) + j) * T;
+      ix.m[2 * j] = q;
+      ix.m[2 * j + 1] = q == 0 ? N / 2 : N - q;
+      ix.ok[2 * j] = ix.ok[2 * j + 1] = true;
+    }
+  } else {
+    ix.sym = 0;
+    ix.lim = 0;
+#pragma unroll
+    for (int i = 0; i < CH; ++i) {
+      const int x = ow.t + (c * CH + i) * T;
+      ix.ok[i] = x < ow.lim;
+      ix.m[i] = ix.ok[i] ? x : 0;
+    }
   }
   return ix;
 }
@@ -584,7 +601,7 @@ __device__ __forceinline__ void load_coef(const rks_tableau& tb, const char* cba
   // address and the caches serve the repeat.
   int ci[CH];
 #pragma unroll
-  for (int i = 0; i < CH; ++i) ci[i] = (ix.fold && ix.m[i] > ix.fold / 2) ? ix.fold - ix.m[i] : ix.m[i];
+  for (int i = 0; i < CH; ++i) ci[i] = ix.m[i];
   if constexpr (CH % 2 == 0 && sizeof(RS) > 4) {
 #pragma unroll
     for (int j = 0; j < CH / 2; ++j)
@@ -1195,6 +1212,7 @@ __device__ int run_instance(const rks_launch& P, int idx, cx<R>* buf, const cx<R
   constexpr int MPT = OW::MPT;
   constexpr int CH = Chunk<MPT, (int)sizeof(C)>::CH;
   constexpr bool METHOD = METH != RKS_METH_ANY;
+  constexpr bool PAIRED = !METHOD && M == N && NLK != NLK_HANKEL;  // pass_chunk: other modes than the transforms'
   using TT = MethodTab<METHOD ? METH : 0, (int)sizeof(C), (int)sizeof(CN), NLK == NLK_ADVECT>;
   constexpr bool FUSED = TT::tab.st[TT::tab.nstage - 1].has_nl == 0;  // (METHOD) no NL in the last stage
   constexpr int LAST_SLOT = TT::tab.st[FUSED ? TT::tab.nstage - 2 : TT::tab.nstage - 1].nl_slot;
@@ -1396,7 +1414,7 @@ __device__ int run_instance(const rks_launch& P, int idx, cx<R>* buf, const cx<R
             // per-mode |u_new| and |err|^2 (FP32 buffer: |err|) wait in the idle LDS buffer
 #pragma unroll 1
             for (int c = 0; c < Chunk<MPT, (int)sizeof(C)>::NCH; ++c) {
-              const ChunkIdx<CH> ix = own_chunk<N, M, T, NLK, CH>(c, ow.fresh());
+              const ChunkIdx<CH> ix = pass_chunk<N, M, T, NLK, CH>(c, ow.fresh());
               C acc[CH], ev[CH];
               final_chunk<R, RN, CH>(tb, u, slot, cbase, (size_t)Mc, ix, h, acc, ev);
 #pragma unroll
@@ -1416,11 +1434,11 @@ __device__ int run_instance(const rks_launch& P, int idx, cx<R>* buf, const cx<R
             }
             break;
           }
-          // the stage argument through the thread's own places of the LDS buffer: the
-          // run-time term loop stays rolled over the chunks
+          // the stage argument through the LDS buffer: the run-time term loop stays rolled over
+          // the chunks, and the transforms' modes may be other threads'
 #pragma unroll 1
           for (int c = 0; c < Chunk<MPT, (int)sizeof(C)>::NCH; ++c) {
-            const ChunkIdx<CH> ix = own_chunk<N, M, T, NLK, CH>(c, ow.fresh());
+            const ChunkIdx<CH> ix = pass_chunk<N, M, T, NLK, CH>(c, ow.fresh());
             C acc[CH];
             stage_chunk<R, RN, CH>(tb, S, u, slot, cbase, (size_t)Mc, ix, h, acc);
 #pragma unroll
@@ -1434,6 +1452,7 @@ __device__ int run_instance(const rks_launch& P, int idx, cx<R>* buf, const cx<R
               buf[ix.m[i]] = acc[i];
             }
           }
+          if constexpr (PAIRED) __syncthreads();  // buf, and cand for what copies it
           if (!S.has_nl) continue;
           const OW of = ow.fresh();
 #pragma unroll
@@ -1450,6 +1469,7 @@ __device__ int run_instance(const rks_launch& P, int idx, cx<R>* buf, const cx<R
           nv[k] = cvt<RN>(v[k]);
           if (of.ok(k)) gstore(dst, of.m(k), nv[k]);
         }
+        if constexpr (PAIRED) __syncthreads();  // the stage passes read them by pairs
       }
       if (!adaptive) {
         h_suggest = h;
@@ -1532,7 +1552,7 @@ __device__ int run_instance(const rks_launch& P, int idx, cx<R>* buf, const cx<R
         constexpr int NCH = (NO::SLOTS + CH - 1) / CH;
 #pragma unroll 1
         for (int c = 0; c < NCH; ++c) {
-          ChunkIdx<CH> ix = own_chunk<N, M, T, NLK, CH>(c, ow.fresh());
+          ChunkIdx<CH> ix = pass_chunk<N, M, T, NLK, CH>(c, ow.fresh());
 #pragma unroll
           for (int i = 0; i < CH; ++i) {
             ix.ok[i] = NO::ok(c * CH + i, ow.lim);
