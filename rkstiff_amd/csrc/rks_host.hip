@@ -217,11 +217,15 @@ bool lookup(int prec, int nlk, int variant, int log2n, bool learn, KernelEntry* 
 //                n = 2048  x 1   6.68 / 4.09 / 3.24      x 256  13.2 / 7.8 / 5.3     x 1000  6.3 / 4.9 / 4.4
 //                n = 4096  x 1   7.60 / 5.65 / 7.09      x 256  19.1 / 14.5 / 15.3   x 1000  9.7 / 8.1
 //                n = 8192  x 1  12.04 / 12.77            x 256  30.2 / 27.0          x 1000 18.6 / 16.3
-//         ETD34  n = 1024  x 1   1.97 / 1.11 / 0.65                                  x 1000  5.4 / 3.3 / 3.0
-//                n = 2048  x 1   1.40 / 0.84 / 0.61                                  x 1000  5.6 / 3.9 / 4.0
-//                n = 8192  x 1   1.34 / 1.65                                         x 1000 10.1 / 13.5
-//         IF34   n = 1024  x 1   0.35 / 0.23 / 0.17                                  x 1000  1.55 / 1.23 / 1.15
+//         ETD34  n = 512   x 1   1.60 / 0.93             x 256   3.0 / 1.8           x 1000  3.8 / 2.5
+//                n = 1024  x 1   1.89 / 1.04 / 0.63      x 256   4.4 / 2.4 / 1.5     x 1000  5.3 / 3.1 / 2.8
+//                n = 2048  x 1   1.33 / 0.77 / 0.57      x 256   4.1 / 2.3 / 1.6     x 1000  5.3 / 3.5 / 3.7
+//                n = 4096  x 1   1.05 / 0.74             x 256   3.1 / 2.0           x 1000  5.3 / 4.9
+//                n = 8192  x 1   1.17 / 1.36             x 256   3.1 / 3.3           x 1000  8.8 / 10.9
+//         IF34   n = 512   x 1   0.18 / 0.14             x 256   0.47 / 0.39         x 1000  1.00 / 0.89
+//                n = 1024  x 1   0.35 / 0.23 / 0.17                                  x 1000  1.55 / 1.23 / 1.15
 //                n = 2048  x 1   0.37 / 0.26 / 0.24                                  x 1000  2.00 / 1.84 / 2.11
+//                n = 4096  x 1   0.43 / 0.35             x 256   1.29 / 1.00         x 1000  3.30 / 3.26
 //                n = 8192  x 1   0.71 / 0.77                                         x 1000  6.9 / 7.0
 //   advect IF34  n = 512   x 1   1.85 / 1.60             x 256   2.8 / 2.5           x 1000  1.03 / 1.00
 //                n = 1024  x 1   3.28 / 2.26 / 2.03      x 256   4.0 / 3.0 / 2.8     x 1000  1.54 / 1.24 / 1.21
@@ -230,9 +234,10 @@ bool lookup(int prec, int nlk, int variant, int log2n, bool learn, KernelEntry* 
 //                n = 8192  x 1   7.91 / 9.71             x 256  12.7 / 16.7
 //         ETD35  n = 1024  x 1   0.62 / 0.38 / 0.29      x 256   1.37 / 0.85 / 0.68  x 1000  2.06 / 1.47 / 1.59
 //                n = 4096  x 1   0.64 / 0.52             x 256   1.72 / 1.28         x 1000  4.32 / 3.93
-//         ETD34  n = 1024  x 1   0.90 / 0.53 / 0.38      x 256   1.30 / 0.84 / 0.66  x 1000  2.15 / 1.57 / 1.68
-//                n = 2048  x 1   0.83 / 0.50             x 256   1.39 / 0.93         x 1000  2.40 / 2.23
-//                n = 4096  x 1   0.83 / 0.59             x 256   1.53 / 1.13         x 1000  3.49 / 3.64
+//         ETD34  n = 512   x 1   0.61 / 0.39             x 256   0.95 / 0.62         x 1000  1.46 / 1.19
+//                n = 1024  x 1   0.89 / 0.50 / 0.36      x 256   1.29 / 0.78 / 0.64  x 1000  2.10 / 1.45 / 1.60
+//                n = 2048  x 1   0.77 / 0.48             x 256   1.25 / 0.85         x 1000  2.16 / 2.01
+//                n = 4096  x 1   0.77 / 0.56             x 256   1.37 / 1.03         x 1000  3.09 / 3.31
 // FP32 and MIXED runs gain as much, but keep the base tile: a tile has its own order of
 // rounding, and in FP32 storage that moves the step sizes and with them the results (MIXED
 // soliton ensembles by 4e-9, FP32 KS by 3e-6), so there the caller chooses.  Likewise an

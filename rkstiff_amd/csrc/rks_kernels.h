@@ -590,10 +590,10 @@ struct NormOrder {
 };
 
 // coefficient array c of the chunk's modes; M is the array stride (modes)
-template <typename RS, typename RN, int CH>
-__device__ __forceinline__ void load_coef(const rks_tableau& tb, const char* cbase, size_t M, int c,
+template <typename RS, typename RN, int CH, typename TB>
+__device__ __forceinline__ void load_coef(TB& tb, const char* cbase, size_t M, int c,
                                           const ChunkIdx<CH>& ix, cx<RS> (&w)[CH]) {
-  const char* q = cbase + (size_t)tb.coef_off[c] * M;
+  const char* q = uni(cbase + (size_t)tb.coef_off[c] * M);
   const int kind = tb.coef_rs[c];
   // Mirror pairs: FP32-state kernels issue one load per pair (plus the n/2
   // partner of q = 0).  The FP64-state kernels have no registers to spare
@@ -630,36 +630,36 @@ __device__ __forceinline__ void load_coef(const rks_tableau& tb, const char* cba
   };
   if (kind == RKS_CST_RS) {
     const cx<RS>* p = (const cx<RS>*)q;
-    gather([&](int m) { return p[m]; });
+    gather([&](int m) { return gload(p, m); });
   } else if (kind == RKS_CST_RN) {
     const cx<RN>* p = (const cx<RN>*)q;
-    gather([&](int m) { return cvt<RS>(p[m]); });
+    gather([&](int m) { return cvt<RS>(gload(p, m)); });
   } else if (kind == RKS_CST_RS_REAL) {
     const RS* p = (const RS*)q;
-    gather([&](int m) { return mkc(p[m], (RS)0); });
+    gather([&](int m) { return mkc(gload_real(p, m), (RS)0); });
   } else {
     const RN* p = (const RN*)q;
-    gather([&](int m) { return mkc((RS)p[m], (RS)0); });
+    gather([&](int m) { return mkc((RS)gload_real(p, m), (RS)0); });
   }
 }
 
 // slotp(s): NL array of slot s (const cx<RN>*)
-template <typename RS, typename RN, int CH, bool HSUM, typename SlotF>
-__device__ __forceinline__ void add_terms(const rks_tableau& tb, const rks_term* terms, int nterm, SlotF slotp,
+template <typename RS, typename RN, int CH, bool HSUM, typename TB, typename TM, typename SlotF>
+__device__ __forceinline__ void add_terms(TB& tb, TM* terms, int nterm, SlotF slotp,
                                           const char* cbase, size_t M, const ChunkIdx<CH>& ix, double h,
                                           cx<RS> (&acc)[CH]) {
   using C = cx<RS>;
   for (int j = 0; j < nterm; ++j) {
-    const rks_term& tm = terms[j];
-    const cx<RN>* nl = slotp(tm.src);
+    auto& tm = terms[j];
+    const cx<RN>* nl = uni(slotp(tm.src));
     C v[CH];
 #pragma unroll
-    for (int i = 0; i < CH; ++i) v[i] = cvt<RS>(nl[ix.m[i]]);
+    for (int i = 0; i < CH; ++i) v[i] = cvt<RS>(gload(nl, ix.m[i]));
     if (tm.src2 >= 0) {
-      const cx<RN>* nl2 = slotp(tm.src2);
+      const cx<RN>* nl2 = uni(slotp(tm.src2));
       const RS s2 = (RS)tm.scale2;
 #pragma unroll
-      for (int i = 0; i < CH; ++i) v[i] = v[i] + s2 * cvt<RS>(nl2[ix.m[i]]);
+      for (int i = 0; i < CH; ++i) v[i] = v[i] + s2 * cvt<RS>(gload(nl2, ix.m[i]));
     }
     if (tm.hmode == 2) {
       const RS hs = (RS)((tm.scale * h) / tm.den);
@@ -694,13 +694,13 @@ __device__ __forceinline__ void add_terms(const rks_tableau& tb, const rks_term*
 
 // k = E u + terms, or E u + h * sum(terms) for stages that factor h out (if34.py:126-128);
 // lanes past mlim come back zero
-template <typename RS, typename RN, int CH, typename SlotF>
-__device__ __forceinline__ void stage_chunk(const rks_tableau& tb, const rks_stage& S, const cx<RS>* __restrict__ u,
+template <typename RS, typename RN, int CH, typename TB, typename ST, typename SlotF>
+__device__ __forceinline__ void stage_chunk(TB& tb, ST& S, const cx<RS>* __restrict__ u,
                                             SlotF slotp, const char* cbase, size_t M, const ChunkIdx<CH>& ix,
                                             double h, cx<RS> (&acc)[CH]) {
   using C = cx<RS>;
 #pragma unroll
-  for (int i = 0; i < CH; ++i) acc[i] = u[ix.m[i]];
+  for (int i = 0; i < CH; ++i) acc[i] = gload(u, ix.m[i]);
   if (S.ecoef >= 0) {
     C e[CH];
     load_coef<RS, RN, CH>(tb, cbase, M, S.ecoef, ix, e);
@@ -721,16 +721,16 @@ __device__ __forceinline__ void stage_chunk(const rks_tableau& tb, const rks_sta
 }
 
 // modes m0 + i*T below mlim
-template <typename RS, typename RN, int CH, typename SlotF>
-__device__ __forceinline__ void stage_chunk(const rks_tableau& tb, const rks_stage& S, const cx<RS>* __restrict__ u,
+template <typename RS, typename RN, int CH, typename TB, typename ST, typename SlotF>
+__device__ __forceinline__ void stage_chunk(TB& tb, ST& S, const cx<RS>* __restrict__ u,
                                             SlotF slotp, const char* cbase, size_t M, int m0, int T, int mlim,
                                             double h, cx<RS> (&acc)[CH]) {
   stage_chunk<RS, RN, CH>(tb, S, u, slotp, cbase, M, ChunkIdx<CH>(m0, T, mlim), h, acc);
 }
 
 // embedded error estimate (etd35.py:344, etd34.py:190, if34.py:130, if45dp.py:170-177)
-template <typename RS, typename RN, int CH, typename SlotF>
-__device__ __forceinline__ void error_chunk(const rks_tableau& tb, SlotF slotp, const char* cbase, size_t M,
+template <typename RS, typename RN, int CH, typename TB, typename SlotF>
+__device__ __forceinline__ void error_chunk(TB& tb, SlotF slotp, const char* cbase, size_t M,
                                             const ChunkIdx<CH>& ix, double h, cx<RS> (&ev)[CH]) {
   add_terms<RS, RN, CH, true>(tb, tb.err, tb.nerr, slotp, cbase, M, ix, h, ev);
   if (tb.err_factored) {
@@ -754,8 +754,8 @@ __device__ __forceinline__ void error_chunk(const rks_tableau& tb, SlotF slotp, 
     if (!ix.ok[i]) ev[i] = mkc((RS)0, (RS)0);
 }
 
-template <typename RS, typename RN, int CH, typename SlotF>
-__device__ __forceinline__ void error_chunk(const rks_tableau& tb, SlotF slotp, const char* cbase, size_t M, int m0,
+template <typename RS, typename RN, int CH, typename TB, typename SlotF>
+__device__ __forceinline__ void error_chunk(TB& tb, SlotF slotp, const char* cbase, size_t M, int m0,
                                             int T, int mlim, double h, cx<RS> (&ev)[CH]) {
   error_chunk<RS, RN, CH>(tb, slotp, cbase, M, ChunkIdx<CH>(m0, T, mlim), h, ev);
 }
@@ -776,14 +776,14 @@ __host__ __device__ __forceinline__ bool rks_fused_final(const rks_tableau& tb) 
   return true;
 }
 
-template <typename RS, typename RN, int CH, typename SlotF>
-__device__ __forceinline__ void final_chunk(const rks_tableau& tb, const cx<RS>* __restrict__ u, SlotF slotp,
+template <typename RS, typename RN, int CH, typename TB, typename SlotF>
+__device__ __forceinline__ void final_chunk(TB& tb, const cx<RS>* __restrict__ u, SlotF slotp,
                                             const char* cbase, size_t M, const ChunkIdx<CH>& ix, double h,
                                             cx<RS> (&acc)[CH], cx<RS> (&ev)[CH]) {
   using C = cx<RS>;
-  const rks_stage& S = tb.st[tb.nstage - 1];
+  auto& S = tb.st[tb.nstage - 1];
 #pragma unroll
-  for (int i = 0; i < CH; ++i) acc[i] = u[ix.m[i]];
+  for (int i = 0; i < CH; ++i) acc[i] = gload(u, ix.m[i]);
   if (S.ecoef >= 0) {
     C e[CH];
     load_coef<RS, RN, CH>(tb, cbase, M, S.ecoef, ix, e);
@@ -791,11 +791,11 @@ __device__ __forceinline__ void final_chunk(const rks_tableau& tb, const cx<RS>*
     for (int i = 0; i < CH; ++i) acc[i] = e[i] * acc[i];
   }
   for (int j = 0; j < S.nterm; ++j) {
-    const rks_term& tm = S.t[j];
-    const cx<RN>* nl = slotp(tm.src);
+    auto& tm = S.t[j];
+    const cx<RN>* nl = uni(slotp(tm.src));
     C v[CH];
 #pragma unroll
-    for (int i = 0; i < CH; ++i) v[i] = cvt<RS>(nl[ix.m[i]]);
+    for (int i = 0; i < CH; ++i) v[i] = cvt<RS>(gload(nl, ix.m[i]));
     {
       C c[CH];
       if (tm.coef >= 0) {
@@ -849,12 +849,14 @@ __device__ __forceinline__ void final_chunk(const rks_tableau& tb, const cx<RS>*
 // barriers.  Called by all threads; the LDS buffers are free at the call and at the
 // return.
 // ---------------------------------------------------------------------------
-// Modes per chunk of the stage combination of the generic kernels.  Eight FP64 modes with
-// their NL values, coefficients and addresses spill (992 bytes of scratch per lane at n =
-// 8192, four: 352; an ETD34 step 213 us, four: 179).
-template <int MPT, int ES>
+// Modes per chunk of the stage passes of the general kernels.  Eight FP64 modes take all the
+// registers of general_pass and leave nothing to overlap a chunk's loads with; four are faster
+// (eight / four, FP64: ETD34 n = 8192 1.63 / 1.27 ms, ETD5 n = 4096 3.75 / 3.22) except in a
+// one-wave workgroup, where a term costs its latency whatever the chunk holds (MIXED n = 1024,
+// IF45DP: 157 / 172 ms).
+template <int MPT, int ES, int T>
 struct Chunk {
-  static constexpr int MAX = ES > 8 && MPT >= 8 ? 4 : 8;
+  static constexpr int MAX = ES > 8 && MPT >= 8 && T > 64 ? 4 : 8;
   static constexpr int CH = MPT < MAX ? MPT : MAX;
   static constexpr int NCH = (MPT + CH - 1) / CH;
 };
@@ -1077,6 +1079,157 @@ __device__ __forceinline__ void nl_regs(cx<R> (&v)[MPT], cx<R>* buf, const cx<R>
 }
 
 // ---------------------------------------------------------------------------
+// Stage passes of the general kernels, in functions of their own (noinline).  Their term loops
+// are bound by the instructions that walk the tableau; inlined beside the transforms, whose
+// butterflies take every register, they spilled and read the tableau by vector loads.  Here a
+// pass has the registers to itself and reads the tableau by scalar loads, and every array from a
+// uniform base.  One evolve, inlined / like this: FP64 n = 8192 ETD34 1.54 / 1.27 ms, ETD5 6.4 /
+// 4.8, IF45DP 373 / 262; MIXED n = 4096 x 300 2.04 / 1.69, 7.8 / 5.6, 534 / 344; FP32 n = 8192 x
+// 300 3.13 / 2.70, 12.4 / 9.5, 718 / 522.
+// ---------------------------------------------------------------------------
+#define RKS_AS3 __attribute__((address_space(3)))
+
+// what every pass reads (uniform)
+struct PassArgs {
+  const void* ws;       // NL slots
+  const char* cbase;    // coefficients, arrays of stride Mc
+  double h;
+  unsigned smap;
+  int Mc, lim, fold;    // Own
+};
+
+// One stage: its argument (fin: the last stage and the error estimate from one load of each NL
+// value, rks_fused_final) into the LDS buffer at `lds` by mode, the last stage's into cand as
+// well.  Returns the thread's largest |u_new| (fin) or |u_new|^2.
+template <typename R, typename RN, int LOG2N, int T, int NLK>
+__device__ __attribute__((noinline)) double general_pass(const rks_tableau* tbp, int s, int fin, const cx<R>* u,
+                                                         cx<R>* cand, RKS_AS3 unsigned char* lds, PassArgs A) {
+  using C = cx<R>;
+  using CN = cx<RN>;
+  constexpr int N = 1 << LOG2N;
+  constexpr int M = (NLK == NLK_ADVECT) ? N / 2 + 1 : N;
+  using OW = Own<N, M, T, NLK>;
+  using CK = Chunk<OW::MPT, (int)sizeof(C), T>;
+  constexpr int CH = CK::CH;
+  rks_ctab& tb = *rks_uniform_const<rks_ctab>(tbp);
+  s = uni(s);
+  fin = uni(fin);
+  u = uni(u);
+  cand = uni(cand);
+  const unsigned base = (unsigned)uni((int)(unsigned)(unsigned long long)lds);
+  const char* cbase = uni(A.cbase);
+  const unsigned smap = (unsigned)uni((int)A.smap);
+  CN* const slot_base = (CN*)uni((char*)A.ws);
+  const size_t Mc = (size_t)uni(A.Mc);
+  const double h = uni(A.h);
+  OW ow;
+  ow.lim = uni(A.lim);
+  ow.fold = uni(A.fold);
+  ow.t = threadIdx.x;
+  auto slot = [&](int k) -> CN* { return slot_base + (size_t)((smap >> (4 * k)) & 15u) * M; };
+  auto put = [&](int m, C v) {
+    typedef typename GVec<R>::t V;
+    V w;
+    w.x = v.re;
+    w.y = v.im;
+    ((RKS_AS3 V*)base)[m] = w;
+  };
+  auto& S = tb.st[s];
+  const bool last = s == tb.nstage - 1;
+  double mx = 0.0;
+#pragma unroll 1
+  for (int c = 0; c < CK::NCH; ++c) {
+    const ChunkIdx<CH> ix = pass_chunk<N, M, T, NLK, CH>(c, ow.fresh());
+    C acc[CH];
+    if (fin) {
+      C ev[CH];
+      final_chunk<R, RN, CH>(tb, u, slot, cbase, Mc, ix, h, acc, ev);
+#pragma unroll
+      for (int i = 0; i < CH; ++i) {
+        if (!ix.ok[i]) continue;
+        gstore(cand, ix.m[i], acc[i]);
+        const double a = hypot((double)acc[i].re, (double)acc[i].im);
+        const double er = (double)ev[i].re, ei = (double)ev[i].im;
+        mx = nanmax(mx, a);
+        // FP64 keeps |err|^2; an FP32 buffer keeps |err| (|err|^2 would flush to zero
+        // below ~1e-19 and turn a real error into an unconditional accept)
+        if constexpr (sizeof(R) == sizeof(double)) put(ix.m[i], mkc((R)a, (R)(er * er + ei * ei)));
+        else put(ix.m[i], mkc((R)a, (R)hypot(er, ei)));
+      }
+    } else {
+      stage_chunk<R, RN, CH>(tb, S, u, slot, cbase, Mc, ix, h, acc);
+#pragma unroll
+      for (int i = 0; i < CH; ++i) {
+        if (!ix.ok[i]) continue;
+        if (last) {
+          gstore(cand, ix.m[i], acc[i]);
+          if (tb.adaptive)
+            mx = nanmax(mx, (double)acc[i].re * (double)acc[i].re + (double)acc[i].im * (double)acc[i].im);
+        }
+        put(ix.m[i], acc[i]);
+      }
+    }
+  }
+  return mx;
+}
+
+// The thread's masked sums of the error norm where the last stage has an NL (NormOrder):
+// modes with lim < |u_new|^2 <= DBL_MAX.
+struct NormSums {
+  double su, se;
+};
+template <typename R, typename RN, int LOG2N, int T, int NLK>
+__device__ __attribute__((noinline)) NormSums general_error(const rks_tableau* tbp, const cx<R>* cand, double lim,
+                                                            PassArgs A) {
+#pragma clang fp contract(off)
+  using C = cx<R>;
+  using CN = cx<RN>;
+  constexpr int N = 1 << LOG2N;
+  constexpr int M = (NLK == NLK_ADVECT) ? N / 2 + 1 : N;
+  using OW = Own<N, M, T, NLK>;
+  constexpr int CH = Chunk<OW::MPT, (int)sizeof(C), T>::CH;
+  using NO = NormOrder<N, M, T, NLK>;
+  constexpr int NCH = (NO::SLOTS + CH - 1) / CH;
+  rks_ctab& tb = *rks_uniform_const<rks_ctab>(tbp);
+  cand = uni(cand);
+  lim = uni(lim);
+  const char* cbase = uni(A.cbase);
+  const unsigned smap = (unsigned)uni((int)A.smap);
+  CN* const slot_base = (CN*)uni((char*)A.ws);
+  const size_t Mc = (size_t)uni(A.Mc);
+  const double h = uni(A.h);
+  OW ow;
+  ow.lim = uni(A.lim);
+  ow.fold = uni(A.fold);
+  ow.t = threadIdx.x;
+  auto slot = [&](int k) -> CN* { return slot_base + (size_t)((smap >> (4 * k)) & 15u) * M; };
+  NormSums n = {0.0, 0.0};
+#pragma unroll 1
+  for (int c = 0; c < NCH; ++c) {
+    ChunkIdx<CH> ix = pass_chunk<N, M, T, NLK, CH>(c, ow.fresh());
+#pragma unroll
+    for (int i = 0; i < CH; ++i) {
+      ix.ok[i] = NO::ok(c * CH + i, ow.lim);
+      ix.m[i] = ix.ok[i] ? NO::mode(c * CH + i) : 0;
+    }
+    C ev[CH];
+    error_chunk<R, RN, CH>(tb, slot, cbase, Mc, ix, h, ev);
+#pragma unroll
+    for (int i = 0; i < CH; ++i) {
+      if (!ix.ok[i]) continue;
+      const C kv = gload(cand, ix.m[i]);
+      const double kr = (double)kv.re, ki = (double)kv.im, er = (double)ev[i].re, ei = (double)ev[i].im;
+      const double a = fma(kr, kr, ki * ki);
+      if (a > lim && a <= __DBL_MAX__) {
+        n.su += a;
+        n.se += fma(er, er, ei * ei);
+      }
+    }
+  }
+  return n;
+}
+
+// ---------------------------------------------------------------------------
 // learned step-size proposer: features of an accepted state, the training
 // record, and the proposal that replaces the controller's next step
 // ---------------------------------------------------------------------------
@@ -1210,7 +1363,6 @@ __device__ int run_instance(const rks_launch& P, int idx, cx<R>* buf, const cx<R
   constexpr int M = (NLK == NLK_ADVECT) ? N / 2 + 1 : N;
   using OW = Own<N, M, T, NLK>;
   constexpr int MPT = OW::MPT;
-  constexpr int CH = Chunk<MPT, (int)sizeof(C)>::CH;
   constexpr bool METHOD = METH != RKS_METH_ANY;
   constexpr bool PAIRED = !METHOD && M == N && NLK != NLK_HANKEL;  // pass_chunk: other modes than the transforms'
   using TT = MethodTab<METHOD ? METH : 0, (int)sizeof(C), (int)sizeof(CN), NLK == NLK_ADVECT>;
@@ -1294,7 +1446,7 @@ __device__ int run_instance(const rks_launch& P, int idx, cx<R>* buf, const cx<R
     h_coeff = __builtin_nan("");
     smap = 0x76543210u;
   }
-  const bool adaptive = METHOD ? TT::tab.adaptive != 0 : tb.adaptive != 0;
+  const bool adaptive = METHOD ? TT::tab.adaptive != 0 : uni(tb.adaptive) != 0;
   const bool evolve = (P.mode == RKS_MODE_EVOLVE);
   if (reenter) {
     // back from the proposer: h_next holds its proposal (solveras.py:638-641)
@@ -1334,10 +1486,11 @@ __device__ int run_instance(const rks_launch& P, int idx, cx<R>* buf, const cx<R
   }
 
   auto slot = [&](int s) -> CN* { return slot_base + (size_t)((smap >> (4 * s)) & 15u) * M; };
+  auto pass_args = [&]() { return PassArgs{ws, cbase, h, smap, Mc, ow.lim, ow.fold}; };
   auto cur_u = [&]() -> const C* { return ubuf < 0 ? uin : (const C*)(ubuf == 0 ? cand0 : cand1); };
-  const bool fused = METHOD ? FUSED : rks_fused_final(tb);
-  const bool recompute = (METHOD ? TT::tab.nl1_policy : tb.nl1_policy) == RKS_NL1_RECOMPUTE;
-  const int nstage = METHOD ? TT::tab.nstage : tb.nstage;
+  const bool fused = METHOD ? FUSED : uni((int)rks_fused_final(tb)) != 0;
+  const bool recompute = (METHOD ? TT::tab.nl1_policy : uni(tb.nl1_policy)) == RKS_NL1_RECOMPUTE;
+  const int nstage = METHOD ? TT::tab.nstage : uni(tb.nstage);
 
   bool done = false;
   int pending = 0;      // proposer variant: stopped after an accept for the proposer
@@ -1376,7 +1529,7 @@ __device__ int run_instance(const rks_launch& P, int idx, cx<R>* buf, const cx<R
         if (recompute) {
           first_nl = true;
         } else {
-          const unsigned f4 = 4u * (unsigned)(METHOD ? TT::tab.fsal_slot : tb.fsal_slot);
+          const unsigned f4 = 4u * (unsigned)(METHOD ? TT::tab.fsal_slot : uni(tb.fsal_slot));
           const unsigned a = smap & 15u, b = (smap >> f4) & 15u;
           smap = (smap & ~(15u | (15u << f4))) | b | (a << f4);
         }
@@ -1387,78 +1540,53 @@ __device__ int run_instance(const rks_launch& P, int idx, cx<R>* buf, const cx<R
 #pragma unroll
       for (int k = 0; k < MPT; ++k) nv[k] = mkc((RN)0, (RN)0);
 #pragma unroll 1
-      for (int s = first_nl ? -1 : 0; s < nstage; ++s) {
+      for (int s = uni(first_nl ? -1 : 0); s < nstage; ++s) {
         const bool last = s == nstage - 1;
         C v[MPT];
         int ns = 0;  // NL slot this pass writes
-        if (s < 0) {
-          load_modes(v, u);
-        } else if constexpr (METHOD) {
-          if (FUSED && last) break;
-          stage_switch<TT, 0, true>(s, v, nv, u, ow, slot, cbase, (size_t)Mc, h);
-          if (!FUSED && last) {
+        if constexpr (METHOD) {
+          if (s < 0) {
+            load_modes(v, u);
+          } else {
+            if (FUSED && last) break;
+            stage_switch<TT, 0, true>(s, v, nv, u, ow, slot, cbase, (size_t)Mc, h);
+            if (!FUSED && last) {
 #pragma unroll
-            for (int k = 0; k < MPT; ++k) {
-              if (ow.ok(k)) {
-                gstore(cand, ow.m(k), v[k]);
-                if (TT::tab.adaptive)
-                  mx = nanmax(mx, (double)v[k].re * (double)v[k].re + (double)v[k].im * (double)v[k].im);
-              }
-            }
-          }
-          static_assert(TT::tab.st[0].nl_slot == 1 && LAST_SLOT == TT::tab.nslot - 1, "stage s writes slot s + 1");
-          ns = s + 1;
-        } else {
-          const rks_stage& S = tb.st[s];
-          if (last && fused) {
-            // per-mode |u_new| and |err|^2 (FP32 buffer: |err|) wait in the idle LDS buffer
-#pragma unroll 1
-            for (int c = 0; c < Chunk<MPT, (int)sizeof(C)>::NCH; ++c) {
-              const ChunkIdx<CH> ix = pass_chunk<N, M, T, NLK, CH>(c, ow.fresh());
-              C acc[CH], ev[CH];
-              final_chunk<R, RN, CH>(tb, u, slot, cbase, (size_t)Mc, ix, h, acc, ev);
-#pragma unroll
-              for (int i = 0; i < CH; ++i) {
-                const int m = ix.m[i];
-                if (ix.ok[i]) {
-                  cand[m] = acc[i];
-                  const double a = hypot((double)acc[i].re, (double)acc[i].im);
-                  const double er = (double)ev[i].re, ei = (double)ev[i].im;
-                  mx = nanmax(mx, a);
-                  // FP64 keeps |err|^2; an FP32 buffer keeps |err| (|err|^2 would flush to zero
-                  // below ~1e-19 and turn a real error into an unconditional accept)
-                  if constexpr (sizeof(R) == sizeof(double)) buf[m] = mkc((R)a, (R)(er * er + ei * ei));
-                  else buf[m] = mkc((R)a, (R)hypot(er, ei));
+              for (int k = 0; k < MPT; ++k) {
+                if (ow.ok(k)) {
+                  gstore(cand, ow.m(k), v[k]);
+                  if (TT::tab.adaptive)
+                    mx = nanmax(mx, (double)v[k].re * (double)v[k].re + (double)v[k].im * (double)v[k].im);
                 }
               }
             }
-            break;
+            static_assert(TT::tab.st[0].nl_slot == 1 && LAST_SLOT == TT::tab.nslot - 1, "stage s writes slot s + 1");
+            ns = s + 1;
           }
-          // the stage argument through the LDS buffer: the run-time term loop stays rolled over
-          // the chunks, and the transforms' modes may be other threads'
-#pragma unroll 1
-          for (int c = 0; c < Chunk<MPT, (int)sizeof(C)>::NCH; ++c) {
-            const ChunkIdx<CH> ix = pass_chunk<N, M, T, NLK, CH>(c, ow.fresh());
-            C acc[CH];
-            stage_chunk<R, RN, CH>(tb, S, u, slot, cbase, (size_t)Mc, ix, h, acc);
+        } else {
+          // the argument through the LDS buffer, u itself too: loaded into v here, it would be
+          // held through the call of the other branch
+          bool has_nl = true;
+          if (s < 0) {
+            const OW of = ow.fresh();
 #pragma unroll
-            for (int i = 0; i < CH; ++i) {
-              if (!ix.ok[i]) continue;
-              if (last) {
-                cand[ix.m[i]] = acc[i];
-                if (adaptive)
-                  mx = nanmax(mx, (double)acc[i].re * (double)acc[i].re + (double)acc[i].im * (double)acc[i].im);
-              }
-              buf[ix.m[i]] = acc[i];
-            }
+            for (int k = 0; k < MPT; ++k)
+              if (of.ok(k)) buf[of.m(k)] = gload(u, of.m(k));
+          } else {
+            const bool fin = last && fused;
+            const double m = general_pass<R, RN, LOG2N, T, NLK>(tbp, s, fin, u, cand, (RKS_AS3 unsigned char*)buf,
+                                                                pass_args());
+            if (last) mx = m;
+            if (fin) break;
+            has_nl = uni(tb.st[s].has_nl) != 0;
+            ns = uni(tb.st[s].nl_slot);
           }
           if constexpr (PAIRED) __syncthreads();  // buf, and cand for what copies it
-          if (!S.has_nl) continue;
+          if (!has_nl) continue;
           const OW of = ow.fresh();
 #pragma unroll
           for (int k = 0; k < MPT; ++k) v[k] = buf[of.m(k)];
           __syncthreads();
-          ns = S.nl_slot;
         }
         nl_regs<R, LOG2N, T, NLK>(v, buf, twl, nlc, kx, Mr, hs);
         ++nl_calls;
@@ -1549,37 +1677,21 @@ __device__ int run_instance(const rks_launch& P, int idx, cx<R>* buf, const cx<R
         const double lim = fused ? cut * mx : (cut < 0.0 ? -1.0 : cut * cut * mx);
         __syncthreads();  // every thread's last NL values, candidate and buffer values
         using NO = NormOrder<N, M, T, NLK>;
-        constexpr int NCH = (NO::SLOTS + CH - 1) / CH;
+        if (fused) {
 #pragma unroll 1
-        for (int c = 0; c < NCH; ++c) {
-          ChunkIdx<CH> ix = pass_chunk<N, M, T, NLK, CH>(c, ow.fresh());
-#pragma unroll
-          for (int i = 0; i < CH; ++i) {
-            ix.ok[i] = NO::ok(c * CH + i, ow.lim);
-            ix.m[i] = ix.ok[i] ? NO::mode(c * CH + i) : 0;
-          }
-          C ev[CH];
-          if (!fused) error_chunk<R, RN, CH>(tb, slot, cbase, (size_t)Mc, ix, h, ev);
-#pragma unroll
-          for (int i = 0; i < CH; ++i) {
-            if (!ix.ok[i]) continue;
-            if (fused) {
-              const C q = buf[ix.m[i]];
-              const double a = (double)q.re, e = (double)q.im;
-              if (a > lim && a <= __DBL_MAX__) {
-                su = fma(a, a, su);
-                se = sizeof(R) < sizeof(double) ? fma(e, e, se) : se + e;
-              }
-            } else {
-              const C kv = cand[ix.m[i]];
-              const double kr = (double)kv.re, ki = (double)kv.im, er = (double)ev[i].re, ei = (double)ev[i].im;
-              const double a = fma(kr, kr, ki * ki);
-              if (a > lim && a <= __DBL_MAX__) {
-                su += a;
-                se += fma(er, er, ei * ei);
-              }
+          for (int k = 0; k < NO::SLOTS; ++k) {
+            if (!NO::ok(k, ow.lim)) continue;
+            const C q = buf[NO::mode(k)];
+            const double a = (double)q.re, e = (double)q.im;
+            if (a > lim && a <= __DBL_MAX__) {
+              su = fma(a, a, su);
+              se = sizeof(R) < sizeof(double) ? fma(e, e, se) : se + e;
             }
           }
+        } else {
+          const NormSums n = general_error<R, RN, LOG2N, T, NLK>(tbp, cand, lim, pass_args());
+          su = n.su;
+          se = n.se;
         }
         if (fused) __syncthreads();  // the buffer's values are read
       }
