@@ -730,7 +730,9 @@ int rks_dense_coeffs_ws(int method, int n, int batch, const void* L, const doubl
     S.E = E;
     S.Q = Q;
     const int lds = 6 * (int)(nn * sizeof(z64));
-    e = hipFuncSetAttribute((const void*)dense_small, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    // the limit of every size: another thread may be between its own call and launch
+    e = hipFuncSetAttribute((const void*)dense_small, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            6 * DSMALL * DSMALL * (int)sizeof(z64));
     if (e != hipSuccess) return dfail(RKS_ERR_HIP, std::string("rks_dense_coeffs: ") + hipGetErrorString(e));
     hipLaunchKernelGGL(dense_small, dim3(S.npts + 1, nf, batch), dim3(DT), lds, stream, S);
   } else {
