@@ -24,12 +24,16 @@ struct rks2_ctx {
 template <typename R, typename RN, int LOG2, int METH>
 struct Eng2 {
   using G = Geo2<R, LOG2>;
+  // a last stage that forms the error estimate too exists (rks_fused_final; IF34's has an NL)
+  static constexpr bool FUSES = METH != RKS_M_IF34;
   static hipError_t setup() {
     hipError_t e = hipFuncSetAttribute((const void*)k2_col<R, RN, LOG2, false, METH>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, G::COL_LDS);
-    if (e == hipSuccess)
-      e = hipFuncSetAttribute((const void*)k2_col<R, RN, LOG2, true, METH>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              G::COL_LDS);
+    if constexpr (FUSES) {
+      if (e == hipSuccess)
+        e = hipFuncSetAttribute((const void*)k2_col<R, RN, LOG2, true, METH>,
+                                hipFuncAttributeMaxDynamicSharedMemorySize, G::COL_LDS);
+    }
     if (e != hipSuccess) return e;
     return hipFuncSetAttribute((const void*)k2_row<R, LOG2>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                G::ROW_LDS);
@@ -37,12 +41,15 @@ struct Eng2 {
   static int ncg() { return G::NCG; }
   static int nnb() { return G::NNB; }
   static void col(const rks2_launch& L, hipStream_t s, int fwd, int cond, int arg, int prelude, bool fuse = false) {
-    if (fuse)
-      hipLaunchKernelGGL((k2_col<R, RN, LOG2, true, METH>), dim3(G::NCG, L.ninst), dim3(G::CT), G::COL_LDS, s, L, fwd,
-                         cond, arg, prelude);
-    else
-      hipLaunchKernelGGL((k2_col<R, RN, LOG2, false, METH>), dim3(G::NCG, L.ninst), dim3(G::CT), G::COL_LDS, s, L, fwd,
-                         cond, arg, prelude);
+    if constexpr (FUSES) {
+      if (fuse) {
+        hipLaunchKernelGGL((k2_col<R, RN, LOG2, true, METH>), dim3(G::NCG, L.ninst), dim3(G::CT), G::COL_LDS, s, L,
+                           fwd, cond, arg, prelude);
+        return;
+      }
+    }
+    hipLaunchKernelGGL((k2_col<R, RN, LOG2, false, METH>), dim3(G::NCG, L.ninst), dim3(G::CT), G::COL_LDS, s, L, fwd,
+                       cond, arg, prelude);
   }
   static void row(const rks2_launch& L, hipStream_t s, int prelude) {
     hipLaunchKernelGGL((k2_row<R, LOG2>), dim3(G::NRG, L.ninst), dim3(G::RT), G::ROW_LDS, s, L, prelude);

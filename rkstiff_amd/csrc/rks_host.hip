@@ -802,7 +802,7 @@ static std::vector<LaunchPart> launch_parts(const rks_plan* p) {
   return v;
 }
 
-static int launch_all(rks_plan* p, int mode, double h_mode, hipStream_t stream) {
+static int launch_all(rks_plan* p, int mode, hipStream_t stream) {
   if (p->c2) {
     const hipError_t e = rks2_run(p->c2, p->tab, mode, p->store_freq > 0, stream);
     if (e != hipSuccess) return fail(RKS_ERR_HIP, std::string("2-D engine: ") + hipGetErrorString(e));
@@ -815,7 +815,6 @@ static int launch_all(rks_plan* p, int mode, double h_mode, hipStream_t stream) 
   L.inst = p->d_inst;
   L.io = p->d_io;
   L.mode = mode;
-  L.h_mode = h_mode;
   const std::vector<LaunchPart> parts = launch_parts(p);
   const size_t np = parts.size();
   const bool learn = learns(p);
@@ -917,14 +916,14 @@ int rks_evolve(rks_plan* p, const void* const* u0, void* const* uf, const double
   }
   int rc = upload_io(p, u0, uf, t0, tf, h, 1, 0, stream);
   if (rc) return rc;
-  return launch_all(p, RKS_MODE_EVOLVE, 0.0, stream);
+  return launch_all(p, RKS_MODE_EVOLVE, stream);
 }
 
 int rks_resume(rks_plan* p, hipStream_t stream) {
   if (!p) return fail(RKS_ERR_INVALID, "null plan");
   int rc = upload_io(p, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 1, stream);
   if (rc) return rc;
-  return launch_all(p, RKS_MODE_EVOLVE, 0.0, stream);
+  return launch_all(p, RKS_MODE_EVOLVE, stream);
 }
 
 int rks_step(rks_plan* p, const void* const* u, void* const* u_new, const double* h, hipStream_t stream) {
@@ -934,7 +933,7 @@ int rks_step(rks_plan* p, const void* const* u, void* const* u_new, const double
     if (!(h && h[i] >= 0.0)) return fail(RKS_ERR_INVALID, "step size must be >= 0");
   int rc = upload_io(p, u, u_new, nullptr, nullptr, h, 0, 0, stream);
   if (rc) return rc;
-  return launch_all(p, RKS_MODE_STEP, 0.0, stream);
+  return launch_all(p, RKS_MODE_STEP, stream);
 }
 
 int rks_reset(rks_plan* p, hipStream_t stream) {
@@ -959,7 +958,7 @@ int rks_nl_eval(rks_plan* p, const void* const* u, void* const* nl_out, hipStrea
   if (p->nlk == RKS_NL_NONE) return fail(RKS_ERR_INVALID, "no built-in nonlinearity");
   int rc = upload_io(p, u, nl_out, nullptr, nullptr, nullptr, 0, 0, stream);
   if (rc) return rc;
-  return launch_all(p, RKS_MODE_NL, 0.0, stream);
+  return launch_all(p, RKS_MODE_NL, stream);
 }
 
 int rks_coeffs(rks_plan* p, int inst, double h, void* dst, hipStream_t stream) {

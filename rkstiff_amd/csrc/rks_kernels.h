@@ -46,7 +46,6 @@ struct rks_launch {
   int mode;
   int* queue;      // next item, or null where the grid has a workgroup per trajectory
   const void* tw;  // exp(-2 pi i x / N), x < N, engine precision
-  double h_mode;   // RKS_MODE_COEFFS
   rks_mlp_dev mlp; // learned step-size proposer (mlp.on = 0: the reference's controller only)
 };
 

@@ -5,7 +5,7 @@
 // for every stage the linear combination k = E .* u + sum_j scale_j h^p_j C_j .* NL_j
 // that feeds the nonlinear term.  All seven diagonal methods of the reference
 // (etd35.py, etd34.py, etd4.py, etd5.py, if34.py, if45dp.py, if4.py) are
-// encoded as tableaux in rks_tableau.cpp; the kernels are method-agnostic.
+// encoded as tableaux in rks_tableau.h; the kernels read them, or (ETD35, IF34) are compiled for one.
 #pragma once
 #include <stdint.h>
 
@@ -54,7 +54,6 @@
 #define RKS_MODE_EVOLVE 0
 #define RKS_MODE_STEP 1
 #define RKS_MODE_NL 2      // NL = nl(u) only
-#define RKS_MODE_COEFFS 3  // coefficient arrays at h only
 
 // One term of a stage combination, in the reference's grouping:
 //   inner = NL[src] + scale2 * NL[src2]                      (src2 < 0: inner = NL[src])
