@@ -169,10 +169,14 @@ int rks_error_s(rks_plan* p, int inst, const void* u_new, const void* err, doubl
  * twice its threads (n = 512 .. 4096; without a proposer or records also the cubic
  * n = 8192), 2 four times (n = 1024 and the cubic n = 2048, without a proposer or
  * records; these, attached later, bring the base tile back), -1 (also tile NULL, as
- * before the first call) the library's choice by size, precision and number of
- * trajectories: the base tile with a proposer, records or an attempt log.  Results
- * do not depend on the shape or, beyond rounding, the tile.
- * rks_plan_tiles: the tile each bucket (up to cap) runs on now (0, 1 or 2). */
+ * before the first call) the library's choice.  That is a wider tile for FP64
+ * trajectories of n >= 512, by their own size, method and (advective term) damping at
+ * the grid's end, whatever else is in the plan; the base tile in other precisions and
+ * while a proposer, records or an attempt log are attached.  Results do not depend on
+ * the shape; another tile rounds in another order, so an FP64 run with a log repeats
+ * the run without one to rounding, and bit for bit where both set the same tile.
+ * rks_plan_tiles: the tile each bucket (up to cap) runs on now (0, 1 or 2; where only
+ * some of its trajectories keep the base tile for lack of damping, the others'). */
 int rks_plan_buckets(rks_plan* p, int* nbucket, int* log2n, int* count, int* max_wg_per_cu, int* ntile, int cap);
 int rks_plan_set_launch(rks_plan* p, int concurrent, const int* wg_per_cu, const int* tile, int nbucket);
 int rks_plan_tiles(rks_plan* p, int* tile, int cap);

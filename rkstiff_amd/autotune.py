@@ -1,7 +1,8 @@
 """Launch-shape autotuner for the persistent stepping kernels.
 
 A plan groups its trajectories in size buckets, one persistent-kernel launch
-per bucket.  Two launch choices change throughput and not results:
+per bucket.  Three launch choices change throughput, and results by rounding
+at most (the tile):
 
 * whether the buckets run one after another on the caller's stream or
   overlap on private streams.  In a mixed-size ensemble a bucket's last
@@ -19,8 +20,8 @@ keeps the fastest shape.  Finally each bucket's trajectories are ordered by
 the attempts they took in a pilot over the whole interval, most first, so
 the longest trajectories start first and a bucket's tail stays short
 (longest-processing-time-first; trajectories of one bucket differ mainly in
-their step counts).  Order and shape change throughput, never results.  The per-bucket choices (the second tile, then half
-and a quarter of the resident workgroups) are timed on pilots in which only
+their step counts).  The per-bucket choices (another tile than the library's,
+then half and a quarter of the resident workgroups) are timed on pilots in which only
 that bucket's trajectories move (the others get tf = t0, which leaves them
 untouched), so one bucket's choice is not lost in the noise of the others;
 a choice that wins there is kept only if the whole ensemble, buckets

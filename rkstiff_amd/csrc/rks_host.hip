@@ -168,11 +168,13 @@ namespace {
 typedef rks_kernel_entry KernelEntry;
 
 // Which stepping kernel runs a plan: the one compiled for its method where that exists, else
-// the one that reads the tableau.  ETD35 and IF34 are the methods of every workload; their
-// kernels are compiled for lin_ops of one kind (real with the advective and the rfft2 terms,
-// complex with the cubic ones) and read every L of the plan so.  A complex lin_op with the
+// the one that reads the tableau.  ETD35 and IF34 are the methods of the benchmark's workloads;
+// their kernels are compiled for lin_ops of one kind (real with the advective and the rfft2
+// terms, complex with the cubic ones) and read every L of the plan so.  A complex lin_op with the
 // advective term (KdV), a real one with a cubic term, or a plan that holds both kinds takes the
-// general kernel, which reads each trajectory's kind.
+// general kernel, which reads each trajectory's kind.  IF34 with the Hankel term is not compiled
+// either: its general kernel takes 1.19 ms for one beam of nr = 100 and 3.00 for 1024, one of its
+// own 0.79 and 2.56, and the radial runs use ETD35.
 int method_variant(int method, int nlk, int n_complex, int ninst) {
   const bool real = nlk == RKS_NL_ADVECT_RFFT || nlk == RKS_NL_AC2D_RFFT2;
   if (n_complex != (real ? 0 : ninst)) return RKS_METH_ANY;

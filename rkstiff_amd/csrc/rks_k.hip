@@ -7,7 +7,8 @@
 // The proposer variant exists for the sizes whose workgroups can be whole waves (n >= 128;
 // the host refuses smaller rfft grids), the second tile for n = 2^9 .. 2^12, with and
 // without the proposer.  Without it also (rks_host.hip default_tile) twice the threads for
-// the cubic n = 2^13, four times for n = 2^10 and the cubic n = 2^11.  The Hankel kind has the size classes 2^4 .. 2^10 and one tile.
+// the cubic n = 2^13, four times for n = 2^10 and the cubic n = 2^11.  The Hankel kind has the
+// size classes 2^4 .. 2^10 and one tile.
 #include "rks_kernels.h"
 
 namespace {

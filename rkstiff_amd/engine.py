@@ -163,7 +163,7 @@ class Plan:
 
     def tiles(self):
         """The FFT tile each size bucket runs on: as set by ``set_launch``, else by size,
-        precision and number of trajectories (rks_plan_set_launch)."""
+        method and precision (rks_plan_set_launch)."""
         nb = len(self.buckets())
         arr = (ctypes.c_int * max(nb, 1))()
         _lib.check(self.lib.rks_plan_tiles(self.h, arr, nb))

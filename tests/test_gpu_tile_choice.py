@@ -104,3 +104,22 @@ def test_result_does_not_depend_on_the_rest_of_the_plan(kind, n):
         mixed, tiles = run(which, cost)
         assert tiles == own
         assert all(torch.equal(x, b if w else a) for x, w in zip(mixed, which))
+
+
+@pytest.mark.parametrize("kind,n", [("advect", 1024), ("cubic", 2048)])
+def test_logged_run_on_the_same_tile_has_the_same_bits(kind, n):
+    from rkstiff_amd import _lib
+    plan = _plan(kind, n)
+    x = np.arange(n) / n
+    u = np.fft.fft(np.exp(-200 * (x - 0.5) ** 2)) if kind == "cubic" else np.fft.rfft(np.cos(2 * np.pi * x))
+    ut = torch.as_tensor(u).cuda()
+    uf = [torch.empty_like(ut) for _ in range(2)]
+    own = plan.tiles()
+    for out, log in zip(uf, (0, 64)):
+        if log:
+            plan.set_launch(tile=own)
+            plan.set_storage(0, 0, log)
+        assert plan.tiles() == own
+        plan.evolve([ut], [out], [0.0], [0.2], [0.02])
+        assert plan.stats()[0]["status"] == _lib.RKS_OK
+    assert torch.equal(uf[0], uf[1])
