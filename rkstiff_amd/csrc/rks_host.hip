@@ -173,7 +173,7 @@ typedef rks_kernel_entry KernelEntry;
 // terms, complex with the cubic ones) and read every L of the plan so.  A complex lin_op with the
 // advective term (KdV), a real one with a cubic term, or a plan that holds both kinds takes the
 // general kernel, which reads each trajectory's kind.  IF34 with the Hankel term is not compiled
-// either: its general kernel takes 1.19 ms for one beam of nr = 100 and 3.00 for 1024, one of its
+// either: its general kernel takes 1.10 ms for one beam of nr = 100 and 2.95 for 1024, one of its
 // own 0.79 and 2.56, and the radial runs use ETD35.
 int method_variant(int method, int nlk, int n_complex, int ninst) {
   const bool real = nlk == RKS_NL_ADVECT_RFFT || nlk == RKS_NL_AC2D_RFFT2;

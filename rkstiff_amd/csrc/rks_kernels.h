@@ -588,11 +588,39 @@ struct NormOrder {
   static __device__ __forceinline__ bool ok(int k, int lim) { return (int)threadIdx.x < NT && mode(k) < lim; }
 };
 
+// How a pass reads its arrays.  Through the scalar view of the tableau (rks_ctab: the general
+// passes below) the array's base is uniform, kept in scalar registers and indexed by 32 bits;
+// with a plain tableau an array is read as the pointer stands.
+template <typename TB>
+struct ViewOf {
+  static constexpr bool SCALAR = false;
+};
+template <>
+struct ViewOf<rks_ctab> {
+  static constexpr bool SCALAR = true;
+};
+template <bool SCALAR, typename P>
+__device__ __forceinline__ P* view(P* p) {
+  if constexpr (SCALAR) return uni(p);
+  else return p;
+}
+template <bool SCALAR, typename R>
+__device__ __forceinline__ cx<R> vload(const cx<R>* p, int i) {
+  if constexpr (SCALAR) return gload(p, i);
+  else return p[i];
+}
+template <bool SCALAR, typename R>
+__device__ __forceinline__ R vload_real(const R* p, int i) {
+  if constexpr (SCALAR) return gload_real(p, i);
+  else return p[i];
+}
+
 // coefficient array c of the chunk's modes; M is the array stride (modes)
 template <typename RS, typename RN, int CH, typename TB>
 __device__ __forceinline__ void load_coef(TB& tb, const char* cbase, size_t M, int c,
                                           const ChunkIdx<CH>& ix, cx<RS> (&w)[CH]) {
-  const char* q = uni(cbase + (size_t)tb.coef_off[c] * M);
+  constexpr bool SC = ViewOf<TB>::SCALAR;
+  const char* q = view<SC>(cbase + (size_t)tb.coef_off[c] * M);
   const int kind = tb.coef_rs[c];
   // Mirror pairs: FP32-state kernels issue one load per pair (plus the n/2
   // partner of q = 0).  The FP64-state kernels have no registers to spare
@@ -629,16 +657,16 @@ __device__ __forceinline__ void load_coef(TB& tb, const char* cbase, size_t M, i
   };
   if (kind == RKS_CST_RS) {
     const cx<RS>* p = (const cx<RS>*)q;
-    gather([&](int m) { return gload(p, m); });
+    gather([&](int m) { return vload<SC>(p, m); });
   } else if (kind == RKS_CST_RN) {
     const cx<RN>* p = (const cx<RN>*)q;
-    gather([&](int m) { return cvt<RS>(gload(p, m)); });
+    gather([&](int m) { return cvt<RS>(vload<SC>(p, m)); });
   } else if (kind == RKS_CST_RS_REAL) {
     const RS* p = (const RS*)q;
-    gather([&](int m) { return mkc(gload_real(p, m), (RS)0); });
+    gather([&](int m) { return mkc(vload_real<SC>(p, m), (RS)0); });
   } else {
     const RN* p = (const RN*)q;
-    gather([&](int m) { return mkc((RS)gload_real(p, m), (RS)0); });
+    gather([&](int m) { return mkc((RS)vload_real<SC>(p, m), (RS)0); });
   }
 }
 
@@ -648,17 +676,18 @@ __device__ __forceinline__ void add_terms(TB& tb, TM* terms, int nterm, SlotF sl
                                           const char* cbase, size_t M, const ChunkIdx<CH>& ix, double h,
                                           cx<RS> (&acc)[CH]) {
   using C = cx<RS>;
+  constexpr bool SC = ViewOf<TB>::SCALAR;
   for (int j = 0; j < nterm; ++j) {
     auto& tm = terms[j];
-    const cx<RN>* nl = uni(slotp(tm.src));
+    const cx<RN>* nl = view<SC>(slotp(tm.src));
     C v[CH];
 #pragma unroll
-    for (int i = 0; i < CH; ++i) v[i] = cvt<RS>(gload(nl, ix.m[i]));
+    for (int i = 0; i < CH; ++i) v[i] = cvt<RS>(vload<SC>(nl, ix.m[i]));
     if (tm.src2 >= 0) {
-      const cx<RN>* nl2 = uni(slotp(tm.src2));
+      const cx<RN>* nl2 = view<SC>(slotp(tm.src2));
       const RS s2 = (RS)tm.scale2;
 #pragma unroll
-      for (int i = 0; i < CH; ++i) v[i] = v[i] + s2 * cvt<RS>(gload(nl2, ix.m[i]));
+      for (int i = 0; i < CH; ++i) v[i] = v[i] + s2 * cvt<RS>(vload<SC>(nl2, ix.m[i]));
     }
     if (tm.hmode == 2) {
       const RS hs = (RS)((tm.scale * h) / tm.den);
@@ -698,8 +727,9 @@ __device__ __forceinline__ void stage_chunk(TB& tb, ST& S, const cx<RS>* __restr
                                             SlotF slotp, const char* cbase, size_t M, const ChunkIdx<CH>& ix,
                                             double h, cx<RS> (&acc)[CH]) {
   using C = cx<RS>;
+  constexpr bool SC = ViewOf<TB>::SCALAR;
 #pragma unroll
-  for (int i = 0; i < CH; ++i) acc[i] = gload(u, ix.m[i]);
+  for (int i = 0; i < CH; ++i) acc[i] = vload<SC>(u, ix.m[i]);
   if (S.ecoef >= 0) {
     C e[CH];
     load_coef<RS, RN, CH>(tb, cbase, M, S.ecoef, ix, e);
@@ -780,9 +810,10 @@ __device__ __forceinline__ void final_chunk(TB& tb, const cx<RS>* __restrict__ u
                                             const char* cbase, size_t M, const ChunkIdx<CH>& ix, double h,
                                             cx<RS> (&acc)[CH], cx<RS> (&ev)[CH]) {
   using C = cx<RS>;
+  constexpr bool SC = ViewOf<TB>::SCALAR;
   auto& S = tb.st[tb.nstage - 1];
 #pragma unroll
-  for (int i = 0; i < CH; ++i) acc[i] = gload(u, ix.m[i]);
+  for (int i = 0; i < CH; ++i) acc[i] = vload<SC>(u, ix.m[i]);
   if (S.ecoef >= 0) {
     C e[CH];
     load_coef<RS, RN, CH>(tb, cbase, M, S.ecoef, ix, e);
@@ -791,10 +822,10 @@ __device__ __forceinline__ void final_chunk(TB& tb, const cx<RS>* __restrict__ u
   }
   for (int j = 0; j < S.nterm; ++j) {
     auto& tm = S.t[j];
-    const cx<RN>* nl = uni(slotp(tm.src));
+    const cx<RN>* nl = view<SC>(slotp(tm.src));
     C v[CH];
 #pragma unroll
-    for (int i = 0; i < CH; ++i) v[i] = cvt<RS>(gload(nl, ix.m[i]));
+    for (int i = 0; i < CH; ++i) v[i] = cvt<RS>(vload<SC>(nl, ix.m[i]));
     {
       C c[CH];
       if (tm.coef >= 0) {
@@ -1136,7 +1167,7 @@ __device__ __attribute__((noinline)) double general_pass(const rks_tableau* tbp,
     V w;
     w.x = v.re;
     w.y = v.im;
-    ((RKS_AS3 V*)base)[m] = w;
+    ((RKS_AS3 V*)(unsigned long long)base)[m] = w;
   };
   auto& S = tb.st[s];
   const bool last = s == tb.nstage - 1;
@@ -1368,6 +1399,10 @@ __device__ int run_instance(const rks_launch& P, int idx, cx<R>* buf, const cx<R
   using OW = Own<N, M, T, NLK>;
   constexpr int MPT = OW::MPT;
   constexpr bool METHOD = METH != RKS_METH_ANY;
+  using CK = Chunk<MPT, (int)sizeof(C), T>;
+  constexpr int CH = CK::CH;
+  // the general kernel's tableau entries as uniform values (the Hankel kind: as they stand)
+  auto un = [](int x) { return NLK == NLK_HANKEL ? x : uni(x); };
   constexpr bool PAIRED = !METHOD && M == N && NLK != NLK_HANKEL;  // pass_chunk: other modes than the transforms'
   using TT = MethodTab<METHOD ? METH : 0, (int)sizeof(C), (int)sizeof(CN), NLK == NLK_ADVECT>;
   constexpr bool FUSED = TT::tab.st[TT::tab.nstage - 1].has_nl == 0;  // (METHOD) no NL in the last stage
@@ -1450,7 +1485,7 @@ __device__ int run_instance(const rks_launch& P, int idx, cx<R>* buf, const cx<R
     h_coeff = __builtin_nan("");
     smap = 0x76543210u;
   }
-  const bool adaptive = METHOD ? TT::tab.adaptive != 0 : uni(tb.adaptive) != 0;
+  const bool adaptive = METHOD ? TT::tab.adaptive != 0 : un(tb.adaptive) != 0;
   const bool evolve = (P.mode == RKS_MODE_EVOLVE);
   if (reenter) {
     // back from the proposer: h_next holds its proposal (solveras.py:638-641)
@@ -1492,9 +1527,9 @@ __device__ int run_instance(const rks_launch& P, int idx, cx<R>* buf, const cx<R
   auto slot = [&](int s) -> CN* { return slot_base + (size_t)((smap >> (4 * s)) & 15u) * M; };
   auto pass_args = [&]() { return PassArgs{ws, cbase, h, smap, Mc, ow.lim, ow.fold}; };
   auto cur_u = [&]() -> const C* { return ubuf < 0 ? uin : (const C*)(ubuf == 0 ? cand0 : cand1); };
-  const bool fused = METHOD ? FUSED : uni((int)rks_fused_final(tb)) != 0;
-  const bool recompute = (METHOD ? TT::tab.nl1_policy : uni(tb.nl1_policy)) == RKS_NL1_RECOMPUTE;
-  const int nstage = METHOD ? TT::tab.nstage : uni(tb.nstage);
+  const bool fused = METHOD ? FUSED : un((int)rks_fused_final(tb)) != 0;
+  const bool recompute = (METHOD ? TT::tab.nl1_policy : un(tb.nl1_policy)) == RKS_NL1_RECOMPUTE;
+  const int nstage = METHOD ? TT::tab.nstage : un(tb.nstage);
 
   bool done = false;
   int pending = 0;      // proposer variant: stopped after an accept for the proposer
@@ -1533,7 +1568,7 @@ __device__ int run_instance(const rks_launch& P, int idx, cx<R>* buf, const cx<R
         if (recompute) {
           first_nl = true;
         } else {
-          const unsigned f4 = 4u * (unsigned)(METHOD ? TT::tab.fsal_slot : uni(tb.fsal_slot));
+          const unsigned f4 = 4u * (unsigned)(METHOD ? TT::tab.fsal_slot : un(tb.fsal_slot));
           const unsigned a = smap & 15u, b = (smap >> f4) & 15u;
           smap = (smap & ~(15u | (15u << f4))) | b | (a << f4);
         }
@@ -1544,7 +1579,7 @@ __device__ int run_instance(const rks_launch& P, int idx, cx<R>* buf, const cx<R
 #pragma unroll
       for (int k = 0; k < MPT; ++k) nv[k] = mkc((RN)0, (RN)0);
 #pragma unroll 1
-      for (int s = uni(first_nl ? -1 : 0); s < nstage; ++s) {
+      for (int s = un(first_nl ? -1 : 0); s < nstage; ++s) {
         const bool last = s == nstage - 1;
         C v[MPT];
         int ns = 0;  // NL slot this pass writes
@@ -1566,6 +1601,64 @@ __device__ int run_instance(const rks_launch& P, int idx, cx<R>* buf, const cx<R
             }
             static_assert(TT::tab.st[0].nl_slot == 1 && LAST_SLOT == TT::tab.nslot - 1, "stage s writes slot s + 1");
             ns = s + 1;
+          }
+        } else if constexpr (NLK == NLK_HANKEL) {
+          // Inlined, tableau and arrays read as they stand: with a mode or two per thread nothing
+          // spills, and the code around the products decides how the compiler orders their loads.
+          // By general_pass IF34 takes 0.47 ms for 84 MIXED beams of nr = 126 (like this 0.43) and
+          // 1.06 for 64 FP32 beams of nr = 500 (0.92).
+          if (s < 0) {
+            load_modes(v, u);
+          } else {
+            const rks_stage& S = tb.st[s];
+            if (last && fused) {
+              // per-mode |u_new| and |err|^2 (FP32 buffer: |err|) wait in the idle LDS buffer
+#pragma unroll 1
+              for (int c = 0; c < CK::NCH; ++c) {
+                const ChunkIdx<CH> ix = pass_chunk<N, M, T, NLK, CH>(c, ow.fresh());
+                C acc[CH], ev[CH];
+                final_chunk<R, RN, CH>(tb, u, slot, cbase, (size_t)Mc, ix, h, acc, ev);
+#pragma unroll
+                for (int i = 0; i < CH; ++i) {
+                  const int m = ix.m[i];
+                  if (ix.ok[i]) {
+                    cand[m] = acc[i];
+                    const double a = hypot((double)acc[i].re, (double)acc[i].im);
+                    const double er = (double)ev[i].re, ei = (double)ev[i].im;
+                    mx = nanmax(mx, a);
+                    // FP64 keeps |err|^2; an FP32 buffer keeps |err| (|err|^2 would flush to zero
+                    // below ~1e-19 and turn a real error into an unconditional accept)
+                    if constexpr (sizeof(R) == sizeof(double)) buf[m] = mkc((R)a, (R)(er * er + ei * ei));
+                    else buf[m] = mkc((R)a, (R)hypot(er, ei));
+                  }
+                }
+              }
+              break;
+            }
+            // the stage argument through the thread's own places of the LDS buffer: the run-time
+            // term loop stays rolled over the chunks
+#pragma unroll 1
+            for (int c = 0; c < CK::NCH; ++c) {
+              const ChunkIdx<CH> ix = pass_chunk<N, M, T, NLK, CH>(c, ow.fresh());
+              C acc[CH];
+              stage_chunk<R, RN, CH>(tb, S, u, slot, cbase, (size_t)Mc, ix, h, acc);
+#pragma unroll
+              for (int i = 0; i < CH; ++i) {
+                if (!ix.ok[i]) continue;
+                if (last) {
+                  cand[ix.m[i]] = acc[i];
+                  if (adaptive)
+                    mx = nanmax(mx, (double)acc[i].re * (double)acc[i].re + (double)acc[i].im * (double)acc[i].im);
+                }
+                buf[ix.m[i]] = acc[i];
+              }
+            }
+            if (!S.has_nl) continue;
+            const OW of = ow.fresh();
+#pragma unroll
+            for (int k = 0; k < MPT; ++k) v[k] = buf[of.m(k)];
+            __syncthreads();
+            ns = S.nl_slot;
           }
         } else {
           // the argument through the LDS buffer, u itself too: loaded into v here, it would be
@@ -1681,7 +1774,40 @@ __device__ int run_instance(const rks_launch& P, int idx, cx<R>* buf, const cx<R
         const double lim = fused ? cut * mx : (cut < 0.0 ? -1.0 : cut * cut * mx);
         __syncthreads();  // every thread's last NL values, candidate and buffer values
         using NO = NormOrder<N, M, T, NLK>;
-        if (fused) {
+        if constexpr (NLK == NLK_HANKEL) {
+          constexpr int NCH = (NO::SLOTS + CH - 1) / CH;
+#pragma unroll 1
+          for (int c = 0; c < NCH; ++c) {
+            ChunkIdx<CH> ix = pass_chunk<N, M, T, NLK, CH>(c, ow.fresh());
+#pragma unroll
+            for (int i = 0; i < CH; ++i) {
+              ix.ok[i] = NO::ok(c * CH + i, ow.lim);
+              ix.m[i] = ix.ok[i] ? NO::mode(c * CH + i) : 0;
+            }
+            C ev[CH];
+            if (!fused) error_chunk<R, RN, CH>(tb, slot, cbase, (size_t)Mc, ix, h, ev);
+#pragma unroll
+            for (int i = 0; i < CH; ++i) {
+              if (!ix.ok[i]) continue;
+              if (fused) {
+                const C q = buf[ix.m[i]];
+                const double a = (double)q.re, e = (double)q.im;
+                if (a > lim && a <= __DBL_MAX__) {
+                  su = fma(a, a, su);
+                  se = sizeof(R) < sizeof(double) ? fma(e, e, se) : se + e;
+                }
+              } else {
+                const C kv = cand[ix.m[i]];
+                const double kr = (double)kv.re, ki = (double)kv.im, er = (double)ev[i].re, ei = (double)ev[i].im;
+                const double a = fma(kr, kr, ki * ki);
+                if (a > lim && a <= __DBL_MAX__) {
+                  su += a;
+                  se += fma(er, er, ei * ei);
+                }
+              }
+            }
+          }
+        } else if (fused) {
 #pragma unroll 1
           for (int k = 0; k < NO::SLOTS; ++k) {
             if (!NO::ok(k, ow.lim)) continue;
